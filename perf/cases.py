@@ -535,8 +535,8 @@ def work(case):
         r, c, k = case["rows"], case["cols"], case["k"]
         scale = 0.75 if case["shape"] else 1.0
         r, c = r * scale, c * scale
-        flops = sum(2.0 * c ** (k - q) * r ** q * c * r / c for q in range(1, k + 1)) * case["nvec"]
-        return dict(bytes=8 * case["nvec"] * (c ** k + r ** k) + 8 * k * r * c, flops=flops * c)
+        flops = sum(2.0 * c ** (k - q) * r ** q * c for q in range(1, k + 1)) * case["nvec"]
+        return dict(bytes=8 * case["nvec"] * (c ** k + r ** k) + 8 * k * r * c, flops=flops)
     nd, deg, lev = case["nd"], case["deg"], case["lev"]
     npts = deg << lev
     flops = sum(2.0 * sum(2 ** c * m for c, m in _level_sums(d, lev)) * deg ** d * npts ** (nd - d + 1)
