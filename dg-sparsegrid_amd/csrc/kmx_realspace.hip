@@ -4,75 +4,118 @@
 // The reference sums, over elements e, kron(Meval_1(:, J_1(e)), ..., Meval_d(:, J_d(e)))
 // times the element's deg^d coefficients, where Meval_k(:, J) is the deg-column
 // block of dimension k's evaluation matrix at the element's 1D index.  Here the
-// elements are grouped by level multi-index: the elements of one group are the
-// cells of a dense tensor, and their summed contribution is one rectangular
-// Kronecker product of the level's column ranges applied to that tensor (absent
-// cells are zeros) -- d mode products per group instead of one kron_multd per
-// element.  Same terms, summed in another order.
+// sum runs dimension by dimension, last first, over the tree of index prefixes:
+// with the elements sorted by (J_1, ..., J_d), a node of depth k is a distinct
+// prefix (J_1, ..., J_k), and
+//
+//   Z_k[node (J_1..J_{k-1}); b_1..b_{k-1}; p_k, p_{k+1}..p_d] =
+//       sum over its children J_k and b_k of Meval_k(p_k, (J_k, b_k)) Z_{k+1}[child; b_1..b_k; p_{k+1}..p_d]
+//
+// with Z_{d+1} the coefficients and Z_1 the result: d launches of products whose k
+// index runs over a node's children, each value of Z written once.  (One Kronecker
+// product per level tuple added into the output instead -- 84 tuples x 4 launches
+// on a 3D lev 6 grid, each re-reading and adding all 192^3 points -- took 6.5 ms.)
+// The products run on the FP64 matrix cores (kmx_mma64.h).  3D lev 6 deg 3 (192^3
+// points): 0.162 ms, error against 64 bits 3.5e-16 (4.6e-16 before); the last stage,
+// 2.7 GFLOP of dense products, is most of it.  Same terms, summed in another order.
 #include "kmx_internal.h"
+#include "kmx_mma64.h"
 
 #include <algorithm>
 #include <map>
+#include <numeric>
 #include <stdexcept>
 #include <vector>
 
 namespace kmx {
 namespace {
 
-struct GatherArgs {
-    const double* fw;
-    double* X;
-    const int* elems;  // cell -> element (row-major over cells, dim 1 slowest), -1 absent
-    int cells[KMX_MAX_DIM];
-    int D, deg, B;
-    long long n;  // entries of X
-};
-
-// X[(c_1 deg + a_1), ..., (c_d deg + a_d)] (row-major, dim 1 slowest) from the
-// element-major coefficient vector.
-__global__ void __launch_bounds__(256) k_gather(GatherArgs g) {
-    for (long long v = blockIdx.x * 256ll + threadIdx.x; v < g.n; v += (long long)gridDim.x * 256) {
-        long long rest = v;
-        int ci = 0, ai = 0, cstride = 1, astride = 1;
-        for (int k = g.D - 1; k >= 0; --k) {
-            const int ext = g.cells[k] * g.deg;
-            const int m = int(rest % ext);
-            rest /= ext;
-            ci += (m / g.deg) * cstride;
-            ai += (m % g.deg) * astride;
-            cstride *= g.cells[k];
-            astride *= g.deg;
-        }
-        const int e = g.elems[ci];
-        g.X[v] = e >= 0 ? g.fw[(long long)e * g.B + ai] : 0.0;
-    }
-}
-
-struct ModeArgs {
+// One stage.  Nodes are consecutive; node q's children are cptr[q] .. cptr[q + 1] - 1
+// with first Meval columns col[c]; nbeta = deg^(k - 1) values of (b_1..b_{k-1}).
+struct StageArgs {
     const double* in;
     double* out;
-    const double* A;  // M x K column-major, leading dimension lda
-    long long pre, post;
-    int M, K, lda;
-    int accumulate;
+    const double* A;   // Meval_k, M x (columns), column-major
+    const int* cptr;
+    const int* col;
+    const int* row;    // last dimension: the child's element
+    long long R;       // values of (p_{k+1}..p_d)
+    int M, deg, nbeta, B;
+    unsigned magic;    // 2^32 / deg + 1
+    int items;         // node x beta (node alone in the last dimension)
+    int mt, nt;        // tiles per item
+    int xcd;           // 1: the row tiles of a column tile run on one XCD
 };
 
-// out[p, i, q] (= or +=) sum_j A(i, j) in[p, j, q]; one thread per output.
-__global__ void __launch_bounds__(256) k_mode(ModeArgs m) {
-    const long long total = m.pre * m.M * m.post;
-    for (long long e = blockIdx.x * 256ll + threadIdx.x; e < total; e += (long long)gridDim.x * 256) {
-        const long long q = e % m.post;
-        const long long r = e / m.post;
-        const int i = int(r % m.M);
-        const long long p = r / m.M;
-        const double* in = m.in + p * m.K * m.post + q;
-        double acc = 0.0;
-        for (int j = 0; j < m.K; ++j) acc = __builtin_fma(m.A[i + (long long)j * m.lda], in[j * m.post], acc);
-        if (m.accumulate)
-            m.out[e] += acc;
-        else
-            m.out[e] = acc;
+// k / deg and k % deg of a position in a child list (k < 2^28; magic = 2^32 / deg + 1)
+__device__ __forceinline__ void split_k(int k, const StageArgs& a, int& c, int& b) {
+    c = a.deg == 1 ? k : int(__umulhi(unsigned(k), a.magic));
+    b = k - c * a.deg;
+}
+
+// The last dimension: Z_d[node; beta; p] = sum_k f[element(k), beta, b(k)] Meval_d(p, k).
+// Rows beta (few), columns p; a chunk of 32 k keeps enough loads in flight for the
+// long child lists of the low prefixes.
+__global__ void __launch_bounds__(256) k_rs_last(StageArgs a) {
+    __shared__ double lds[mma64_lds<16, 32>()];
+    const int tiles = a.mt * a.nt;
+    const int q = int(blockIdx.x) / tiles, t = int(blockIdx.x) - q * tiles;
+    if (q >= a.items) return;
+    const int i0 = 16 * (t % a.mt), j0 = 64 * (t / a.mt);
+    const int c0 = a.cptr[q], K = (a.cptr[q + 1] - c0) * a.deg;
+    const int deg = a.deg;
+    auto fa = [&](int i, int k) {
+        int c, b;
+        split_k(k, a, c, b);
+        return a.in[(long long)a.row[c0 + c] * a.B + (i0 + i) * deg + b];
+    };
+    auto fb = [&](int k, int j) {
+        int c, b;
+        split_k(k, a, c, b);
+        return a.A[(long long)(a.col[c0 + c] + b) * a.M + j0 + j];
+    };
+    double* out = a.out + (long long)q * a.nbeta * a.M;
+    auto st = [&](int i, int j, double v) { out[(long long)(i0 + i) * a.M + j0 + j] = v; };
+    mma64_tile<16, 32>(a.nbeta - i0, a.M - j0, K, fa, fb, st, lds);
+}
+
+// Dimension k < d: Z_k[node; beta; p, r] = sum_k Meval_k(p, k) Z_{k+1}[child(k); beta, b(k); r].
+// The column tiles of an item are dealt so that the workgroups of one column tile
+// (its row tiles, which read the same values of Z_{k+1}) share an XCD's L2.
+__global__ void __launch_bounds__(256) k_rs_mode(StageArgs a) {
+    __shared__ double lds[mma64_lds<64, 16>()];
+    const int per = a.xcd ? a.mt * ((a.nt + 7) / 8) * 8 : a.mt * a.nt;
+    const int item = int(blockIdx.x) / per, t = int(blockIdx.x) - item * per;
+    if (item >= a.items) return;
+    int rt, ct;
+    if (a.xcd) {
+        rt = (t / 8) % a.mt;
+        ct = (t / 8) / a.mt * 8 + t % 8;
+        if (ct >= a.nt) return;
+    } else {
+        rt = t % a.mt;
+        ct = t / a.mt;
     }
+    const int q = item / a.nbeta, beta = item - q * a.nbeta;
+    const int i0 = 64 * rt;
+    const long long j0 = 64LL * ct;
+    const int c0 = a.cptr[q], K = (a.cptr[q + 1] - c0) * a.deg;
+    const int deg = a.deg;
+    auto fa = [&](int i, int k) {
+        int c, b;
+        split_k(k, a, c, b);
+        return a.A[(long long)(a.col[c0 + c] + b) * a.M + i0 + i];
+    };
+    const double* in = a.in + ((long long)c0 * a.nbeta + beta) * deg * a.R + j0;
+    const long long cs = (long long)a.nbeta * deg * a.R;
+    auto fb = [&](int k, int j) {
+        int c, b;
+        split_k(k, a, c, b);
+        return in[c * cs + b * a.R + j];
+    };
+    double* out = a.out + (long long)item * a.M * a.R + j0;
+    auto st = [&](int i, int j, double v) { out[(long long)(i0 + i) * a.R + j] = v; };
+    mma64_tile<64, 16>(a.M - i0, int(min(64LL, a.R - j0)), K, fa, fb, st, lds);
 }
 
 __global__ void __launch_bounds__(256) k_zero(double* y, long long n) {
@@ -97,20 +140,26 @@ struct kmx_realspace {
     int npts[KMX_MAX_DIM] = {0}, ncols[KMX_MAX_DIM] = {0};
     long long nout = 0;
     double* d_meval[KMX_MAX_DIM] = {nullptr};
-    struct Block {
-        int cells[KMX_MAX_DIM];
-        int col0[KMX_MAX_DIM];  // first column of the level range in Meval_d
-        int eoff;
+    // stage k (contracting dimension k): its nodes (prefixes of length k), their
+    // children (nodes of stage k + 1; elements in the last) and the children's columns
+    struct Stage {
+        int nodes = 0;
+        int* d_cptr = nullptr;
+        int* d_col = nullptr;
     };
-    std::vector<Block> blocks;
-    int* d_elems = nullptr;
-    double* d_buf[3] = {nullptr, nullptr, nullptr};
+    Stage stage[KMX_MAX_DIM];
+    int* d_row = nullptr;                   // elements in prefix order
+    double* d_buf[2] = {nullptr, nullptr};  // Z_d, Z_{d-1}, ... in turn
 };
 
 static void free_rs(kmx_realspace* r) {
     for (auto& m : r->d_meval)
         if (m) hipFree(m);
-    if (r->d_elems) hipFree(r->d_elems);
+    for (auto& st : r->stage) {
+        if (st.d_cptr) hipFree(st.d_cptr);
+        if (st.d_col) hipFree(st.d_col);
+    }
+    if (r->d_row) hipFree(r->d_row);
     for (auto& b : r->d_buf)
         if (b) hipFree(b);
 }
@@ -143,68 +192,81 @@ extern "C" int kmx_realspace_create(int ndim, int deg, int num_elem, const int* 
             if (hipMemcpy(r->d_meval[k], meval[k], sz * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
                 throw std::runtime_error("hipMemcpy failed");
         }
-        // elements by level multi-index
-        std::map<std::vector<int>, int> bid;
-        std::vector<std::vector<int>> members;
-        std::vector<std::vector<int>> ecell(num_elem);
+        // element indices, level tuples and cells as the transform takes them
+        std::map<std::vector<int>, long long> lev_cells;
+        std::vector<int> idx(size_t(num_elem) * ndim);
         for (int e = 0; e < num_elem; ++e) {
             std::vector<int> lev(ndim);
-            ecell[e].resize(ndim);
             for (int k = 0; k < ndim; ++k) {
                 const int I0 = elem_idx1d[size_t(e) * ndim + k] - index_base;
                 if (I0 < 0 || (I0 + 1) * deg > ncols[k]) throw std::invalid_argument("elem_idx1d out of range");
+                idx[size_t(e) * ndim + k] = I0;
                 lev[k] = level_of(I0);
-                ecell[e][k] = lev[k] == 0 ? 0 : I0 - (1 << (lev[k] - 1));
             }
-            auto it = bid.find(lev);
-            if (it == bid.end()) {
-                it = bid.emplace(lev, int(members.size())).first;
-                members.emplace_back();
-            }
-            members[it->second].push_back(e);
-        }
-        std::vector<int> elems;
-        long long maxX = 1, maxI = 1;
-        r->blocks.resize(members.size());
-        for (const auto& kv : bid) {
-            auto& b = r->blocks[kv.second];
+            if (lev_cells.count(lev)) continue;
             long long ncell = 1;
             for (int k = 0; k < ndim; ++k) {
-                const int l = kv.first[k];
-                b.col0[k] = l == 0 ? 0 : (1 << (l - 1));
-                b.cells[k] = std::min(l == 0 ? 1 : (1 << (l - 1)), ncols[k] / deg - b.col0[k]);
-                ncell *= b.cells[k];
+                const int c0 = lev[k] == 0 ? 0 : (1 << (lev[k] - 1));
+                ncell *= std::min(lev[k] == 0 ? 1 : (1 << (lev[k] - 1)), ncols[k] / deg - c0);
             }
             if (ncell * r->B > (1LL << 30)) throw std::invalid_argument("level block too large");
-            b.eoff = int(elems.size());
-            elems.resize(elems.size() + size_t(ncell), -1);
-            for (int e : members[kv.second]) {
-                long long ci = 0;
-                for (int k = 0; k < ndim; ++k) ci = ci * b.cells[k] + ecell[e][k];
-                int& slot = elems[size_t(b.eoff) + size_t(ci)];
-                if (slot >= 0) throw std::invalid_argument("two elements share one 1D index tuple");
-                slot = e;
-            }
-            maxX = std::max(maxX, ncell * r->B);
-            // intermediates of the chain: dims d..k+1 already at npts
-            long long ext[KMX_MAX_DIM];
-            for (int k = 0; k < ndim; ++k) ext[k] = (long long)b.cells[k] * deg;
-            for (int k = ndim - 1; k >= 1; --k) {
-                ext[k] = npts[k];
-                long long sz = 1;
-                for (int m = 0; m < ndim; ++m) sz *= ext[m];
-                maxI = std::max(maxI, sz);
-            }
+            lev_cells[lev] = ncell;
         }
-        if (!elems.empty()) {
-            if (hipMalloc(&r->d_elems, elems.size() * sizeof(int)) != hipSuccess) throw std::bad_alloc();
-            if (hipMemcpy(r->d_elems, elems.data(), elems.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess)
+        // elements sorted by index tuple; the distinct prefixes of each length
+        std::vector<int> order(static_cast<size_t>(num_elem));
+        std::iota(order.begin(), order.end(), 0);
+        auto ix = [&](int e, int k) { return idx[size_t(e) * ndim + k]; };
+        std::sort(order.begin(), order.end(), [&](int a, int b) {
+            for (int k = 0; k < ndim; ++k)
+                if (ix(a, k) != ix(b, k)) return ix(a, k) < ix(b, k);
+            return a < b;
+        });
+        // first position (in `order`) of every node of depth k: positions where one of
+        // the indices 0..k-1 changes
+        std::vector<std::vector<int>> first(size_t(ndim) + 1);
+        for (int p = 0; p < num_elem; ++p) {
+            int diff = p == 0 ? 0 : ndim;  // the first differing dimension
+            for (int k = 0; p > 0 && k < ndim; ++k)
+                if (ix(order[size_t(p)], k) != ix(order[size_t(p) - 1], k)) {
+                    diff = k;
+                    break;
+                }
+            if (p > 0 && diff == ndim) throw std::invalid_argument("two elements share one 1D index tuple");
+            for (int k = diff + 1; k <= ndim; ++k) first[size_t(k)].push_back(p);
+        }
+        if (num_elem > 0) first[0].push_back(0);
+        auto up = [](const std::vector<int>& h, int*& d) {
+            if (h.empty()) return;
+            if (hipMalloc(&d, h.size() * sizeof(int)) != hipSuccess) throw std::bad_alloc();
+            if (hipMemcpy(d, h.data(), h.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess)
                 throw std::runtime_error("hipMemcpy failed");
+        };
+        long long need[2] = {1, 1}, R = 1;
+        for (int k = ndim - 1; k >= 0; --k) {
+            const std::vector<int>& par = first[size_t(k)];
+            const std::vector<int>& chl = first[size_t(k) + 1];
+            std::vector<int> cptr, col(chl.size());
+            size_t c = 0;
+            for (size_t q = 0; q < par.size(); ++q) {
+                cptr.push_back(int(c));
+                const int end = q + 1 < par.size() ? par[q + 1] : num_elem;
+                while (c < chl.size() && chl[c] < end) ++c;
+            }
+            cptr.push_back(int(c));
+            for (size_t q = 0; q < chl.size(); ++q) col[q] = ix(order[size_t(chl[q])], k) * deg;
+            r->stage[k].nodes = int(par.size());
+            up(cptr, r->stage[k].d_cptr);
+            up(col, r->stage[k].d_col);
+            if (k > 0) {  // Z_{k+1} of the comment above (k from 1 there)
+                R *= npts[k];
+                long long nb = 1;
+                for (int q = 0; q < k; ++q) nb *= deg;
+                need[(ndim - 1 - k) & 1] = std::max(need[(ndim - 1 - k) & 1], (long long)par.size() * nb * R);
+            }
         }
-        if (hipMalloc(&r->d_buf[0], size_t(maxX) * sizeof(double)) != hipSuccess ||
-            hipMalloc(&r->d_buf[1], size_t(maxI) * sizeof(double)) != hipSuccess ||
-            hipMalloc(&r->d_buf[2], size_t(maxI) * sizeof(double)) != hipSuccess)
-            throw std::bad_alloc();
+        up(order, r->d_row);
+        for (int q = 0; q < 2; ++q)
+            if (hipMalloc(&r->d_buf[q], size_t(need[q]) * sizeof(double)) != hipSuccess) throw std::bad_alloc();
         *out = r;
         return KMX_OK;
     } catch (const std::bad_alloc&) {
@@ -226,45 +288,52 @@ extern "C" int kmx_realspace_apply(kmx_realspace* r, const double* f_w, double* 
         return KMX_E_ARG;
     }
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(k_zero, dim3(grid_for(r->nout)), dim3(256), 0, s, f_r, r->nout);
-    const int D = r->D, deg = r->deg;
-    for (const auto& b : r->blocks) {
-        GatherArgs g;
-        g.fw = f_w;
-        g.X = r->d_buf[0];
-        g.elems = r->d_elems + b.eoff;
-        g.D = D;
-        g.deg = deg;
-        g.B = r->B;
-        g.n = r->B;
-        for (int k = 0; k < D; ++k) {
-            g.cells[k] = b.cells[k];
-            g.n *= b.cells[k];
+    if (r->N == 0) hipLaunchKernelGGL(k_zero, dim3(grid_for(r->nout)), dim3(256), 0, s, f_r, r->nout);
+    const int D = r->D;
+    const double* cur = f_w;
+    long long R = 1;
+    for (int k = D - 1; k >= 0 && r->N > 0; --k) {
+        StageArgs a;
+        a.in = cur;
+        a.out = k == 0 ? f_r : r->d_buf[(D - 1 - k) & 1];
+        a.A = r->d_meval[k];
+        a.cptr = r->stage[k].d_cptr;
+        a.col = r->stage[k].d_col;
+        a.row = r->d_row;
+        a.R = R;
+        a.M = r->npts[k];
+        a.deg = r->deg;
+        a.magic = unsigned((1ULL << 32) / unsigned(r->deg) + 1);
+        a.B = r->B;
+        a.nbeta = 1;
+        for (int q = 0; q < k; ++q) a.nbeta *= r->deg;
+        long long grid;
+        if (k == D - 1) {
+            a.items = r->stage[k].nodes;
+            a.mt = (a.nbeta + 15) / 16;
+            a.nt = (a.M + 63) / 64;
+            a.xcd = 0;
+            grid = (long long)a.items * a.mt * a.nt;
+        } else {
+            a.items = r->stage[k].nodes * a.nbeta;
+            a.mt = (a.M + 63) / 64;
+            const long long nt = (R + 63) / 64;
+            if (nt >= (1LL << 30)) {
+                set_error("kmx_realspace_apply: too many points");
+                return KMX_E_UNSUPPORTED;
+            }
+            a.nt = int(nt);
+            a.xcd = a.mt > 1 && a.nt >= 8 ? 1 : 0;
+            grid = (long long)a.items * a.mt * (a.xcd ? (nt + 7) / 8 * 8 : nt);
         }
-        hipLaunchKernelGGL(k_gather, dim3(grid_for(g.n)), dim3(256), 0, s, g);
-        long long ext[KMX_MAX_DIM];
-        for (int k = 0; k < D; ++k) ext[k] = (long long)b.cells[k] * deg;
-        const double* cur = r->d_buf[0];
-        int ping = 1;
-        for (int k = D - 1; k >= 0; --k) {  // last dimension first (kron_multd's method-1 order)
-            ModeArgs m;
-            m.in = cur;
-            m.out = k == 0 ? f_r : r->d_buf[ping];
-            m.A = r->d_meval[k] + (long long)b.col0[k] * deg * r->npts[k];
-            m.lda = r->npts[k];
-            m.M = r->npts[k];
-            m.K = int(ext[k]);
-            m.pre = 1;
-            m.post = 1;
-            for (int q = 0; q < k; ++q) m.pre *= ext[q];
-            for (int q = k + 1; q < D; ++q) m.post *= ext[q];
-            m.accumulate = k == 0;
-            const long long total = m.pre * m.M * m.post;
-            hipLaunchKernelGGL(k_mode, dim3(grid_for(total)), dim3(256), 0, s, m);
-            ext[k] = r->npts[k];
-            cur = m.out;
-            ping = 3 - ping;
+        if (grid >= (1LL << 31)) {
+            set_error("kmx_realspace_apply: too many points");
+            return KMX_E_UNSUPPORTED;
         }
+        if (k == D - 1) hipLaunchKernelGGL(k_rs_last, dim3(unsigned(grid)), dim3(256), 0, s, a);
+        else hipLaunchKernelGGL(k_rs_mode, dim3(unsigned(grid)), dim3(256), 0, s, a);
+        R *= r->npts[k];
+        cur = a.out;
     }
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) {

@@ -98,3 +98,31 @@ def test_asgard_realspace_matches_gold(kmx_gpu, gold, name, deg, lev, doms):
     key = f"transformations/wavelet_to_realspace_{name}"
     ref = gold[key].ravel()
     assert rel(fr[:: int(gold[key + "/stride"][0])], ref) <= 1e-13
+
+
+@pytest.mark.parametrize(
+    "nd,lev,deg,npts",
+    [
+        (1, 3, 1, [1]), (1, 6, 8, [65]),            # one row of points; a list of 512 k, one tile and a column more
+        (2, 4, 1, [64, 63]), (2, 3, 5, [16, 129]),  # exact and ragged tiles, deg without a shift
+        (3, 2, 5, [17, 33, 65]),                    # 25 prefix values: more than one 16-row tile
+        (3, 3, 2, [70, 9, 70]),                     # several row tiles over >= 8 column tiles (630 values)
+        (6, 1, 2, [3, 2, 4, 2, 3, 5]),
+    ],
+)
+def test_realspace_tile_edges(kmx_gpu, nd, lev, deg, npts):
+    """Tile edges and remainders of the staged products.  Every result is a sum of at most
+    N deg^d products of d + 1 factors ~ N(0, 1): (N deg^d)^(1/2) eps relative, below 1e-13."""
+    rng = np.random.default_rng(nd * 10 + deg)
+    h = O.hash_table_sparse_nd([lev] * nd, lev, "SG")
+    meval = [rng.standard_normal((npts[d], deg * 2 ** lev)) for d in range(nd)]
+    assert run_case(kmx_gpu, meval, h["idx1d"], deg, seed=lev) <= 1e-13
+
+
+def test_realspace_no_elements(kmx_gpu):
+    import torch
+
+    rs = kmx_gpu.RealSpace([np.ones((5, 4)), np.ones((3, 4))], np.zeros((0, 2), np.int32), 2)
+    out = torch.full((15,), 7.0, dtype=torch.float64, device="cuda")
+    rs.apply(torch.empty(0, dtype=torch.float64, device="cuda"), out)
+    assert torch.count_nonzero(out) == 0
