@@ -87,3 +87,15 @@ def test_asgard_build_A_sparse_and_dense(kmx_gpu):
     f = np.random.default_rng(2).standard_normal(f0.size)
     y = AS.apply_A(pde, opts, A_data, f, 2)
     assert np.linalg.norm(Ad @ f - y) <= 1e-13 * np.linalg.norm(y)
+
+
+@pytest.mark.parametrize("nd,lev,deg,T,conn", [(1, 2, 1, 1, False), (2, 2, 4, 2, True), (2, 1, 5, 1, False),
+                                               (3, 1, 4, 2, False), (5, 1, 2, 3, True), (6, 1, 2, 2, False),
+                                               (2, 6, 2, 6, True), (1, 9, 4, 2, True)])
+def test_assembled_blocks_edges(kmx_gpu, nd, lev, deg, T, conn):
+    """Blocks of 1, 256 and more entries, rows of more pairs than a chunk, strips beyond
+    LDS (1D lev 9): bit-exact like the shapes above."""
+    mats, idx, rp, cols = make_case(nd, lev, deg, T, conn, seed=7 + nd + lev)
+    plan = kmx_gpu.Plan(mats, idx, deg, rp, cols)
+    A = dense_from_blocks(plan.assemble().cpu().numpy(), plan.N, plan.B, rp, cols)
+    assert np.array_equal(A, O.build_A(O.ApplyInputs(mats, idx, deg, rp, cols)))
