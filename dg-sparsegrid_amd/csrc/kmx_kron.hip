@@ -13,7 +13,8 @@ namespace kmx {
 
 // One mode product of the method-1 chain: contract dim `dim` (0 = slowest) of a
 // column-major tensor whose dims have current extents ext[] (ext of dim k is
-// ncol_k before its contraction and nrow_k after).  One thread per output entry.
+// ncol_k before its contraction and nrow_k after).  One thread per output entry:
+// the form for factors whose mode alone is beyond k_mode_group's LDS tile.
 struct ModeArgs {
     const double* in;
     double* out;
@@ -34,6 +35,119 @@ __global__ void __launch_bounds__(256) k_mode_product(ModeArgs m) {
         double acc = 0.0;
         for (int b = 0; b < m.ncol; ++b) acc = __builtin_fma(m.A[(long long)b * m.nrow + a], in[b * m.inner], acc);
         m.out[e] = acc;
+    }
+}
+
+// Several consecutive modes of the chain in one launch.  A workgroup holds, for OC
+// values of the slower indices and IC of the faster ones, every value of the group's
+// modes in LDS (two buffers) and contracts them last first; each tensor value is read
+// and written in HBM once per group instead of once per mode.  A thread takes fibres
+// along the mode: the inputs come one by one from LDS, the factor's column -- the same
+// for every lane -- through the scalar cache, and up to 16 outputs accumulate in
+// registers (1 LDS read per NR FMAs; one thread per output read two values per FMA).
+// Every output sums its products in column order with FMAs from zero, as the one-mode
+// kernel does: the results are bit-identical however the chain is grouped.  LDS index
+// i sits at i + i / 8: fibres of the fastest mode, ncol apart, spread over the banks.
+// Four 8 x 8 factors on 128 vectors: 4 launches, 32 us of kernel time -> 1.
+constexpr int KG_THREADS = 512;
+constexpr int KG_TILE = 8704;   // values of a tile at most: 2 buffers x 9/8 x 8 bytes = 153 KB of the 160 KB
+constexpr int KG_MIN_IC = 8;    // contiguous values per access at least when the modes are strided
+struct GroupArgs {
+    const double* in;
+    double* out;
+    const double* A[KMX_KRON_MAX_FACTORS];  // the group's factors, slowest first
+    int nrow[KMX_KRON_MAX_FACTORS], ncol[KMX_KRON_MAX_FACTORS];
+    long long inner;  // extent of the faster (already contracted) modes
+    long long outer;  // extent of the slower modes times nvec
+    int k, OC, IC, buf;  // buf: doubles of one LDS buffer
+    int chunks;          // workgroups along inner
+};
+__device__ __forceinline__ int kg_at(int i) { return i + (i >> 3); }
+
+template <int NR>
+__device__ __forceinline__ void kg_fibre(const double* __restrict__ A, int nrow, int ncol, const double* __restrict__ src,
+                                         double* __restrict__ dst, int ib, int ob, int inner) {
+    double acc[NR];
+#pragma unroll
+    for (int a = 0; a < NR; ++a) acc[a] = 0.0;
+#pragma unroll 4
+    for (int b = 0; b < ncol; ++b) {
+        const double x = src[kg_at(ib + b * inner)];
+#pragma unroll
+        for (int a = 0; a < NR; ++a) acc[a] = __builtin_fma(A[(long long)b * nrow + a], x, acc[a]);
+    }
+#pragma unroll
+    for (int a = 0; a < NR; ++a) dst[kg_at(ob + a * inner)] = acc[a];
+}
+
+template <int NR>
+__device__ __forceinline__ void kg_mode(const double* __restrict__ A, int nrow, int ncol, int a0,
+                                        const double* __restrict__ src, double* __restrict__ dst, int nf, int inner) {
+    for (int f = threadIdx.x; f < nf; f += blockDim.x) {
+        const int o = f / inner, s = f - o * inner;
+        kg_fibre<NR>(A + a0, nrow, ncol, src, dst, o * ncol * inner + s, (o * nrow + a0) * inner + s, inner);
+    }
+}
+
+__global__ void __launch_bounds__(KG_THREADS) k_mode_group(GroupArgs g) {
+    extern __shared__ __align__(16) double kg_lds[];
+    const long long wg = blockIdx.x;
+    const long long ob = wg / g.chunks;
+    const long long o0 = ob * g.OC, s0 = (wg - ob * g.chunks) * g.IC;
+    const int oc = int(min((long long)g.OC, g.outer - o0)), ic = int(min((long long)g.IC, g.inner - s0));
+    int pin = 1, pout = 1;
+    for (int d = 0; d < g.k; ++d) {
+        pin *= g.ncol[d];
+        pout *= g.nrow[d];
+    }
+    double* src = kg_lds;
+    double* dst = kg_lds + g.buf;
+    {  // the tile in: value p of the modes, s of the faster indices (IC = inner unless OC = 1)
+        const double* in = g.in + o0 * pin * g.inner + s0;
+        const int n = oc * pin * g.IC;
+        for (int i = threadIdx.x; i < n; i += blockDim.x) {
+            const int p = i / g.IC, s = i - p * g.IC;
+            src[kg_at(i)] = s < ic ? in[(long long)p * g.inner + s] : 0.0;
+        }
+    }
+    __syncthreads();
+    int fast = g.IC;  // extent of the faster indices inside the tile
+    int slow = oc * pin;
+    for (int d = g.k - 1; d >= 0; --d) {
+        const int nr = g.nrow[d], nc = g.ncol[d];
+        slow /= nc;
+        const int nf = slow * fast;
+        for (int a0 = 0; a0 < nr; a0 += 16) {
+            switch (min(16, nr - a0)) {
+                case 1: kg_mode<1>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
+                case 2: kg_mode<2>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
+                case 3: kg_mode<3>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
+                case 4: kg_mode<4>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
+                case 5: kg_mode<5>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
+                case 6: kg_mode<6>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
+                case 7: kg_mode<7>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
+                case 8: kg_mode<8>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
+                case 9: kg_mode<9>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
+                case 10: kg_mode<10>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
+                case 11: kg_mode<11>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
+                case 12: kg_mode<12>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
+                case 13: kg_mode<13>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
+                case 14: kg_mode<14>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
+                case 15: kg_mode<15>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
+                default: kg_mode<16>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
+            }
+        }
+        fast *= nr;
+        __syncthreads();
+        double* t = src;
+        src = dst;
+        dst = t;
+    }
+    double* out = g.out + o0 * pout * g.inner + s0;
+    const int n = oc * pout * g.IC;
+    for (int i = threadIdx.x; i < n; i += blockDim.x) {
+        const int p = i / g.IC, s = i - p * g.IC;
+        if (s < ic) out[(long long)p * g.inner + s] = src[kg_at(i)];
     }
 }
 
@@ -258,33 +372,140 @@ long long chain_workspace(int k, const int* nrow, const int* ncol, int nvec) {
     return maxsz;
 }
 
+// The chain's launches: modes [first, last] each, last modes first.  group: one
+// k_mode_group launch; otherwise one mode through k_mode_product.
+struct ChainStep {
+    int first, last;
+    bool group;
+};
+
+// As many modes as fit the LDS tile go into one launch: the trailing modes with every
+// value of theirs contiguous, earlier ones with at least KG_MIN_IC contiguous values of
+// the faster indices (all of them where there are fewer).
+// A chain of several modes may be given Y on top of X (its first launch has read X
+// before its last one writes): then every mode has a launch of its own.
+std::vector<ChainStep> plan_chain(int k, const int* nrow, const int* ncol, int nvec, const double* X,
+                                  const double* Y) {
+    std::vector<ChainStep> steps;
+    double nx = nvec, ny = nvec;
+    for (int i = 0; i < k; ++i) {
+        nx *= ncol[i];
+        ny *= nrow[i];
+    }
+    const double gap = double(reinterpret_cast<intptr_t>(Y) - reinterpret_cast<intptr_t>(X));
+    if (k > 1 && gap < 8.0 * nx && -gap < 8.0 * ny) {
+        for (int d = k - 1; d >= 0; --d) steps.push_back(ChainStep{d, d, false});
+        return steps;
+    }
+    double inner = 1.0;  // extent of the modes contracted so far
+    for (int d = k - 1; d >= 0;) {
+        const double ic = std::min<double>(inner, KG_MIN_IC);
+        int e = d + 1;  // modes [e, d] fit
+        double rows = 1.0;
+        for (int q = d; q >= 0; --q) {  // largest extent of modes [q, d] during their contraction
+            double cols = 1.0, r = 1.0, most = 0.0;
+            for (int i = q; i <= d; ++i) cols *= ncol[i];
+            most = cols;
+            for (int i = d; i >= q; --i) {
+                cols /= ncol[i];
+                r *= nrow[i];
+                most = std::max(most, cols * r);
+            }
+            if (most * ic > KG_TILE) break;
+            e = q;
+            rows = r;
+        }
+        if (e > d) {
+            steps.push_back(ChainStep{d, d, false});
+            inner *= nrow[d];
+            --d;
+        } else {
+            steps.push_back(ChainStep{e, d, true});
+            inner *= rows;
+            d = e - 1;
+        }
+    }
+    return steps;
+}
+
 // The mode products of kron(A1..Ak) X, last factor first (method 1), through the
-// ping-pong buffers buf[0] / buf[1] (buf[1] used only for k > 2).  For k > 6 this
-// is also the order of kron_multd.m's recursion (kron_multd.m:64-86: Z = A_k X,
+// ping-pong buffers buf[0] / buf[1] (used only when the steps need them).  For k > 6
+// this is also the order of kron_multd.m's recursion (kron_multd.m:64-86: Z = A_k X,
 // then kron(A_1..A_{k-1}) on Z's transpose).
-void launch_chain(int k, const int* nrow, const int* ncol, const double* const* A, const double* X, int nvec,
-                  double* Y, double* const* buf, hipStream_t s) {
+hipError_t launch_chain(const std::vector<ChainStep>& steps, int k, const int* nrow, const int* ncol,
+                        const double* const* A, const double* X, int nvec, double* Y, double* const* buf,
+                        hipStream_t s) {
     std::vector<long long> ext(ncol, ncol + k);
     const double* cur = X;
     int ping = 0;
-    for (int d = k - 1; d >= 0; --d) {
-        ModeArgs m;
-        m.in = cur;
-        m.out = (d == 0) ? Y : buf[ping];
-        m.A = A[d];
-        m.nrow = nrow[d];
-        m.ncol = ncol[d];
-        m.inner = 1;
-        for (int i = d + 1; i < k; ++i) m.inner *= ext[i];
-        m.outer = nvec;
-        for (int i = 0; i < d; ++i) m.outer *= ext[i];
-        const long long total = m.inner * m.nrow * m.outer;
-        const int grid = int(std::min<long long>((total + 255) / 256, 65536));
-        if (grid > 0) hipLaunchKernelGGL(k_mode_product, dim3(grid), dim3(256), 0, s, m);
-        ext[d] = nrow[d];
-        cur = m.out;
+    for (const ChainStep& st : steps) {
+        double* out = st.first == 0 ? Y : buf[ping];
+        long long inner = 1, outer = nvec;
+        for (int i = st.last + 1; i < k; ++i) inner *= ext[i];
+        for (int i = 0; i < st.first; ++i) outer *= ext[i];
+        if (!st.group) {
+            ModeArgs m;
+            m.in = cur;
+            m.out = out;
+            m.A = A[st.first];
+            m.nrow = nrow[st.first];
+            m.ncol = ncol[st.first];
+            m.inner = inner;
+            m.outer = outer;
+            const long long total = m.inner * m.nrow * m.outer;
+            const int grid = int(std::min<long long>((total + 255) / 256, 65536));
+            if (grid > 0) hipLaunchKernelGGL(k_mode_product, dim3(grid), dim3(256), 0, s, m);
+        } else {
+            GroupArgs g;
+            g.in = cur;
+            g.out = out;
+            g.k = st.last - st.first + 1;
+            long long cols = 1, rows = 1;
+            for (int i = 0; i < g.k; ++i) {
+                g.A[i] = A[st.first + i];
+                g.nrow[i] = nrow[st.first + i];
+                g.ncol[i] = ncol[st.first + i];
+                cols *= g.ncol[i];
+            }
+            long long most = cols, c = cols;
+            for (int i = g.k - 1; i >= 0; --i) {
+                c /= g.ncol[i];
+                rows *= g.nrow[i];
+                most = std::max(most, c * rows);
+            }
+            g.inner = inner;
+            g.outer = outer;
+            // faster indices per tile: all of them if they fit, or else multiples of
+            // KG_MIN_IC; slower ones until there are ~1024 workgroups, a wave of fibres each
+            const long long fit = KG_TILE / most;
+            long long ic = std::min(inner, fit);
+            if (ic < inner && ic > KG_MIN_IC) ic -= ic % KG_MIN_IC;
+            if (ic > 64 && ic < inner && inner * outer / ic < 512) ic = 64;
+            long long oc = 1;
+            if (ic == inner) {
+                oc = std::max((outer + 1023) / 1024, 64 / std::max(1LL, cols * ic / std::max(1, g.ncol[g.k - 1])));
+                oc = std::max(1LL, std::min({oc, outer, fit / ic}));
+            }
+            g.IC = int(ic);
+            g.OC = int(oc);
+            g.buf = int(most * ic * oc * 9 / 8 + 2);
+            g.chunks = int((inner + ic - 1) / ic);
+            const long long grid = (outer + oc - 1) / oc * g.chunks;
+            const size_t lds = 2 * size_t(g.buf) * sizeof(double);
+            const int nt = most * ic * oc >= 2048 ? KG_THREADS : most * ic * oc >= 512 ? 256 : 64;
+            if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+            if (lds > 65536) {
+                const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_mode_group),
+                                                         hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+                if (e != hipSuccess) return e;
+            }
+            hipLaunchKernelGGL(k_mode_group, dim3(unsigned(grid)), dim3(nt), lds, s, g);
+        }
+        for (int i = st.first; i <= st.last; ++i) ext[i] = nrow[i];
+        cur = out;
         ping ^= 1;
     }
+    return hipGetLastError();
 }
 
 bool kron_args_ok(int k, const int* nrow, const int* ncol, const double* const* A, const double* X, int nvec,
@@ -305,19 +526,19 @@ extern "C" int kmx_kronmult(int k, const int* nrow, const int* ncol, const doubl
     }
     if (nvec == 0) return KMX_OK;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    const long long maxsz = chain_workspace(k, nrow, ncol, nvec);
+    const std::vector<ChainStep> steps = plan_chain(k, nrow, ncol, nvec, X, Y);
     double* buf[2] = {nullptr, nullptr};
-    if (k > 1) {
+    if (steps.size() > 1) {  // intermediates between the launches
+        const long long maxsz = chain_workspace(k, nrow, ncol, nvec);
         if (hipMalloc(&buf[0], sizeof(double) * maxsz) != hipSuccess ||
-            (k > 2 && hipMalloc(&buf[1], sizeof(double) * maxsz) != hipSuccess)) {
+            (steps.size() > 2 && hipMalloc(&buf[1], sizeof(double) * maxsz) != hipSuccess)) {
             hipFree(buf[0]);
             set_error("kmx_kronmult: workspace allocation failed");
             return KMX_E_NOMEM;
         }
     }
-    launch_chain(k, nrow, ncol, A, X, nvec, Y, buf, s);
-    hipError_t e = hipGetLastError();
-    if (k > 1) {
+    const hipError_t e = launch_chain(steps, k, nrow, ncol, A, X, nvec, Y, buf, s);
+    if (buf[0]) {
         hipStreamSynchronize(s);
         hipFree(buf[0]);
         if (buf[1]) hipFree(buf[1]);
@@ -377,8 +598,8 @@ extern "C" int kmx_kronmult_noalloc(int k, const int* nrow, const int* ncol, con
         return KMX_E_HIP;
     }
     double* buf[2] = {base, base + half};
-    launch_chain(k, nrow, ncol, A, X, nvec, Y, buf, reinterpret_cast<hipStream_t>(stream));
-    const hipError_t e = hipGetLastError();
+    const hipError_t e = launch_chain(plan_chain(k, nrow, ncol, nvec, X, Y), k, nrow, ncol, A, X, nvec, Y, buf,
+                                      reinterpret_cast<hipStream_t>(stream));
     if (e != hipSuccess) {
         set_error(std::string("kmx_kronmult_noalloc: ") + hipGetErrorString(e));
         return KMX_E_HIP;

@@ -353,6 +353,8 @@ def kronmult(mats, X, stream=None, noalloc=False, Y=None):
     fn = lib().kmx_kronmult_noalloc if noalloc else lib().kmx_kronmult
     check(fn(k, (C.c_int * k)(*nr), (C.c_int * k)(*nc), (C.c_void_p * k)(*[m.data_ptr() for m in cm]),
              C.c_void_p(xs.data_ptr()), int(nvec), C.c_void_p(y.data_ptr()), _stream(stream)))
+    if stream is not None and not noalloc:
+        check(lib().kmx_sync(_stream(stream)))  # the copies above belong to the current stream
     return y.view(nvec, -1).t()
 
 

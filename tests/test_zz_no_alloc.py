@@ -49,3 +49,47 @@ def test_kronmult_noalloc_matches_allocating_entry(kmx_gpu):
     with pytest.raises(kmx_gpu.KmxError) as e:
         kmx_gpu.kronmult(mats, X, noalloc=True)
     assert e.value.code == _lib.KMX_E_SHAPE
+
+
+@pytest.mark.parametrize("shapes,nvec", [
+    ([(1, 1)], 1), ([(17, 33)], 5), ([(40, 3), (3, 40)], 7),           # more than 16 rows, one mode
+    ([(16, 16), (16, 16), (2, 2)], 3),                                 # 16 rows exactly
+    ([(8, 8)] * 4 + [(2, 2)], 2),                                      # 8192 values: the largest power of two in a tile
+    ([(9, 9)] * 4 + [(2, 2)], 2),                                      # 13122: two launches, the second strided
+    ([(3, 2), (97, 89), (91, 95)], 3),                                 # a mode with ragged runs of the faster values
+    ([(2, 9000)], 2), ([(9000, 2), (2, 3)], 1),                        # a mode beyond the tile: launches of its own
+    ([(2, 2)] * 16, 1),
+])
+def test_kronmult_groups(kmx_gpu, shapes, nvec):
+    """The grouped launches at the edges of their tile and of their 16-row passes, allocating
+    and not, against numpy's products factor by factor: sums of at most 9000 products per
+    factor, so well below 1e-13 relative (2-norm); and Y written over X."""
+    import torch
+
+    rng = np.random.default_rng(len(shapes) * 100 + nvec)
+    mats, X = _case(rng, shapes, nvec)
+    want = X.cpu().numpy()
+    pre = 1
+    for m in mats:
+        a = m.cpu().numpy()
+        want = np.matmul(a, want.reshape(pre, a.shape[1], -1)).reshape(pre * a.shape[0], -1)
+        pre *= a.shape[0]
+    want = want.reshape(pre, nvec)
+    tol = 1e-13 * np.linalg.norm(want)
+    got = kmx_gpu.kronmult(mats, X)
+    assert np.linalg.norm(got.cpu().numpy() - want) <= tol
+    again = kmx_gpu.kronmult(mats, X, noalloc=True)
+    assert torch.equal(again, got)
+    if len(shapes) > 1 and pre == X.shape[0]:
+        import ctypes as C
+
+        from kmx._lib import check, lib
+
+        k = len(mats)
+        xs = X.t().contiguous()
+        cm = [m.t().contiguous() for m in mats]
+        check(lib().kmx_kronmult(k, (C.c_int * k)(*[s[0] for s in shapes]), (C.c_int * k)(*[s[1] for s in shapes]),
+                                 (C.c_void_p * k)(*[m.data_ptr() for m in cm]), C.c_void_p(xs.data_ptr()), nvec,
+                                 C.c_void_p(xs.data_ptr()), C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+        torch.cuda.synchronize()
+        assert torch.equal(xs.view(nvec, -1).t(), got)
