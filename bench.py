@@ -472,7 +472,7 @@ def single_instance_leg(plan, tuned, op, xd, yd, steps, warmup):
 def gemm_leg():
     """kmx_gemm_vbatched (gemm_vbatched.m, FP64, 'N','N', beta = 0) on three batches:
     2,000 GEMMs of 27 x 81 x 27 (a kronmult3 stage at deg 3), 200 of 256^3 and one
-    of 2048^3; host time of the call (it waits for its launch), best of three, and
+    of 2048^3; host time of the call and of its launches (synchronised), best of three, and
     the largest error against torch's FP64 batched product."""
     import torch
 
@@ -523,7 +523,7 @@ def gemm_leg():
     out["kronmult 4 x 8x8, 128 vectors"] = {
         "us": round(best * 1e6, 1), "GBs": round(4 * 2 * 8 * 4096 * 128 / best / 1e9, 1),
         "rel_err_vs_torch_fp64": float((got - ref).abs().max() / ref.abs().max()),
-        "note": "host time of the call (four mode-product launches plus the wrapper's column-major copies)"}
+        "note": "host time of the call (one launch for the four mode products plus the wrapper's column-major copies)"}
     return out
 
 

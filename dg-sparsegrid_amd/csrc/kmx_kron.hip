@@ -3,6 +3,7 @@
 //   kmx_gemm_vbatched        variable-size batched GEMM (Kronmult/gemm_vbatched.m)
 //   kmx_kronmult_batch_plan  the per-stage GEMM lists of Kronmult/kronmult{k}_batch.m
 #include "kmx_internal.h"
+#include "kmx_mma64.h"
 
 #include <algorithm>
 #include <cstdio>
@@ -42,15 +43,17 @@ __global__ void __launch_bounds__(256) k_mode_product(ModeArgs m) {
 // values of the slower indices and IC of the faster ones, every value of the group's
 // modes in LDS (two buffers) and contracts them last first; each tensor value is read
 // and written in HBM once per group instead of once per mode.  A thread takes fibres
-// along the mode: the inputs come one by one from LDS, the factor's column -- the same
-// for every lane -- through the scalar cache, and up to 16 outputs accumulate in
-// registers (1 LDS read per NR FMAs; one thread per output read two values per FMA).
+// along the mode: the inputs and the factor's columns (the same for every lane) come
+// from LDS and up to 16 outputs accumulate in registers.  Factors of more than KG_FACTOR
+// values together are read through the scalar cache instead, whose loads cannot be
+// waited for one by one (the chain below: 17.0 us so, 16.1 us from LDS).
 // Every output sums its products in column order with FMAs from zero, as the one-mode
 // kernel does: the results are bit-identical however the chain is grouped.  LDS index
 // i sits at i + i / 8: fibres of the fastest mode, ncol apart, spread over the banks.
-// Four 8 x 8 factors on 128 vectors: 4 launches, 32 us of kernel time -> 1.
+// Four 8 x 8 factors on 128 vectors: 4 launches, 32 us of kernel time, now 1 of 16 us.
 constexpr int KG_THREADS = 512;
-constexpr int KG_TILE = 8704;   // values of a tile at most: 2 buffers x 9/8 x 8 bytes = 153 KB of the 160 KB
+constexpr int KG_TILE = 8448;   // values of a tile at most: 2 buffers x 9/8 x 8 bytes = 152 KB of the 160 KB
+constexpr int KG_FACTOR = 1000;  // values of the factors kept in LDS
 constexpr int KG_MIN_IC = 8;    // contiguous values per access at least when the modes are strided
 struct GroupArgs {
     const double* in;
@@ -61,11 +64,13 @@ struct GroupArgs {
     long long outer;  // extent of the slower modes times nvec
     int k, OC, IC, buf;  // buf: doubles of one LDS buffer
     int chunks;          // workgroups along inner
+    int foff[KMX_KRON_MAX_FACTORS], nfac;  // the factors' places in LDS, their values (0: not kept there)
 };
 __device__ __forceinline__ int kg_at(int i) { return i + (i >> 3); }
+typedef const __attribute__((address_space(4))) double* kg_factor;  // read through the scalar cache
 
-template <int NR>
-__device__ __forceinline__ void kg_fibre(const double* __restrict__ A, int nrow, int ncol, const double* __restrict__ src,
+template <int NR, class P>
+__device__ __forceinline__ void kg_fibre(P A, int nrow, int ncol, const double* __restrict__ src,
                                          double* __restrict__ dst, int ib, int ob, int inner) {
     double acc[NR];
 #pragma unroll
@@ -74,18 +79,44 @@ __device__ __forceinline__ void kg_fibre(const double* __restrict__ A, int nrow,
     for (int b = 0; b < ncol; ++b) {
         const double x = src[kg_at(ib + b * inner)];
 #pragma unroll
-        for (int a = 0; a < NR; ++a) acc[a] = __builtin_fma(A[(long long)b * nrow + a], x, acc[a]);
+        for (int a = 0; a < NR; ++a) acc[a] = __builtin_fma(A[b * nrow + a], x, acc[a]);
     }
 #pragma unroll
     for (int a = 0; a < NR; ++a) dst[kg_at(ob + a * inner)] = acc[a];
 }
 
-template <int NR>
-__device__ __forceinline__ void kg_mode(const double* __restrict__ A, int nrow, int ncol, int a0,
+template <int NR, class P>
+__device__ __forceinline__ void kg_mode(P A, int nrow, int ncol, int a0,
                                         const double* __restrict__ src, double* __restrict__ dst, int nf, int inner) {
     for (int f = threadIdx.x; f < nf; f += blockDim.x) {
         const int o = f / inner, s = f - o * inner;
         kg_fibre<NR>(A + a0, nrow, ncol, src, dst, o * ncol * inner + s, (o * nrow + a0) * inner + s, inner);
+    }
+}
+
+// One mode of the tile: every fibre, 16 rows of the factor at a time.
+template <class P>
+__device__ __forceinline__ void kg_rows(P A, int nr, int nc, const double* __restrict__ src, double* __restrict__ dst,
+                                        int nf, int fast) {
+    for (int a0 = 0; a0 < nr; a0 += 16) {
+        switch (min(16, nr - a0)) {
+            case 1: kg_mode<1>(A, nr, nc, a0, src, dst, nf, fast); break;
+            case 2: kg_mode<2>(A, nr, nc, a0, src, dst, nf, fast); break;
+            case 3: kg_mode<3>(A, nr, nc, a0, src, dst, nf, fast); break;
+            case 4: kg_mode<4>(A, nr, nc, a0, src, dst, nf, fast); break;
+            case 5: kg_mode<5>(A, nr, nc, a0, src, dst, nf, fast); break;
+            case 6: kg_mode<6>(A, nr, nc, a0, src, dst, nf, fast); break;
+            case 7: kg_mode<7>(A, nr, nc, a0, src, dst, nf, fast); break;
+            case 8: kg_mode<8>(A, nr, nc, a0, src, dst, nf, fast); break;
+            case 9: kg_mode<9>(A, nr, nc, a0, src, dst, nf, fast); break;
+            case 10: kg_mode<10>(A, nr, nc, a0, src, dst, nf, fast); break;
+            case 11: kg_mode<11>(A, nr, nc, a0, src, dst, nf, fast); break;
+            case 12: kg_mode<12>(A, nr, nc, a0, src, dst, nf, fast); break;
+            case 13: kg_mode<13>(A, nr, nc, a0, src, dst, nf, fast); break;
+            case 14: kg_mode<14>(A, nr, nc, a0, src, dst, nf, fast); break;
+            case 15: kg_mode<15>(A, nr, nc, a0, src, dst, nf, fast); break;
+            default: kg_mode<16>(A, nr, nc, a0, src, dst, nf, fast); break;
+        }
     }
 }
 
@@ -102,14 +133,31 @@ __global__ void __launch_bounds__(KG_THREADS) k_mode_group(GroupArgs g) {
     }
     double* src = kg_lds;
     double* dst = kg_lds + g.buf;
-    {  // the tile in: value p of the modes, s of the faster indices (IC = inner unless OC = 1)
-        const double* in = g.in + o0 * pin * g.inner + s0;
-        const int n = oc * pin * g.IC;
-        for (int i = threadIdx.x; i < n; i += blockDim.x) {
-            const int p = i / g.IC, s = i - p * g.IC;
-            src[kg_at(i)] = s < ic ? in[(long long)p * g.inner + s] : 0.0;
+    double* fac = kg_lds + 2 * g.buf;
+    const bool staged = g.nfac > 0;
+    const int nt = blockDim.x;
+    // the tile in: value p of the modes, s of the faster indices (IC = inner unless OC = 1),
+    // eight loads of a thread in flight
+    typedef const __attribute__((address_space(1))) double* gptr;
+    const gptr in = (gptr)(g.in + o0 * pin * g.inner + s0);
+    const int n_in = oc * pin * g.IC;
+    for (int i0 = threadIdx.x; i0 < n_in; i0 += 8 * nt) {
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int i = min(i0 + u * nt, n_in - 1);
+            const int p = g.IC == 1 ? i : i / g.IC, s = i - p * g.IC;
+            v[u] = in[(long long)p * g.inner + min(s, ic - 1)];
         }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (i0 + u * nt < n_in) src[kg_at(i0 + u * nt)] = v[u];
     }
+    if (staged)
+        for (int d = 0; d < g.k; ++d) {
+            const gptr A = (gptr)g.A[d];
+            for (int i = threadIdx.x; i < g.nrow[d] * g.ncol[d]; i += nt) fac[g.foff[d] + i] = A[i];
+        }
     __syncthreads();
     int fast = g.IC;  // extent of the faster indices inside the tile
     int slow = oc * pin;
@@ -117,36 +165,19 @@ __global__ void __launch_bounds__(KG_THREADS) k_mode_group(GroupArgs g) {
         const int nr = g.nrow[d], nc = g.ncol[d];
         slow /= nc;
         const int nf = slow * fast;
-        for (int a0 = 0; a0 < nr; a0 += 16) {
-            switch (min(16, nr - a0)) {
-                case 1: kg_mode<1>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
-                case 2: kg_mode<2>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
-                case 3: kg_mode<3>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
-                case 4: kg_mode<4>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
-                case 5: kg_mode<5>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
-                case 6: kg_mode<6>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
-                case 7: kg_mode<7>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
-                case 8: kg_mode<8>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
-                case 9: kg_mode<9>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
-                case 10: kg_mode<10>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
-                case 11: kg_mode<11>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
-                case 12: kg_mode<12>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
-                case 13: kg_mode<13>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
-                case 14: kg_mode<14>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
-                case 15: kg_mode<15>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
-                default: kg_mode<16>(g.A[d], nr, nc, a0, src, dst, nf, fast); break;
-            }
-        }
+        if (staged) kg_rows(fac + g.foff[d], nr, nc, src, dst, nf, fast);
+        else kg_rows((kg_factor)g.A[d], nr, nc, src, dst, nf, fast);
         fast *= nr;
         __syncthreads();
         double* t = src;
         src = dst;
         dst = t;
     }
-    double* out = g.out + o0 * pout * g.inner + s0;
+    __attribute__((address_space(1))) double* out =
+        (__attribute__((address_space(1))) double*)(g.out + o0 * pout * g.inner + s0);
     const int n = oc * pout * g.IC;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        const int p = i / g.IC, s = i - p * g.IC;
+    for (int i = threadIdx.x; i < n; i += nt) {
+        const int p = g.IC == 1 ? i : i / g.IC, s = i - p * g.IC;
         if (s < ic) out[(long long)p * g.inner + s] = src[kg_at(i)];
     }
 }
@@ -157,70 +188,52 @@ struct GemmDescDev {
     double* C;
     int m, n, k, lda, ldb, ldc;
 };
+// Descriptors that travel with the launch (kernel arguments are limited to 4 KB)
+constexpr int GV_CHUNK = 80;
+// Batches of up to this many GEMMs run in chunks; beyond, one launch over a device table
+// (a launch of 80 small products is ~5 us, the table's set-up ~40 us)
+constexpr int GV_MAX_CHUNKED = 8 * GV_CHUNK;
+struct GemmChunk {
+    GemmDescDev d[GV_CHUNK];
+};
 
 // The batch's GEMMs in 64 x 64 tiles of C: workgroup (g, t) takes tiles t, t +
-// gridDim.y, ... of GEMM g (row-tile fastest).  k runs in chunks of 16: the chunk's
-// 64 x 16 values of op(A) and 16 x 64 of op(B) are staged in LDS, each loaded
-// along the matrix's contiguous index, and each thread accumulates a 4 x 4 set of
-// C entries (rows tx + 16 r, columns ty + 16 c) over the chunk.  Every entry sums
-// its k products in order with FMAs, then C = alpha sum + beta C (C not read when
-// beta = 0), as the reference's gemm does entry by entry.
-constexpr int GV_T = 64, GV_K = 16;
-__global__ void __launch_bounds__(256) k_gemm_vbatched(const GemmDescDev* __restrict__ d, int count, int ta, int tb,
-                                                       double alpha, double beta) {
-    __shared__ double As[GV_K][GV_T + 1];  // As[l][i] = op(A)(i0 + i, l0 + l)
-    __shared__ double Bs[GV_K][GV_T + 1];  // Bs[l][j] = op(B)(l0 + l, j0 + j)
-    const int g = blockIdx.x;
-    if (g >= count) return;
-    const GemmDescDev q = d[g];
+// gridDim.y, ... of GEMM g (row-tile fastest), on the FP64 matrix cores
+// (kmx_mma64.h).  Every entry sums its k products in order with FMAs, then C = alpha
+// sum + beta C (C not read when beta = 0), as the reference's gemm does entry by
+// entry.  FP64: 200 ragged products of 33..256 in 84 us of kernel time (121 us with VALU
+// FMAs; a workgroup's time is its k), 2048^3 at 51 TFLOP/s (22), 80 x 256^3 at 37 (23).
+constexpr int GV_T = 64;
+template <bool TA, bool TB>
+__device__ __forceinline__ void gemm_tiles(const GemmDescDev& d, double alpha, double beta, double* lds) {
+    const GemmDescDev q = d;
     const int mt = (q.m + GV_T - 1) / GV_T, nt = (q.n + GV_T - 1) / GV_T;
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    for (int tile = blockIdx.y; tile < mt * nt; tile += gridDim.y) {
-        const int i0 = (tile % mt) * GV_T, j0 = (tile / mt) * GV_T;
-        double acc[4][4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int c = 0; c < 4; ++c) acc[r][c] = 0.0;
-        for (int l0 = 0; l0 < q.k; l0 += GV_K) {
-            for (int t = threadIdx.x; t < GV_T * GV_K; t += 256) {
-                const int ii = ta ? t / GV_K : t % GV_T, ll = ta ? t % GV_K : t / GV_T;
-                const int i = i0 + ii, l = l0 + ll;
-                As[ll][ii] = (i < q.m && l < q.k) ? (ta ? q.A[(long long)i * q.lda + l] : q.A[(long long)l * q.lda + i])
-                                                  : 0.0;
-            }
-            for (int t = threadIdx.x; t < GV_T * GV_K; t += 256) {
-                const int jj = tb ? t % GV_T : t / GV_K, ll = tb ? t / GV_T : t % GV_K;
-                const int j = j0 + jj, l = l0 + ll;
-                Bs[ll][jj] = (j < q.n && l < q.k) ? (tb ? q.B[(long long)l * q.ldb + j] : q.B[(long long)j * q.ldb + l])
-                                                  : 0.0;
-            }
-            __syncthreads();
-            const int lk = min(GV_K, q.k - l0);
-            for (int l = 0; l < lk; ++l) {
-                double a[4], b[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) a[r] = As[l][tx + 16 * r];
-#pragma unroll
-                for (int c = 0; c < 4; ++c) b[c] = Bs[l][ty + 16 * c];
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) acc[r][c] = __builtin_fma(a[r], b[c], acc[r][c]);
-            }
-            __syncthreads();  // the chunk's reads before the next chunk's stores
-        }
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int i = i0 + tx + 16 * r, j = j0 + ty + 16 * c;
-                if (i < q.m && j < q.n) {
-                    double& cv = q.C[(long long)j * q.ldc + i];
-                    cv = (beta == 0.0 ? 0.0 : beta * cv) + alpha * acc[r][c];
-                }
-            }
+    const long long tiles = (long long)mt * nt;
+    for (long long tile = blockIdx.y; tile < tiles; tile += gridDim.y) {
+        const int i0 = int(tile % mt) * GV_T, j0 = int(tile / mt) * GV_T;
+        // loads run along each matrix's contiguous index: i or k of A, k or j of B
+        const double* A = TA ? q.A + (long long)i0 * q.lda : q.A + i0;
+        const double* B = TB ? q.B + j0 : q.B + (long long)j0 * q.ldb;
+        double* C = q.C + (long long)j0 * q.ldc + i0;
+        Mma64Strided<Mma64Map<64, 16, TA>> la(A, TA ? q.lda : 1, TA ? 1 : q.lda, q.m - i0, q.k);
+        Mma64Strided<Mma64Map<64, 16, !TB>> lb(B, TB ? 1 : q.ldb, TB ? q.ldb : 1, q.n - j0, q.k);
+        auto st = [&](int i, int j, double v) {
+            double& c = C[(long long)j * q.ldc + i];
+            c = (beta == 0.0 ? 0.0 : beta * c) + alpha * v;
+        };
+        mma64_tile<64, 16>(q.m - i0, q.n - j0, q.k, la, lb, st, lds);
+        __syncthreads();  // a next tile's first chunk after this one's last reads
     }
+}
+template <bool TA, bool TB>
+__global__ void __launch_bounds__(256, 2) k_gemm_chunk(GemmChunk c, double alpha, double beta) {
+    __shared__ double lds[mma64_lds<64, 16>()];
+    gemm_tiles<TA, TB>(c.d[blockIdx.x], alpha, beta, lds);
+}
+template <bool TA, bool TB>
+__global__ void __launch_bounds__(256, 2) k_gemm_vbatched(const GemmDescDev* __restrict__ d, double alpha, double beta) {
+    __shared__ double lds[mma64_lds<64, 16>()];
+    gemm_tiles<TA, TB>(d[blockIdx.x], alpha, beta, lds);
 }
 
 // ---- flops_kron{k} (Kronmult/flops_kron2.m:22-46, flops_kron3..6.m): cost of the
@@ -491,7 +504,13 @@ hipError_t launch_chain(const std::vector<ChainStep>& steps, int k, const int* n
             g.buf = int(most * ic * oc * 9 / 8 + 2);
             g.chunks = int((inner + ic - 1) / ic);
             const long long grid = (outer + oc - 1) / oc * g.chunks;
-            const size_t lds = 2 * size_t(g.buf) * sizeof(double);
+            g.nfac = 0;
+            for (int i = 0; i < g.k; ++i) {
+                g.foff[i] = g.nfac;
+                g.nfac = int(std::min<long long>(KG_FACTOR + 1LL, g.nfac + (long long)g.nrow[i] * g.ncol[i]));
+            }
+            if (g.nfac > KG_FACTOR) g.nfac = 0;
+            const size_t lds = (2 * size_t(g.buf) + size_t(g.nfac)) * sizeof(double);
             const int nt = most * ic * oc >= 2048 ? KG_THREADS : most * ic * oc >= 512 ? 256 : 64;
             if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
             if (lds > 65536) {
@@ -636,17 +655,45 @@ extern "C" int kmx_gemm_vbatched(char transA, char transB, const int* m, const i
         h[i] = GemmDescDev{A[i], B[i], C[i], m[i], n[i], k[i], lda[i], ldb[i], ldc[i]};
     }
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    // C tiles of the largest of GEMMs [i0, i1) (grid y; more loop)
+    auto tiles_of = [&](int i0, int i1) {
+        long long tiles = 1;
+        for (int i = i0; i < i1; ++i)
+            tiles = std::max(tiles, (long long)((h[i].m + 63) / 64) * ((h[i].n + 63) / 64));
+        return unsigned(std::min<long long>(tiles, 65535));
+    };
+    const bool ta = tr(transA), tb = tr(transB);
+    if (count <= GV_MAX_CHUNKED) {
+        // Descriptors as kernel arguments, GV_CHUNK a launch: no table to allocate, copy,
+        // wait for and free (some 40 us a call whatever its size).  Longest k first: a
+        // workgroup's time goes with k, so a launch holds workgroups of about one length.
+        std::stable_sort(h.begin(), h.end(), [](const GemmDescDev& u, const GemmDescDev& v) { return u.k > v.k; });
+        const int launches = (count + GV_CHUNK - 1) / GV_CHUNK;
+        for (int l = 0; l < launches; ++l) {
+            const int i0 = int((long long)count * l / launches), i1 = int((long long)count * (l + 1) / launches);
+            GemmChunk c;
+            std::copy(h.begin() + i0, h.begin() + i1, c.d);
+            const dim3 grid(unsigned(i1 - i0), tiles_of(i0, i1));
+            auto* kern = ta ? (tb ? k_gemm_chunk<true, true> : k_gemm_chunk<true, false>)
+                            : (tb ? k_gemm_chunk<false, true> : k_gemm_chunk<false, false>);
+            hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, c, alpha, beta);
+        }
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) {
+            set_error(std::string("kmx_gemm_vbatched: ") + hipGetErrorString(e));
+            return KMX_E_HIP;
+        }
+        return KMX_OK;
+    }
     GemmDescDev* d = nullptr;
     if (hipMalloc(&d, sizeof(GemmDescDev) * count) != hipSuccess) {
         set_error("kmx_gemm_vbatched: descriptor allocation failed");
         return KMX_E_NOMEM;
     }
     hipMemcpyAsync(d, h.data(), sizeof(GemmDescDev) * count, hipMemcpyHostToDevice, s);
-    long long tiles = 1;  // C tiles of the batch's largest GEMM (grid y; more loop)
-    for (int i = 0; i < count; ++i)
-        tiles = std::max(tiles, (long long)((m[i] + 63) / 64) * ((n[i] + 63) / 64));
-    hipLaunchKernelGGL(k_gemm_vbatched, dim3(unsigned(count), unsigned(std::min<long long>(tiles, 65535))), dim3(256),
-                       0, s, d, count, int(tr(transA)), int(tr(transB)), alpha, beta);
+    auto* kern = ta ? (tb ? k_gemm_vbatched<true, true> : k_gemm_vbatched<true, false>)
+                    : (tb ? k_gemm_vbatched<false, true> : k_gemm_vbatched<false, false>);
+    hipLaunchKernelGGL(kern, dim3(unsigned(count), tiles_of(0, count)), dim3(256), 0, s, d, alpha, beta);
     hipError_t e = hipGetLastError();
     hipStreamSynchronize(s);
     hipFree(d);

@@ -16,8 +16,8 @@
 // product per level tuple added into the output instead -- 84 tuples x 4 launches
 // on a 3D lev 6 grid, each re-reading and adding all 192^3 points -- took 6.5 ms.)
 // The products run on the FP64 matrix cores (kmx_mma64.h).  3D lev 6 deg 3 (192^3
-// points): 0.162 ms, error against 64 bits 3.5e-16 (4.6e-16 before); the last stage,
-// 2.7 GFLOP of dense products, is most of it.  Same terms, summed in another order.
+// points): 0.106 ms, error against 64 bits 3.5e-16 (4.6e-16 before); the last stage,
+// 2.7 GFLOP of dense products, is 71 us of it.  Same terms, summed in another order.
 #include "kmx_internal.h"
 #include "kmx_mma64.h"
 
@@ -53,36 +53,89 @@ __device__ __forceinline__ void split_k(int k, const StageArgs& a, int& c, int& 
     b = k - c * a.deg;
 }
 
+// A list of k positions of a node, 64 at a time, one per lane (each lane works its
+// own out once); the next 64 are fetched while these are used.  Chunks are read in
+// order and never straddle a block of 64.
+template <class F>
+struct KList {
+    const F f;
+    const int K;
+    int cur, nxt, blk;
+    __device__ __forceinline__ KList(const F& fn, int k) : f(fn), K(k), blk(0) {
+        const int l = int(threadIdx.x) & 63;
+        cur = f(min(l, K - 1));
+        nxt = f(min(64 + l, K - 1));
+    }
+    __device__ __forceinline__ void to(int k0) {
+        if (k0 < K && k0 >> 6 != blk) {
+            blk = k0 >> 6;
+            cur = nxt;
+            nxt = f(min(64 * (blk + 1) + (int(threadIdx.x) & 63), K - 1));
+        }
+    }
+    __device__ __forceinline__ int at(int k) const { return __builtin_amdgcn_readlane(cur, k & 63); }
+};
+
+// Operand whose k-th line (64 consecutive values, one k per wave) starts at base +
+// line(k) ld.
+template <class M, class F>
+struct LineOperand {
+    using Map = M;
+    static_assert(M::WAVEK, "one k per wave");
+    KList<F> list;
+    mma64_gptr at;  // the lane's value of line 0
+    long long ld;
+    __device__ __forceinline__ LineOperand(const F& line, const double* b, long long l, int rows, int K)
+        : list(line, K), at(mma64_global(b) + min(int(threadIdx.x) & 63, rows - 1)), ld(l) {}
+    __device__ __forceinline__ void load(int k0, double (&x)[M::N]) {
+        list.to(k0);
+#pragma unroll
+        for (int u = 0; u < M::N; ++u) x[u] = at[list.at(min(k0 + M::k(u), list.K - 1)) * ld];
+    }
+};
+
+// The coefficients of a node's elements: rows beta, value (beta, k) of element c(k).
+template <class M>
+struct CoefOperand {
+    using Map = M;
+    const StageArgs& a;
+    int c0, K, beta0, rows;
+    __device__ __forceinline__ void load(int k0, double (&x)[M::N]) {
+#pragma unroll
+        for (int u = 0; u < M::N; ++u) {
+            int c, b;
+            split_k(min(k0 + M::k(u), K - 1), a, c, b);
+            x[u] = mma64_global(a.in)[(long long)a.row[c0 + c] * a.B + (beta0 + min(M::row(u), rows - 1)) * a.deg + b];
+        }
+    }
+};
+
 // The last dimension: Z_d[node; beta; p] = sum_k f[element(k), beta, b(k)] Meval_d(p, k).
 // Rows beta (few), columns p; a chunk of 32 k keeps enough loads in flight for the
 // long child lists of the low prefixes.
-__global__ void __launch_bounds__(256) k_rs_last(StageArgs a) {
+__global__ void __launch_bounds__(256, 2) k_rs_last(StageArgs a) {
     __shared__ double lds[mma64_lds<16, 32>()];
     const int tiles = a.mt * a.nt;
     const int q = int(blockIdx.x) / tiles, t = int(blockIdx.x) - q * tiles;
     if (q >= a.items) return;
     const int i0 = 16 * (t % a.mt), j0 = 64 * (t / a.mt);
     const int c0 = a.cptr[q], K = (a.cptr[q + 1] - c0) * a.deg;
-    const int deg = a.deg;
-    auto fa = [&](int i, int k) {
+    auto column = [&](int k) {
         int c, b;
         split_k(k, a, c, b);
-        return a.in[(long long)a.row[c0 + c] * a.B + (i0 + i) * deg + b];
+        return a.col[c0 + c] + b;
     };
-    auto fb = [&](int k, int j) {
-        int c, b;
-        split_k(k, a, c, b);
-        return a.A[(long long)(a.col[c0 + c] + b) * a.M + j0 + j];
-    };
+    CoefOperand<Mma64Map<16, 32, false>> la{a, c0, K, i0, a.nbeta - i0};
+    LineOperand<Mma64Map<64, 32, false>, decltype(column)> lb(column, a.A + j0, a.M, a.M - j0, K);
     double* out = a.out + (long long)q * a.nbeta * a.M;
     auto st = [&](int i, int j, double v) { out[(long long)(i0 + i) * a.M + j0 + j] = v; };
-    mma64_tile<16, 32>(a.nbeta - i0, a.M - j0, K, fa, fb, st, lds);
+    mma64_tile<16, 32>(a.nbeta - i0, a.M - j0, K, la, lb, st, lds);
 }
 
 // Dimension k < d: Z_k[node; beta; p, r] = sum_k Meval_k(p, k) Z_{k+1}[child(k); beta, b(k); r].
 // The column tiles of an item are dealt so that the workgroups of one column tile
 // (its row tiles, which read the same values of Z_{k+1}) share an XCD's L2.
-__global__ void __launch_bounds__(256) k_rs_mode(StageArgs a) {
+__global__ void __launch_bounds__(256, 2) k_rs_mode(StageArgs a) {
     __shared__ double lds[mma64_lds<64, 16>()];
     const int per = a.xcd ? a.mt * ((a.nt + 7) / 8) * 8 : a.mt * a.nt;
     const int item = int(blockIdx.x) / per, t = int(blockIdx.x) - item * per;
@@ -100,22 +153,23 @@ __global__ void __launch_bounds__(256) k_rs_mode(StageArgs a) {
     const int i0 = 64 * rt;
     const long long j0 = 64LL * ct;
     const int c0 = a.cptr[q], K = (a.cptr[q + 1] - c0) * a.deg;
-    const int deg = a.deg;
-    auto fa = [&](int i, int k) {
+    const int n = int(min(64LL, a.R - j0));
+    auto column = [&](int k) {
         int c, b;
         split_k(k, a, c, b);
-        return a.A[(long long)(a.col[c0 + c] + b) * a.M + i0 + i];
+        return a.col[c0 + c] + b;
     };
-    const double* in = a.in + ((long long)c0 * a.nbeta + beta) * deg * a.R + j0;
-    const long long cs = (long long)a.nbeta * deg * a.R;
-    auto fb = [&](int k, int j) {
+    auto line = [&](int k) {  // of Z_{k+1}: child, beta, b
         int c, b;
         split_k(k, a, c, b);
-        return in[c * cs + b * a.R + j];
+        return ((c0 + c) * a.nbeta + beta) * a.deg + b;
     };
+    using Map = Mma64Map<64, 16, false>;
+    LineOperand<Map, decltype(column)> la(column, a.A + i0, a.M, a.M - i0, K);
+    LineOperand<Map, decltype(line)> lb(line, a.in + j0, a.R, n, K);
     double* out = a.out + (long long)item * a.M * a.R + j0;
     auto st = [&](int i, int j, double v) { out[(long long)(i0 + i) * a.R + j] = v; };
-    mma64_tile<64, 16>(a.M - i0, int(min(64LL, a.R - j0)), K, fa, fb, st, lds);
+    mma64_tile<64, 16>(a.M - i0, n, K, la, lb, st, lds);
 }
 
 __global__ void __launch_bounds__(256) k_zero(double* y, long long n) {

@@ -258,7 +258,9 @@ int kmx_arnoldi_step(int64_t n, int k, double* V, const double* u, double s0, do
  * Kronmult/kronmult{k}.m; k > 6 as kron_multd.m:43-86's recursion).
  * A[i]: DEVICE pointer, column-major nrow[i] x ncol[i] (rectangular allowed);
  * X: DEVICE, prod(ncol) x nvec column-major; Y: DEVICE, prod(nrow) x nvec.
- * nrow/ncol/A are host arrays of length k. */
+ * nrow/ncol/A are host arrays of length k.  On `stream`; a chain whose values fit one
+ * launch's tile (up to 8448 per vector) is asynchronous, a longer one allocates its
+ * intermediates and waits for the stream. */
 #define KMX_KRON_MAX_FACTORS 16
 int kmx_kronmult(int k, const int* nrow, const int* ncol, const double* const* A, const double* X, int nvec,
                  double* Y, void* stream);
@@ -279,7 +281,9 @@ int kmx_kronmult_noalloc(int k, const int* nrow, const int* ncol, const double* 
  * C_i = alpha*op(A_i)*op(B_i) + beta*C_i with op from transA/transB ('N'/'T'),
  * m_i x k_i times k_i x n_i.  k is taken from k[] (the reference reads nlist at
  * gemm_vbatched.m:25; identical for its square use).  Size/ld arrays and the
- * pointer arrays are HOST arrays; the pointers address DEVICE memory. */
+ * pointer arrays are HOST arrays (free after the call); the pointers address DEVICE
+ * memory.  On `stream`; batches of up to 640 products are asynchronous, larger ones
+ * allocate a descriptor table and wait for the stream. */
 int kmx_gemm_vbatched(char transA, char transB, const int* m, const int* n, const int* k, double alpha,
                       const double* const* A, const int* lda, const double* const* B, const int* ldb, double beta,
                       double* const* C, const int* ldc, int count, void* stream);

@@ -395,3 +395,40 @@ def test_plain_c_caller(kmx_gpu):
     r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     print(r.stdout, r.stderr)
     assert r.returncode == 0 and "kmx_demo ok" in r.stdout
+
+
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("N", "T"), ("T", "N"), ("T", "T")])
+@pytest.mark.parametrize("count", [1, 80, 81, 641])
+def test_gemm_vbatched_tile_edges(kmx_gpu, ta, tb, count):
+    """Sizes at the edges of the 64 x 64 tiles, their 16 x 16 parts and the k chunks of 16
+    (one, two, three and their remainders), leading dimensions above the sizes, in batches
+    of one launch, several and a device table; against torch's FP64 products.  At most
+    65 products a sum: 65 eps relative to the sums of absolute values, bar 1e-13."""
+    import torch
+
+    edges = [1, 2, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65]
+    rng = np.random.default_rng(count)
+    ms, ns, ks = (rng.choice(edges, size=count).tolist() for _ in range(3))
+    ks[0] = 0 if count > 1 else 33
+    A, B, Cm, ref, lda, ldb, ldc = [], [], [], [], [], [], []
+    for m, n, k in zip(ms, ns, ks):
+        ra, ca = (k, m) if ta == "T" else (m, k)
+        rb, cb = (n, k) if tb == "T" else (k, n)
+        lda.append(ra + 3)
+        ldb.append(rb + 1)
+        ldc.append(m + 2)
+        a, b, c = (torch.from_numpy(rng.standard_normal((max(1, cols), ld))).cuda()
+                   for cols, ld in ((ca, lda[-1]), (cb, ldb[-1]), (n, ldc[-1])))
+        A.append(a)
+        B.append(b)
+        Cm.append(c)
+        am, bm = a[:ca, :ra].t().contiguous(), b[:cb, :rb].t().contiguous()  # column-major storage
+        am, bm = (am.t() if ta == "T" else am), (bm.t() if tb == "T" else bm)
+        r = c.clone()
+        r[:, :m] = 0.5 * c[:, :m] - 1.5 * torch.mm(am.contiguous(), bm.contiguous()).t()
+        ref.append(r)
+    kmx_gpu.gemm_vbatched(ta, tb, ms, ns, ks, -1.5, A, lda, B, ldb, 0.5, Cm, ldc)
+    torch.cuda.synchronize()
+    for i, (c, r) in enumerate(zip(Cm, ref)):
+        scale = max(1.0, float(r.abs().max()))
+        assert float((c - r).abs().max()) <= 1e-13 * scale, (i, ms[i], ns[i], ks[i])
