@@ -64,6 +64,7 @@ void free_plan(kmx_plan* p) {
     dfree(p->d_blkT32);
     dfree(p->d_x_host_stage);
     dfree(p->d_y_host_stage);
+    kmx_factor_free(p);
     kmx_sweep_free(p);
     kmx_blocks_free(p);
 }
@@ -260,6 +261,7 @@ int kmx_plan_create(const kmx_plan_desc* desc, kmx_plan** out) {
             std::vector<const double*> mats(desc->mats, desc->mats + size_t(T) * D);
             kmx_blocks_build(p, idx, rp, cols, mats.data());
         }
+        if (!kmx_sweep_separable(p)) kmx_factor_build(p, idx, rp, cols);
         kmx_plan_apply_cached_variants(p);
         *out = p;
         return KMX_OK;
@@ -305,6 +307,7 @@ int kmx_plan_update_term(kmx_plan* p, int term, int dim, const double* mat, void
         }
         // the float staging vectors die here: wait for the copies that read them
         hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
+        kmx_factor_term_updated(p, term, dim, s);
         kmx_blocks_update_term(p, term, dim, mat, s);
         kmx_sweep_term_updated(p, term, dim);
         ++p->version;

@@ -141,6 +141,12 @@ int kmx_launch_apply(kmx_plan* p, bool transpose, const double* x, double* y, in
         if (kmx_sweep_has_transpose(p)) return kmx_sweep_apply_transpose(p, prec_slot(prec), x, y, s);
     }
     kmx_variant v = p->var[prec_slot(prec)];
+    if (prec == KMX_PREC_FP64 && !v.pairs && kmx_factor_ok(p, transpose)) {
+        KArgs<double> k;
+        fill_args(k, p, transpose, x, y);
+        const int rc = kmx_factor_apply(p, transpose, k, s);
+        if (rc != 0) return rc < 0 ? rc : KMX_OK;
+    }
     return launch_variant(p, transpose, x, y, prec, v, s);
 }
 
@@ -257,7 +263,16 @@ extern "C" int kmx_plan_autotune(kmx_plan* p, void* stream) {
         }
         if (rc != KMX_OK) break;
         p->var[prec_slot(prec)] = bestv;
-        // 2. the dimension-sweep path against it
+        // 2. the factored sum (FP64) against it
+        if (prec == KMX_PREC_FP64 && kmx_factor_ok(p, false)) {
+            float ms;
+            rc = time_calls([&] { return kmx_launch_apply(p, false, x, y, prec, s); }, s, e0, e1, ms);
+            if (rc != KMX_OK) break;
+            if (ms < best) best = ms;
+            else bestv.pairs = 1;
+            p->var[prec_slot(prec)] = bestv;
+        }
+        // 3. the dimension-sweep path against both
         if (p->sw && (prec == KMX_PREC_FP32 || kmx_sweep_fp64_ok(p))) {
             p->var[prec_slot(prec)].sweep = 1;
             float ms;

@@ -56,6 +56,7 @@ struct kmx_variant {
     int lds = -1;
     int kind = 0;          // 0: one lane per pair, 1: pair split over deg lanes
     int sweep = 0;         // 1: the dimension-sweep path (when the plan has one)
+    int pairs = 0;         // 1: pair by pair even where the factored apply serves the plan
 };
 
 // Level-block structure of a plan: elements grouped by their level
@@ -77,7 +78,8 @@ struct kmx_blockset {
     float* d_mat32 = nullptr;
 };
 
-struct kmx_sweep;  // dimension-sweep path (kmx_sweep.hip)
+struct kmx_sweep;   // dimension-sweep path (kmx_sweep.hip)
+struct kmx_factor;  // factored pair sum (kmx_factor.hip)
 
 struct kmx_plan {
     int D = 0, deg = 0, N = 0, T = 0, B = 0;
@@ -121,6 +123,7 @@ struct kmx_plan {
 
     kmx_blockset* bs = nullptr;  // level-block structure (null unless KMX_PLAN_LEVEL_BLOCKS)
     kmx_sweep* sw = nullptr;     // dimension-sweep path (null when the structure does not allow it)
+    kmx_factor* fac = nullptr;   // FP64 applies with the pair sum factored (null: pair by pair)
 };
 
 // Launchers (kmx_apply.hip)
@@ -134,6 +137,16 @@ void kmx_blocks_build(kmx_plan* p, const std::vector<int>& idx, const std::vecto
 void kmx_blocks_update_term(kmx_plan* p, int term, int dim, const double* mat, hipStream_t s);
 void kmx_blocks_free(kmx_plan* p);
 
+// Factored FP64 apply (kmx_factor.hip): built with the plan where the pair list is a tensor
+// product and the sizes make it worth while (idx / rp / cols 0-based).  apply: 1 launched,
+// 0 the call has to run pair by pair (stream capture), negative an error.
+void kmx_factor_build(kmx_plan* p, const std::vector<int>& idx, const std::vector<long long>& rp,
+                      const std::vector<int>& cols);
+void kmx_factor_term_updated(kmx_plan* p, int term, int dim, hipStream_t s);
+bool kmx_factor_ok(const kmx_plan* p, bool transpose);
+int kmx_factor_apply(kmx_plan* p, bool transpose, const kmx::KArgs<double>& k, hipStream_t s);
+void kmx_factor_free(kmx_plan* p);
+
 // Dimension-sweep path (kmx_sweep.hip).  slot: 0 FP64, 1 FP32, 2 BF16 (separable
 // sweeps only: BF16 values of the combined operators on the FP32 arena, BF16
 // matrix-core products with FP32 accumulation).
@@ -141,6 +154,7 @@ void kmx_sweep_build(kmx_plan* p);
 int kmx_sweep_apply(kmx_plan* p, int slot, const double* x, double* y, hipStream_t s);
 void kmx_sweep_free(kmx_plan* p);
 double kmx_sweep_flops(const kmx_plan* p);
+bool kmx_sweep_separable(const kmx_plan* p);  // has a sweep of the separable form
 // whether FP64 applies may use the plan's sweep (a separable sweep whose undeclared
 // identity factors are exact to 4 ulps, or a general sweep)
 bool kmx_sweep_fp64_ok(const kmx_plan* p);

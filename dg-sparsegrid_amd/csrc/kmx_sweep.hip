@@ -2236,6 +2236,8 @@ void kmx_sweep_free(kmx_plan* p) {
     p->sw = nullptr;
 }
 
+bool kmx_sweep_separable(const kmx_plan* p) { return p->sw && p->sw->separable; }
+
 double kmx_sweep_flops(const kmx_plan* p) { return p->sw ? double(p->sw->flops) : 0.0; }
 
 bool kmx_sweep_fp64_ok(const kmx_plan* p) { return p->sw && (!p->sw->separable || p->sw->fp64); }

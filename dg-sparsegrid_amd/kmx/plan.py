@@ -70,6 +70,7 @@ class Plan:
     level_blocks  also detect the level-block structure (KMX_PLAN_LEVEL_BLOCKS)
               and build the dimension sweep on it (set_sweep / autotune; BF16
               applies need its separable form); off, every apply runs pair by pair
+              (large FP64 ones may factor the pair sum over the dimensions)
     identity  None, or T x d booleans declaring factors the identity (MASS
               pterms with g = 1): the separable sweep takes them as exactly I
               (kmx_plan_desc.identity)

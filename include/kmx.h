@@ -50,9 +50,11 @@ extern "C" {
 #define KMX_PLAN_FP32 1u    /* also keep FP32 copies of the coefficient blocks */
 #define KMX_PLAN_ADJOINT 2u /* also keep the transposed pair list / blocks (kmx_apply_transpose) */
 #define KMX_PLAN_LEVEL_BLOCKS 4u /* also detect the level-block structure and build the
-                                    dimension sweep on it (kmx_plan_set_sweep); without it every
+                                    dimension sweep on it (kmx_plan_set_sweep); without it an
                                     apply runs pair by pair, in the reference's order of
-                                    operations (apply_A.m:100-237) */
+                                    operations (apply_A.m:100-237), or, in FP64 on a large pair
+                                    list that is a tensor product of 1D connections, with the
+                                    same sums taken one group of dimensions at a time */
 
 typedef struct kmx_plan kmx_plan;
 
@@ -101,8 +103,8 @@ int kmx_plan_set_term_scale(kmx_plan* plan, int term, double alpha);
 int kmx_plan_destroy(kmx_plan* plan);
 
 /* Time the kernel variants (workgroup size 128/256/512, LDS staging of the
- * row's coefficient strips on/off) on this plan for FP64 and FP32 and keep the
- * fastest; plans of the same (d, deg, terms, pair density) created later in
+ * row's coefficient strips on/off; FP64 with factored sums against them) on
+ * this plan for FP64 and FP32 and keep the fastest; plans of the same (d, deg, terms, pair density) created later in
  * the process start from that choice.  Synchronous on `stream`; not for use
  * under graph capture.  No counterpart in the reference (MATLAB picks nothing;
  * its flops_kron{k} method choice is the only cost model it has). */

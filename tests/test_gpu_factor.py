@@ -1,0 +1,149 @@
+"""The factored FP64 apply (kmx_factor.hip) against the CPU oracle and the pair kernels,
+at sizes below the rule that picks it (KMX_FACTOR_MIN_FMA=0), through the C ABI.
+
+Bars: 1e-13 relative (2-norm) to the oracle, the bar of every FP64 apply (sums of at most
+P T deg^d products, random operands: a few eps (P T deg^d / N)^(1/2), below 1e-14 here)."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def everywhere(monkeypatch):
+    monkeypatch.setenv("KMX_FACTOR_MIN_FMA", "0")
+
+
+def rel(a, b):
+    return float(np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-300))
+
+
+def case(nd, lev, deg, T, conn, seed, shared=False):
+    rng = np.random.default_rng(seed)
+    if conn:
+        h = O.hash_table_nd(nd, lev, "SG")
+        rp, cols = O.connect_nd(nd, lev, "SG", lev, lev)
+    else:
+        h = O.hash_table_sparse_nd([lev] * nd, max(lev, 1), "SG")
+        rp = cols = None
+    n = deg * 2 ** lev
+    mats = [[rng.standard_normal((n, n)) for _ in range(nd)] for _ in range(T)]
+    if shared:  # terms acting in one dimension each, one matrix per dimension in all the others
+        common = [rng.standard_normal((n, n)) for _ in range(nd)]
+        mats = [[m if d == t % nd else common[d] for d, m in enumerate(tm)] for t, tm in enumerate(mats)]
+    idx = np.asarray(h["idx1d"])
+    return mats, idx, rp, cols, rng.standard_normal(idx.shape[0] * deg ** nd)
+
+
+SHAPES = [
+    (2, 3, 2, 2, True), (2, 4, 3, 3, False), (2, 5, 4, 2, True), (2, 3, 5, 1, False), (2, 7, 2, 4, False),
+    (3, 3, 2, 3, True), (3, 4, 3, 3, True), (3, 2, 4, 2, False), (3, 5, 2, 2, False),
+    (4, 3, 2, 4, True), (4, 2, 2, 1, False), (5, 2, 2, 5, True), (5, 3, 2, 2, False), (6, 2, 2, 6, True),
+    (6, 1, 2, 3, False),
+]
+
+
+@pytest.mark.parametrize("nd,lev,deg,T,conn", SHAPES)
+@pytest.mark.parametrize("shared", [False, True])
+def test_matches_oracle_forward_and_adjoint(kmx_gpu, nd, lev, deg, T, conn, shared):
+    import torch
+
+    mats, idx, rp, cols, x = case(nd, lev, deg, T, conn, nd * 100 + lev * 10 + deg, shared)
+    plan = kmx_gpu.Plan(mats, idx, deg, rp, cols, index_base=1, adjoint=True)
+    scales = np.random.default_rng(1).uniform(0.5, 2.0, size=T)
+    for t, s in enumerate(scales):
+        plan.set_term_scale(t, s)
+    scaled = [[scales[t] * m if d == 0 else m for d, m in enumerate(tm)] for t, tm in enumerate(mats)]
+    xd = torch.from_numpy(x).cuda()
+    y = plan.apply(xd).cpu().numpy()
+    assert rel(y, O.apply_A(O.ApplyInputs(scaled, idx, deg, rp, cols), x, nthreads=8)) <= 1e-13
+    # the adjoint is the operator of the transposed matrices over the transposed (symmetric) pair list
+    tr = [[np.ascontiguousarray(m.T) for m in tm] for tm in scaled]
+    yt = plan.apply_transpose(xd).cpu().numpy()
+    assert rel(yt, O.apply_A(O.ApplyInputs(tr, idx, deg, rp, cols), x, nthreads=8)) <= 1e-13
+    # a new matrix (its class of equal prefixes may change), then the old one again
+    new = np.random.default_rng(2).standard_normal(mats[0][0].shape)
+    plan.update_term(0, 0, new)
+    scaled[0][0] = scales[0] * new
+    y2 = plan.apply(xd).cpu().numpy()
+    assert rel(y2, O.apply_A(O.ApplyInputs(scaled, idx, deg, rp, cols), x, nthreads=8)) <= 1e-13
+    plan.update_term(0, 0, mats[0][0])
+    assert np.array_equal(plan.apply(xd).cpu().numpy(), y)
+
+
+def test_lists_that_are_no_product_run_pair_by_pair(kmx_gpu):
+    """One pair taken out of, or repeated in, a product list; and elements given twice."""
+    import torch
+
+    mats, idx, rp, cols, x = case(2, 4, 2, 2, True, 5)
+    rp, cols = np.asarray(rp).copy(), np.asarray(cols).copy()
+    drop, dup = 7, 11
+    c1, r1 = np.delete(cols, drop), rp - (rp > drop)
+    c2, r2 = np.insert(cols, dup, cols[dup]), rp + (rp > dup)
+    for rr, cc in ((r1, c1), (r2, c2)):
+        y = kmx_gpu.Plan(mats, idx, 2, rr, cc, index_base=1).apply(torch.from_numpy(x).cuda()).cpu().numpy()
+        assert rel(y, O.apply_A(O.ApplyInputs(mats, idx, 2, rr, cc), x)) <= 1e-13
+    twice = np.vstack([idx, idx[:3]])
+    x2 = np.random.default_rng(3).standard_normal(twice.shape[0] * 4)
+    y = kmx_gpu.Plan(mats, twice, 2, None, None, index_base=1).apply(torch.from_numpy(x2).cuda()).cpu().numpy()
+    assert rel(y, O.apply_A(O.ApplyInputs(mats, twice, 2), x2)) <= 1e-13
+
+
+@pytest.mark.parametrize("nd,lev,deg,conn", [(2, 4, 3, True), (3, 3, 3, True), (6, 1, 2, True), (2, 4, 4, False)])
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+def test_non_finite_inputs_reach_connected_rows_only(kmx_gpu, monkeypatch, nd, lev, deg, conn, value):
+    """y is not finite exactly where the pair kernels' is, with the same values there, and
+    elsewhere equal to 1e-13."""
+    import torch
+
+    mats, idx, rp, cols, x = case(nd, lev, deg, 2, conn, 9)
+    x[(idx.shape[0] - 1) * deg ** nd + 1] = value  # in the last element: a high level, few connections
+    xd = torch.from_numpy(x).cuda()
+    y = kmx_gpu.Plan(mats, idx, deg, rp, cols, index_base=1).apply(xd).cpu().numpy()
+    monkeypatch.setenv("KMX_FACTOR_MIN_FMA", "1e300")
+    ref = kmx_gpu.Plan(mats, idx, deg, rp, cols, index_base=1).apply(xd).cpu().numpy()
+    fin = np.isfinite(ref)
+    assert np.array_equal(fin, np.isfinite(y)) and np.array_equal(y[~fin], ref[~fin], equal_nan=True)
+    assert not fin.all() and (not fin.any() or rel(y[fin], ref[fin]) <= 1e-13)
+
+
+def test_streams_threads_and_capture(kmx_gpu):
+    """Applies of one plan from two streams and two threads, interleaved, and under graph
+    capture, each against its own result alone (the workspace is the plan's)."""
+    import threading
+
+    import torch
+
+    mats, idx, rp, cols, _ = case(3, 4, 3, 3, True, 4)
+    plan = kmx_gpu.Plan(mats, idx, 3, rp, cols, index_base=1)
+    xs = [torch.randn(plan.dof, dtype=torch.float64, device="cuda") for _ in range(2)]
+    want = [plan.apply(x).clone() for x in xs]
+    torch.cuda.synchronize()
+    out = [[torch.empty_like(x) for _ in range(20)] for x in xs]
+
+    def work(k):
+        st = torch.cuda.Stream()
+        with torch.cuda.stream(st):
+            for y in out[k]:
+                plan.apply(xs[k], y)
+        st.synchronize()
+
+    th = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    for k in range(2):
+        assert all(torch.equal(y, want[k]) for y in out[k])
+    y = torch.empty_like(xs[0])
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        plan.apply(xs[0], y)
+    for x in (xs[1], xs[1] * 2):
+        xs[0].copy_(x)
+        ref = plan.apply(x)
+        g.replay()
+        torch.cuda.synchronize()
+        assert float((y - ref).norm() / ref.norm()) <= 1e-13
