@@ -18,17 +18,17 @@ namespace kmx {
 namespace {
 
 // Bound by the blocks it writes (B^2 values a pair).  A workgroup takes one row
-// element (or a slice of its pairs) and its threads keep fixed places: thread t
-// writes entries t, t + 256, ... of every pair's block, so the digits of (r, c) --
-// divisions -- are worked out once per entry and thread, not once per value
-// written (3D lev 5 deg 3, 372 MB: 1.93 ms with the divisions per value, 0.132 ms
-// so: 2.8 TB/s).  For each entry it walks the pairs of its slice, a wave writing
-// 512 contiguous bytes per pair (non-temporal stores: 0.150 ms).  The block offsets
-// of 128 pairs at a time and, up to 64 KB, the row's coefficient strips (every block
-// (I_k, .) of every term) are staged in LDS; block J of a strip starts at J deg^2 and
-// the entry's place inside a block is fixed, so a value costs d T LDS reads, the
-// products and one store.  Small blocks (B^2 < 256) share the workgroup: G =
-// 256 / B^2 pairs at a time.
+// element (or a slice of its pairs) and its threads keep fixed places inside every
+// pair's block, so the digits of (r, c) -- divisions -- are worked out once per thread,
+// not once per value written.  The block offsets of 128 pairs at a time and, up to
+// 64 KB, the row's coefficient strips (every block (I_k, .) of every term) are staged
+// in LDS; block J of a strip starts at J deg^2 and an entry's place inside a block is
+// fixed.  With one entry a thread a value cost d T LDS reads, as many as the stores
+// take: a thread's entries now share all but the column digits of dimensions 1 and 2
+// (deg^2 of them, B^2 / deg^2 values apart: lanes still store runs), 2 deg + d - 2
+// reads a term for deg^2 values.  3D lev 5 deg 3, 372 MB: 1.93 ms with the divisions
+// per value, 0.132 with one entry a thread, 0.090 now, 4.1 TB/s (a fill of the same
+// size: 6.2); 3D lev 4 deg 4 0.182 -> 0.087.  Small pairs share the workgroup.
 constexpr int AS_THREADS = 256;
 constexpr int AS_PAIRS = 128;
 
@@ -38,7 +38,9 @@ struct AsmArgs {
     int B, slices, strip_off[KMX_MAX_DIM], strip_term;  // LDS offsets of (term 0, dim k); doubles per term
 };
 
-template <int D, bool LDS>
+// A thread's C1 x C2 entries: all column digits of dimension 1 (C1 = deg) and of
+// dimension 2 (C2 = deg), or one
+template <int D, int C1, int C2, bool LDS>
 __global__ void __launch_bounds__(AS_THREADS) k_assemble(AsmArgs g, int deg) {
     extern __shared__ __align__(16) double strip[];
     __shared__ int place[AS_PAIRS][D];
@@ -64,8 +66,11 @@ __global__ void __launch_bounds__(AS_THREADS) k_assemble(AsmArgs g, int deg) {
         __syncthreads();
     }
     const long long BB = (long long)g.B * g.B;
-    const int G = BB < AS_THREADS ? AS_THREADS / int(BB) : 1;  // pairs at a time
-    const int lane_q = BB < AS_THREADS ? tid / int(BB) : 0;
+    constexpr int E = C1 * C2;
+    const int s2 = g.B / (C2 == 1 ? 1 : C1 * C2);  // columns from one digit of dimension 2 to the next
+    const long long BE = BB / E;  // threads of a pair
+    const int G = BE < AS_THREADS ? AS_THREADS / int(BE) : 1;  // pairs at a time
+    const int lane_q = BE < AS_THREADS ? tid / int(BE) : 0;
     for (int qc = qa; qc < qb; qc += AS_PAIRS) {  // the block offsets of the next pairs, in LDS
         const int nc = min(AS_PAIRS, qb - qc);
         if (qc > qa) __syncthreads();
@@ -76,7 +81,7 @@ __global__ void __launch_bounds__(AS_THREADS) k_assemble(AsmArgs g, int deg) {
         }
         __syncthreads();
         if (lane_q >= G) continue;
-        for (long long ent = tid - lane_q * BB; ent < BB; ent += AS_THREADS) {
+        for (long long ent = tid - lane_q * BE; ent < BE; ent += AS_THREADS) {
             const int c = int(ent / g.B), r = int(ent - (long long)c * g.B);  // column-major inside the block
             int in[D];  // the entry's place inside block (I_k, J_k)
             int rr = r, cc = c;
@@ -93,38 +98,67 @@ __global__ void __launch_bounds__(AS_THREADS) k_assemble(AsmArgs g, int deg) {
                 int at[D];
 #pragma unroll
                 for (int k = 0; k < D; ++k) at[k] = place[q][k] + in[k];
-                double s = 0.0;
-                for (int t = 0; t < T; ++t) {
-                    double p = 1.0;
+                double s[E];
 #pragma unroll
-                    for (int k = 0; k < D; ++k) {
-                        const double v = LDS ? strip[t * g.strip_term + at[k]]
-                                             : a.blk[a.off[t * D + k] + (long long)ie[k] * a.nb[k] * dd + at[k]];
-                        p = k == 0 ? v : __dmul_rn(p, v);
+                for (int x = 0; x < E; ++x) s[x] = 0.0;
+                for (int t = 0; t < T; ++t) {
+                    auto factor = [&](int k, int x) {
+                        return LDS ? strip[t * g.strip_term + at[k] + x]
+                                   : a.blk[a.off[t * D + k] + (long long)ie[k] * a.nb[k] * dd + at[k] + x];
+                    };
+                    double v[D], w[C2];
+#pragma unroll
+                    for (int k = 1; k < D; ++k)
+                        if (k > 1 || C2 == 1) v[k] = factor(k, 0);
+                    if constexpr (C2 > 1)
+#pragma unroll
+                        for (int y = 0; y < C2; ++y) w[y] = factor(1, y);
+#pragma unroll
+                    for (int x = 0; x < C1; ++x) {
+                        const double u = factor(0, x);
+#pragma unroll
+                        for (int y = 0; y < C2; ++y) {
+                            double p = u;
+#pragma unroll
+                            for (int k = 1; k < D; ++k) p = __dmul_rn(p, k == 1 && C2 > 1 ? w[y] : v[k]);
+                            s[x * C2 + y] = __dadd_rn(s[x * C2 + y], a.scale[t] == 1.0 ? p : __dmul_rn(a.scale[t], p));
+                        }
                     }
-                    s = __dadd_rn(s, a.scale[t] == 1.0 ? p : __dmul_rn(a.scale[t], p));
                 }
-                out[q * BB] = s;
+#pragma unroll
+                for (int x = 0; x < C1; ++x)
+#pragma unroll
+                    for (int y = 0; y < C2; ++y)
+                        out[q * BB + (long long)(x * (g.B / C1) + y * s2) * g.B] = s[x * C2 + y];
             }
-            if (BB < AS_THREADS) break;  // one entry per thread
+            if (BE < AS_THREADS) break;  // one entry per thread
         }
     }
 }
 
+template <int D, int C1, int C2, bool LDS>
+hipError_t launch_as(const AsmArgs& g, int deg, size_t lds, unsigned grid, hipStream_t s) {
+    hipLaunchKernelGGL((k_assemble<D, C1, C2, LDS>), dim3(grid), dim3(AS_THREADS), lds, s, g, deg);
+    return hipGetLastError();
+}
+
 template <int D>
 hipError_t launch(const AsmArgs& g, int deg, size_t lds, unsigned grid, hipStream_t s) {
-    if (lds > 0) {
-        auto kern = k_assemble<D, true>;
-        if (lds > 65536) {
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
-            if (e != hipSuccess) return e;
-        }
-        hipLaunchKernelGGL(kern, dim3(grid), dim3(AS_THREADS), lds, s, g, deg);
-    } else {
-        hipLaunchKernelGGL((k_assemble<D, false>), dim3(grid), dim3(AS_THREADS), 0, s, g, deg);
+    if (lds == 0) return launch_as<D, 1, 1, false>(g, deg, lds, grid, s);
+    // both digits while a pair's threads fill a wave: shorter runs store in pieces
+    const bool two = D > 1 && (long long)g.B * g.B >= 64ll * deg * deg;
+    switch (deg) {
+        case 2:
+            return two ? launch_as<D, 2, D == 1 ? 1 : 2, true>(g, deg, lds, grid, s)
+                       : launch_as<D, 2, 1, true>(g, deg, lds, grid, s);
+        case 3:
+            return two ? launch_as<D, 3, D == 1 ? 1 : 3, true>(g, deg, lds, grid, s)
+                       : launch_as<D, 3, 1, true>(g, deg, lds, grid, s);
+        case 4:
+            return two ? launch_as<D, 4, D == 1 ? 1 : 4, true>(g, deg, lds, grid, s)
+                       : launch_as<D, 4, 1, true>(g, deg, lds, grid, s);
+        default: return launch_as<D, 1, 1, true>(g, deg, lds, grid, s);
     }
-    return hipGetLastError();
 }
 
 }  // namespace
@@ -158,11 +192,20 @@ extern "C" int kmx_plan_assemble(kmx_plan* p, double* blocks, void* stream) {
     a.nterms = p->T;
     g.out = blocks;
     g.B = p->B;
-    // at least ~2048 workgroups (a few per CU), each with pairs enough to pay for its strips
-    const long long per_row = p->P / p->N + 1;
-    g.slices = int(std::max(1LL, std::min<long long>((2048 + p->N - 1) / p->N, per_row / 16)));
     const size_t strips = size_t(st) * p->T * sizeof(double);
     const size_t lds = strips <= 64 * 1024 ? strips : 0;
+    // Workgroups: about 2048, each of 16 pairs at least to pay for its strips.  Blocks of 256
+    // values and more: two rounds of what the CUs hold (3D lev 5 deg 3, 3.5 thousand: 99 -> 90
+    // us; 3D lev 4 deg 4, whose 37 KB of strips leave four a CU: 85 us with 2 thousand, 96 with
+    // 4), of as few pairs as write twice the strips' values (6D lev 2 deg 2, 28 rows of 28
+    // pairs: 133 -> 38 us).
+    const long long per_row = p->P / p->N + 1, BB = (long long)p->B * p->B;
+    long long want = 2048, least = 16;
+    if (BB >= AS_THREADS) {
+        want = 512 * std::min<long long>(8, 160 * 1024 / (long long)(lds + sizeof(int) * AS_PAIRS * p->D));
+        least = std::min(16LL, 1 + 2LL * st * p->T / BB);
+    }
+    g.slices = int(std::max(1LL, std::min<long long>((want + p->N - 1) / p->N, per_row / least)));
     const unsigned grid = unsigned(p->N) * unsigned(g.slices);
     const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     hipError_t e = hipErrorInvalidValue;

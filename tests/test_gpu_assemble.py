@@ -99,3 +99,16 @@ def test_assembled_blocks_edges(kmx_gpu, nd, lev, deg, T, conn):
     plan = kmx_gpu.Plan(mats, idx, deg, rp, cols)
     A = dense_from_blocks(plan.assemble().cpu().numpy(), plan.N, plan.B, rp, cols)
     assert np.array_equal(A, O.build_A(O.ApplyInputs(mats, idx, deg, rp, cols)))
+
+
+@pytest.mark.parametrize("nd,lev,deg,T,conn", [(1, 3, 2, 2, False), (1, 3, 3, 1, True), (2, 2, 2, 1, False),
+                                               (3, 2, 2, 2, False), (3, 2, 4, 2, True), (4, 1, 3, 2, False),
+                                               (4, 1, 4, 1, False), (5, 1, 3, 2, False), (6, 2, 2, 2, True),
+                                               (3, 1, 5, 2, False), (2, 4, 4, 8, True)])
+def test_assembled_blocks_by_entries_per_thread(kmx_gpu, nd, lev, deg, T, conn):
+    """A thread with one, deg or deg^2 entries (pairs of fewer threads than a wave, than a
+    workgroup and more), rows cut into slices of a few pairs: bit-exact."""
+    mats, idx, rp, cols = make_case(nd, lev, deg, T, conn, seed=70 + nd + deg)
+    plan = kmx_gpu.Plan(mats, idx, deg, rp, cols)
+    A = dense_from_blocks(plan.assemble().cpu().numpy(), plan.N, plan.B, rp, cols)
+    assert np.array_equal(A, O.build_A(O.ApplyInputs(mats, idx, deg, rp, cols)))
