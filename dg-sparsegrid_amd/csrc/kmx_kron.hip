@@ -19,7 +19,8 @@ namespace kmx {
 struct ModeArgs {
     const double* in;
     double* out;
-    const double* A;  // nrow x ncol, column-major
+    const double* A;  // nrow x ncol
+    int sr, sc;       // its strides along rows and columns
     long long inner;  // product of extents of dims faster than `dim`
     long long outer;  // product of extents of dims slower than `dim` times nvec
     int nrow, ncol;
@@ -34,7 +35,7 @@ __global__ void __launch_bounds__(256) k_mode_product(ModeArgs m) {
         const long long o = r / m.nrow;
         const double* in = m.in + o * m.ncol * m.inner + s;
         double acc = 0.0;
-        for (int b = 0; b < m.ncol; ++b) acc = __builtin_fma(m.A[(long long)b * m.nrow + a], in[b * m.inner], acc);
+        for (int b = 0; b < m.ncol; ++b) acc = __builtin_fma(m.A[(long long)b * m.sc + (long long)a * m.sr], in[b * m.inner], acc);
         m.out[e] = acc;
     }
 }
@@ -53,7 +54,7 @@ __global__ void __launch_bounds__(256) k_mode_product(ModeArgs m) {
 // Four 8 x 8 factors on 128 vectors: 4 launches, 32 us of kernel time, now 1 of 16 us.
 constexpr int KG_THREADS = 512;
 constexpr int KG_TILE = 8448;   // values of a tile at most: 2 buffers x 9/8 x 8 bytes = 152 KB of the 160 KB
-constexpr int KG_FACTOR = 1000;  // values of the factors kept in LDS
+constexpr int KG_FACTOR = KMX_KRON_ROWMAJOR_VALUES;  // values of the factors kept in LDS
 constexpr int KG_MIN_IC = 8;    // contiguous values per access at least when the modes are strided
 struct GroupArgs {
     const double* in;
@@ -65,6 +66,7 @@ struct GroupArgs {
     int k, OC, IC, buf;  // buf: doubles of one LDS buffer
     int chunks;          // workgroups along inner
     int foff[KMX_KRON_MAX_FACTORS], nfac;  // the factors' places in LDS, their values (0: not kept there)
+    unsigned rowmajor;                     // bit d: factor d is row-major (staged factors only)
 };
 __device__ __forceinline__ int kg_at(int i) { return i + (i >> 3); }
 typedef const __attribute__((address_space(4))) double* kg_factor;  // read through the scalar cache
@@ -156,7 +158,11 @@ __global__ void __launch_bounds__(KG_THREADS) k_mode_group(GroupArgs g) {
     if (staged)
         for (int d = 0; d < g.k; ++d) {
             const gptr A = (gptr)g.A[d];
-            for (int i = threadIdx.x; i < g.nrow[d] * g.ncol[d]; i += nt) fac[g.foff[d] + i] = A[i];
+            const int nr = g.nrow[d], nc = g.ncol[d];
+            if (g.rowmajor >> d & 1)
+                for (int i = threadIdx.x; i < nr * nc; i += nt) fac[g.foff[d] + i] = A[i % nr * nc + i / nr];
+            else
+                for (int i = threadIdx.x; i < nr * nc; i += nt) fac[g.foff[d] + i] = A[i];
         }
     __syncthreads();
     int fast = g.IC;  // extent of the faster indices inside the tile
@@ -444,10 +450,11 @@ std::vector<ChainStep> plan_chain(int k, const int* nrow, const int* ncol, int n
 // The mode products of kron(A1..Ak) X, last factor first (method 1), through the
 // ping-pong buffers buf[0] / buf[1] (used only when the steps need them).  For k > 6
 // this is also the order of kron_multd.m's recursion (kron_multd.m:64-86: Z = A_k X,
-// then kron(A_1..A_{k-1}) on Z's transpose).
+// then kron(A_1..A_{k-1}) on Z's transpose).  rowmajor: null, or per factor whether it is
+// stored by rows (the factors have KG_FACTOR values at most then: groups keep them in LDS).
 hipError_t launch_chain(const std::vector<ChainStep>& steps, int k, const int* nrow, const int* ncol,
-                        const double* const* A, const double* X, int nvec, double* Y, double* const* buf,
-                        hipStream_t s) {
+                        const double* const* A, const unsigned char* rowmajor, const double* X, int nvec, double* Y,
+                        double* const* buf, hipStream_t s) {
     std::vector<long long> ext(ncol, ncol + k);
     const double* cur = X;
     int ping = 0;
@@ -463,6 +470,9 @@ hipError_t launch_chain(const std::vector<ChainStep>& steps, int k, const int* n
             m.A = A[st.first];
             m.nrow = nrow[st.first];
             m.ncol = ncol[st.first];
+            const bool rm = rowmajor && rowmajor[st.first];
+            m.sr = rm ? m.ncol : 1;
+            m.sc = rm ? 1 : m.nrow;
             m.inner = inner;
             m.outer = outer;
             const long long total = m.inner * m.nrow * m.outer;
@@ -473,8 +483,10 @@ hipError_t launch_chain(const std::vector<ChainStep>& steps, int k, const int* n
             g.in = cur;
             g.out = out;
             g.k = st.last - st.first + 1;
+            g.rowmajor = 0;
             long long cols = 1, rows = 1;
             for (int i = 0; i < g.k; ++i) {
+                g.rowmajor |= rowmajor && rowmajor[st.first + i] ? 1u << i : 0u;
                 g.A[i] = A[st.first + i];
                 g.nrow[i] = nrow[st.first + i];
                 g.ncol[i] = ncol[st.first + i];
@@ -535,12 +547,10 @@ bool kron_args_ok(int k, const int* nrow, const int* ncol, const double* const* 
     return true;
 }
 
-}  // namespace
-
-extern "C" int kmx_kronmult(int k, const int* nrow, const int* ncol, const double* const* A, const double* X,
-                            int nvec, double* Y, void* stream) {
+int kronmult(const char* who, int k, const int* nrow, const int* ncol, const double* const* A,
+             const unsigned char* rowmajor, const double* X, int nvec, double* Y, void* stream) {
     if (!kron_args_ok(k, nrow, ncol, A, X, nvec, Y)) {
-        set_error("kmx_kronmult: bad arguments");
+        set_error(std::string(who) + ": bad arguments");
         return KMX_E_ARG;
     }
     if (nvec == 0) return KMX_OK;
@@ -552,21 +562,28 @@ extern "C" int kmx_kronmult(int k, const int* nrow, const int* ncol, const doubl
         if (hipMalloc(&buf[0], sizeof(double) * maxsz) != hipSuccess ||
             (steps.size() > 2 && hipMalloc(&buf[1], sizeof(double) * maxsz) != hipSuccess)) {
             hipFree(buf[0]);
-            set_error("kmx_kronmult: workspace allocation failed");
+            set_error(std::string(who) + ": workspace allocation failed");
             return KMX_E_NOMEM;
         }
     }
-    const hipError_t e = launch_chain(steps, k, nrow, ncol, A, X, nvec, Y, buf, s);
+    const hipError_t e = launch_chain(steps, k, nrow, ncol, A, rowmajor, X, nvec, Y, buf, s);
     if (buf[0]) {
         hipStreamSynchronize(s);
         hipFree(buf[0]);
         if (buf[1]) hipFree(buf[1]);
     }
     if (e != hipSuccess) {
-        set_error(std::string("kmx_kronmult: ") + hipGetErrorString(e));
+        set_error(std::string(who) + ": " + hipGetErrorString(e));
         return KMX_E_HIP;
     }
     return KMX_OK;
+}
+
+}  // namespace
+
+extern "C" int kmx_kronmult(int k, const int* nrow, const int* ncol, const double* const* A, const double* X,
+                            int nvec, double* Y, void* stream) {
+    return kronmult("kmx_kronmult", k, nrow, ncol, A, nullptr, X, nvec, Y, stream);
 }
 
 // ---- kmx_kronmult without allocation: the chain's two intermediates live in one
@@ -593,10 +610,11 @@ double* scratch_for_current_device() {
 }
 }  // namespace
 
-extern "C" int kmx_kronmult_noalloc(int k, const int* nrow, const int* ncol, const double* const* A,
-                                    const double* X, int nvec, double* Y, void* stream) {
+namespace {
+int kronmult_noalloc(const char* who, int k, const int* nrow, const int* ncol, const double* const* A,
+                     const unsigned char* rowmajor, const double* X, int nvec, double* Y, void* stream) {
     if (!kron_args_ok(k, nrow, ncol, A, X, nvec, Y)) {
-        set_error("kmx_kronmult_noalloc: bad arguments");
+        set_error(std::string(who) + ": bad arguments");
         return KMX_E_ARG;
     }
     if (nvec == 0) return KMX_OK;
@@ -605,25 +623,50 @@ extern "C" int kmx_kronmult_noalloc(int k, const int* nrow, const int* ncol, con
     if (k > 1 && maxsz > half) {
         char msg[200];
         std::snprintf(msg, sizeof msg,
-                      "kmx_kronmult_noalloc: an intermediate of %lld values exceeds the scratch limit of %lld "
+                      "%s: an intermediate of %lld values exceeds the scratch limit of %lld "
                       "(KMX_KRON_SCRATCH_ELEMS / 2); use kmx_kronmult",
-                      maxsz, half);
+                      who, maxsz, half);
         set_error(msg);
         return KMX_E_SHAPE;
     }
     double* base = scratch_for_current_device();
     if (!base) {
-        set_error("kmx_kronmult_noalloc: hipGetSymbolAddress of the scratch array failed");
+        set_error(std::string(who) + ": hipGetSymbolAddress of the scratch array failed");
         return KMX_E_HIP;
     }
     double* buf[2] = {base, base + half};
-    const hipError_t e = launch_chain(plan_chain(k, nrow, ncol, nvec, X, Y), k, nrow, ncol, A, X, nvec, Y, buf,
+    const hipError_t e = launch_chain(plan_chain(k, nrow, ncol, nvec, X, Y), k, nrow, ncol, A, rowmajor, X, nvec, Y, buf,
                                       reinterpret_cast<hipStream_t>(stream));
     if (e != hipSuccess) {
-        set_error(std::string("kmx_kronmult_noalloc: ") + hipGetErrorString(e));
+        set_error(std::string(who) + ": " + hipGetErrorString(e));
         return KMX_E_HIP;
     }
     return KMX_OK;
+}
+}  // namespace
+
+extern "C" int kmx_kronmult_noalloc(int k, const int* nrow, const int* ncol, const double* const* A,
+                                    const double* X, int nvec, double* Y, void* stream) {
+    return kronmult_noalloc("kmx_kronmult_noalloc", k, nrow, ncol, A, nullptr, X, nvec, Y, stream);
+}
+
+extern "C" int kmx_kronmult_layout(int k, const int* nrow, const int* ncol, const double* const* A,
+                                   const unsigned char* rowmajor, const double* X, int nvec, double* Y, int noalloc,
+                                   void* stream) {
+    if (rowmajor && kron_args_ok(k, nrow, ncol, A, X, nvec, Y)) {
+        long long values = 0;
+        bool any = false;
+        for (int i = 0; i < k; ++i) {
+            any = any || rowmajor[i];
+            values += (long long)nrow[i] * ncol[i];
+        }
+        if (any && values > KG_FACTOR) {
+            set_error("kmx_kronmult_layout: row-major factors of more than KMX_KRON_ROWMAJOR_VALUES values together");
+            return KMX_E_SHAPE;
+        }
+    }
+    return noalloc ? kronmult_noalloc("kmx_kronmult_layout", k, nrow, ncol, A, rowmajor, X, nvec, Y, stream)
+                   : kronmult("kmx_kronmult_layout", k, nrow, ncol, A, rowmajor, X, nvec, Y, stream);
 }
 
 extern "C" int kmx_gemm_vbatched(char transA, char transB, const int* m, const int* n, const int* k, double alpha,

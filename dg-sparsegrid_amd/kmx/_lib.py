@@ -21,6 +21,7 @@ PREC_FP32 = 1
 PREC_BF16 = 3
 
 KRON_SCRATCH_ELEMS = 1 << 20
+KRON_ROWMAJOR_VALUES = 1000  # KMX_KRON_ROWMAJOR_VALUES
 ARNOLDI_MAX_K = 127
 
 
@@ -158,6 +159,8 @@ PROTOTYPES = {
                                    C.c_void_p, C.c_void_p, C.c_void_p]),
     "kmx_kronmult_noalloc": (C.c_int, [C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_void_p),
                                        C.c_void_p, C.c_int, C.c_void_p, C.c_void_p]),
+    "kmx_kronmult_layout": (C.c_int, [C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_void_p),
+                                      C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_void_p]),
     "kmx_gemm_vbatched": (C.c_int, [C.c_char, C.c_char, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_int),
                                     C.c_double, C.POINTER(C.c_void_p), C.POINTER(C.c_int), C.POINTER(C.c_void_p),
                                     C.POINTER(C.c_int), C.c_double, C.POINTER(C.c_void_p), C.POINTER(C.c_int), C.c_int,

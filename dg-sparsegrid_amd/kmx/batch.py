@@ -16,7 +16,7 @@ import numpy as np
 
 from . import coeffs as C
 from . import grid as G
-from .plan import Batch, Plan
+from .plan import Batch, Plan, _ptr
 from .timestep import A21, A31, A32, B1, B2, B3
 
 _MATS = {}
@@ -85,6 +85,7 @@ class BatchedSystem:
         sizes = [p.dof for p in self.plans]
         self.offsets = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int64)
         self.dof = int(self.offsets[-1])
+        self._bytes = [8 * int(o) for o in self.offsets[:-1]]
         self.f = torch.from_numpy(np.concatenate([inst["f0"] for inst in instances])).to(device)
         self.dt = torch.from_numpy(np.concatenate([np.full(p.dof, inst["dt"]) for p, inst in
                                                    zip(self.plans, instances)])).to(device)
@@ -101,15 +102,23 @@ class BatchedSystem:
     def views(self, v):
         return [v[self.offsets[i]:self.offsets[i + 1]] for i in range(len(self.plans))]
 
+    def _addresses(self, v):
+        """The instances' device addresses in v (a contiguous vector of every instance's
+        values), or views of it."""
+        if v.dim() != 1 or v.numel() < self.dof or not v.is_contiguous():
+            return self.views(v)
+        at = _ptr(v)
+        return [at + o for o in self._bytes]
+
     def apply(self, x, y, prec="fp32"):
-        self.batch.apply(self.views(x), self.views(y), prec=prec)
+        self.batch.apply(self._addresses(x), self._addresses(y), prec=prec)
         return y
 
     def rk3(self, nsteps=1, prec="fp32", f=None):
         """nsteps fused RK3 steps of every instance (kmx_batch_rk3) on the
         concatenated state f (default: the system's own), in place."""
         f = self.f if f is None else f
-        self.batch.rk3(self.views(f), [inst["dt"] for inst in self.instances], nsteps, prec=prec)
+        self.batch.rk3(self._addresses(f), [inst["dt"] for inst in self.instances], nsteps, prec=prec)
         return f
 
 

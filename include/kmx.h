@@ -279,6 +279,15 @@ int kmx_kronmult(int k, const int* nrow, const int* ncol, const double* const* A
 int kmx_kronmult_noalloc(int k, const int* nrow, const int* ncol, const double* const* A, const double* X, int nvec,
                          double* Y, void* stream);
 
+/* kmx_kronmult (noalloc = 0) or kmx_kronmult_noalloc (noalloc != 0) with factors stored
+ * by columns or by rows: rowmajor[i] != 0 says that A[i] is row-major (null: none is), so
+ * that row-major callers need no transposed copies.  The same results.  With a row-major
+ * factor, all factors together may have KMX_KRON_ROWMAJOR_VALUES values (else KMX_E_SHAPE). */
+#define KMX_KRON_ROWMAJOR_VALUES 1000
+int kmx_kronmult_layout(int k, const int* nrow, const int* ncol, const double* const* A,
+                        const unsigned char* rowmajor, const double* X, int nvec, double* Y, int noalloc,
+                        void* stream);
+
 /* Variable-size batched GEMM (Kronmult/gemm_vbatched.m:1-38, magmablas-style):
  * C_i = alpha*op(A_i)*op(B_i) + beta*C_i with op from transA/transB ('N'/'T'),
  * m_i x k_i times k_i x n_i.  k is taken from k[] (the reference reads nlist at

@@ -1,0 +1,86 @@
+"""Kronecker chains and batched GEMMs on arguments as callers hold them: row-major
+factors (kmx_kronmult_layout), lists of tensors, addresses, numpy sizes."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+
+def test_rowmajor_factors_beyond_the_limit_are_refused():
+    from kmx import _lib as L
+
+    lib = L.lib()
+    n = (C.c_int * 2)(25, 25)
+    one = (C.c_void_p * 2)(8, 8)  # never read: 1250 values are refused before any launch
+    args = (2, n, n, one)
+    assert lib.kmx_kronmult_layout(*args, bytes([0, 1]), 8, 1, 8, 0, None) == L.KMX_E_SHAPE
+    assert lib.kmx_kronmult_layout(*args, bytes([0, 1]), 8, 1, 8, 1, None) == L.KMX_E_SHAPE
+    assert lib.kmx_kronmult_layout(*args, bytes([1, 1]), 8, 0, None, 0, None) == L.KMX_E_ARG
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("noalloc", [False, True])
+@pytest.mark.parametrize("shapes,nvec", [([(3, 5)], 1), ([(1, 4), (6, 1), (2, 3)], 7), ([(8, 8)] * 4, 9),
+                                         ([(16, 16)] * 3, 5), ([(31, 2), (7, 31), (4, 9)], 33), ([(25, 40)], 3),
+                                         ([(25, 40), (2, 3)], 3), ([(500, 1), (1, 400)], 2), ([(2, 2)] * 12, 1)])
+def test_factor_layouts_give_the_same_bits(kmx_gpu, shapes, nvec, noalloc):
+    """Factors by rows, by columns, as strided views, alone and mixed, up to and beyond the
+    values taken by rows: the bits of column-major factors (given Y: copies are made)."""
+    import torch
+
+    gen = torch.Generator().manual_seed(len(shapes) * 100 + nvec)
+    base = [torch.randn(r, c, dtype=torch.float64, generator=gen).cuda() for r, c in shapes]
+    ncol, nrow = int(np.prod([c for _, c in shapes])), int(np.prod([r for r, _ in shapes]))
+    X = torch.randn(ncol, nvec, dtype=torch.float64, generator=gen).cuda()
+    col = [m.t().contiguous().t() for m in base]
+    wide = [torch.stack([m, m], dim=2)[:, :, 0] for m in base]
+    Y = torch.empty(nrow * nvec, dtype=torch.float64, device="cuda")
+    ref = kmx_gpu.kronmult(col, X, noalloc=noalloc, Y=Y).clone()
+    mixed = [(base, col, wide)[i % 3][i] for i in range(len(base))]
+    for mats in (base, col, wide, mixed):
+        assert torch.equal(kmx_gpu.kronmult(mats, X, noalloc=noalloc), ref)
+    want = X.cpu().numpy()
+    K = np.ones((1, 1))
+    if nrow * ncol <= 1 << 22:
+        for m in base:
+            K = np.kron(K, m.cpu().numpy())
+        # a sum of ncol products of k + 1 factors
+        bound = 8 * (ncol + len(shapes)) * np.finfo(float).eps * (np.abs(K) @ np.abs(want))
+        assert np.all(np.abs(ref.cpu().numpy() - K @ want) <= bound)
+    with pytest.raises((RuntimeError, ValueError, IndexError)):
+        kmx_gpu.kronmult([base[0][None]] + base[1:], X)
+
+
+@pytest.mark.gpu
+def test_gemm_arguments_as_tensors_addresses_and_iterators(kmx_gpu):
+    import torch
+
+    gen = torch.Generator().manual_seed(4)
+    n = [5, 17, 64]
+    A = [torch.randn(i * i, dtype=torch.float64, generator=gen).cuda() for i in n]
+    outs = []
+    for kind in range(4):
+        Cm = [torch.zeros(i * i, dtype=torch.float64, device="cuda") for i in n]
+        size = [n, tuple(n), np.asarray(n), [np.int64(i) for i in n]][kind]
+        a = [A, [t.data_ptr() for t in A], (t for t in A), [A[0].data_ptr(), A[1], A[2]]][kind]
+        kmx_gpu.gemm_vbatched("N", "T", size, size, size, 1.0, a, size, A, size, 0.0, Cm, size)
+        outs.append(torch.cat(Cm))
+    assert all(torch.equal(o, outs[0]) for o in outs[1:])
+    want = torch.cat([(t.view(i, i).t() @ t.view(i, i)).t().reshape(-1) for t, i in zip(A, n)])
+    assert torch.allclose(outs[0], want, rtol=0, atol=1e-12)
+
+
+@pytest.mark.gpu
+def test_batch_state_layouts(kmx_gpu):
+    """A longer vector, and one that is not one contiguous vector, as states of a batch."""
+    import torch
+    from kmx import batch as BT
+
+    s = BT.BatchedSystem(BT.make_instances(count=2, seed=3, lev2d=(4, 5), lev3d=(4, 4)), sweep=("fp64",))
+    ref = s.apply(s.f, torch.empty_like(s.f), "fp64").clone()
+    long = torch.cat([s.f, s.f])
+    y = torch.zeros_like(long)
+    s.apply(long, y, "fp64")
+    assert torch.equal(y[:s.dof], ref) and not y[s.dof:].any()
+    with pytest.raises(ValueError):
+        s.apply(long[::2], y, "fp64")
