@@ -202,13 +202,23 @@ constexpr int GV_MAX_CHUNKED = 8 * GV_CHUNK;
 struct GemmChunk {
     GemmDescDev d[GV_CHUNK];
 };
+// The same in 18 bytes each: sizes below 2^16, leading dimensions the rows stored, matrices
+// within 32 GB.  200 ragged products of 33..256 are one launch instead of three, each of
+// which ended with 2.3 workgroups a CU: 82 -> 59 us a call; 100 of them 56 -> 38, 90 of
+// 200..400 160 -> 140.  Up to GV_CHUNK products one launch does anyway.
+constexpr int GV_PACK = 216;
+struct GemmPack {
+    const double* base;
+    unsigned off[3][GV_PACK];  // of A, B, C from base, in doubles
+    unsigned short mnk[3][GV_PACK];
+};
 
 // The batch's GEMMs in 64 x 64 tiles of C: workgroup (g, t) takes tiles t, t +
 // gridDim.y, ... of GEMM g (row-tile fastest), on the FP64 matrix cores
 // (kmx_mma64.h).  Every entry sums its k products in order with FMAs, then C = alpha
 // sum + beta C (C not read when beta = 0), as the reference's gemm does entry by
-// entry.  FP64: 200 ragged products of 33..256 in 84 us of kernel time (121 us with VALU
-// FMAs; a workgroup's time is its k), 2048^3 at 51 TFLOP/s (22), 80 x 256^3 at 37 (23).
+// entry.  FP64: 200 ragged products of 33..256 in 58 us of kernel time (121 us with VALU
+// FMAs, 84 in three launches), 2048^3 at 51 TFLOP/s (22), 80 x 256^3 at 37 (23).
 constexpr int GV_T = 64;
 template <bool TA, bool TB>
 __device__ __forceinline__ void gemm_tiles(const GemmDescDev& d, double alpha, double beta, double* lds) {
@@ -235,6 +245,14 @@ template <bool TA, bool TB>
 __global__ void __launch_bounds__(256, 2) k_gemm_chunk(GemmChunk c, double alpha, double beta) {
     __shared__ double lds[mma64_lds<64, 16>()];
     gemm_tiles<TA, TB>(c.d[blockIdx.x], alpha, beta, lds);
+}
+template <bool TA, bool TB>
+__global__ void __launch_bounds__(256, 2) k_gemm_pack(GemmPack c, double alpha, double beta) {
+    __shared__ double lds[mma64_lds<64, 16>()];
+    const int g = blockIdx.x, m = c.mnk[0][g], n = c.mnk[1][g], k = c.mnk[2][g];
+    const GemmDescDev d{c.base + c.off[0][g], c.base + c.off[1][g], const_cast<double*>(c.base) + c.off[2][g],
+                        m, n, k, max(1, TA ? k : m), max(1, TB ? n : k), max(1, m)};
+    gemm_tiles<TA, TB>(d, alpha, beta, lds);
 }
 template <bool TA, bool TB>
 __global__ void __launch_bounds__(256, 2) k_gemm_vbatched(const GemmDescDev* __restrict__ d, double alpha, double beta) {
@@ -707,13 +725,42 @@ extern "C" int kmx_gemm_vbatched(char transA, char transB, const int* m, const i
     };
     const bool ta = tr(transA), tb = tr(transB);
     if (count <= GV_MAX_CHUNKED) {
-        // Descriptors as kernel arguments, GV_CHUNK a launch: no table to allocate, copy,
+        // Descriptors as kernel arguments, GV_PACK or GV_CHUNK a launch: no table to allocate, copy,
         // wait for and free (some 40 us a call whatever its size).  Longest k first: a
         // workgroup's time goes with k, so a launch holds workgroups of about one length.
         std::stable_sort(h.begin(), h.end(), [](const GemmDescDev& u, const GemmDescDev& v) { return u.k > v.k; });
-        const int launches = (count + GV_CHUNK - 1) / GV_CHUNK;
+        const double* lo = h[0].A;
+        for (const GemmDescDev& d : h) lo = std::min({lo, d.A, d.B, static_cast<const double*>(d.C)});
+        auto offset = [&](const double* q) {
+            return (unsigned long long)(reinterpret_cast<uintptr_t>(q) - reinterpret_cast<uintptr_t>(lo));
+        };
+        auto packs = [&](const GemmDescDev& d) {
+            for (const double* q : {d.A, d.B, static_cast<const double*>(d.C)})
+                if (offset(q) >> 35 || offset(q) % 8) return false;
+            return std::max({d.m, d.n, d.k}) < 65536 && d.lda == std::max(1, ta ? d.k : d.m) &&
+                   d.ldb == std::max(1, tb ? d.n : d.k) && d.ldc == std::max(1, d.m);
+        };
+        const bool pack = count > GV_CHUNK && std::all_of(h.begin(), h.end(), packs);
+        const int most = pack ? GV_PACK : GV_CHUNK, launches = (count + most - 1) / most;
         for (int l = 0; l < launches; ++l) {
             const int i0 = int((long long)count * l / launches), i1 = int((long long)count * (l + 1) / launches);
+            if (pack) {
+                GemmPack c;
+                c.base = lo;
+                for (int i = i0; i < i1; ++i) {
+                    const GemmDescDev& d = h[i];
+                    c.off[0][i - i0] = unsigned(offset(d.A) / 8);
+                    c.off[1][i - i0] = unsigned(offset(d.B) / 8);
+                    c.off[2][i - i0] = unsigned(offset(d.C) / 8);
+                    c.mnk[0][i - i0] = (unsigned short)d.m;
+                    c.mnk[1][i - i0] = (unsigned short)d.n;
+                    c.mnk[2][i - i0] = (unsigned short)d.k;
+                }
+                auto* kern = ta ? (tb ? k_gemm_pack<true, true> : k_gemm_pack<true, false>)
+                                : (tb ? k_gemm_pack<false, true> : k_gemm_pack<false, false>);
+                hipLaunchKernelGGL(kern, dim3(unsigned(i1 - i0), tiles_of(i0, i1)), dim3(256), 0, s, c, alpha, beta);
+                continue;
+            }
             GemmChunk c;
             std::copy(h.begin() + i0, h.begin() + i1, c.d);
             const dim3 grid(unsigned(i1 - i0), tiles_of(i0, i1));

@@ -84,3 +84,40 @@ def test_batch_state_layouts(kmx_gpu):
     assert torch.equal(y[:s.dof], ref) and not y[s.dof:].any()
     with pytest.raises(ValueError):
         s.apply(long[::2], y, "fp64")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count", [81, 216, 217])
+@pytest.mark.parametrize("ta,tb,beta", [("N", "N", 0.0), ("T", "N", 0.5), ("N", "T", -1.0), ("T", "T", 0.0)])
+def test_packed_descriptors_give_the_same_bits(kmx_gpu, ta, tb, beta, count):
+    """Batches whose descriptors travel packed (leading dimensions the rows stored): the bits
+    of the same products one call each, empty extents and 1 x 1 among them; one leading
+    dimension more than its rows takes the other route."""
+    import torch
+
+    rng = np.random.default_rng(count)
+    gen = torch.Generator().manual_seed(count)
+    shapes = [tuple(int(v) for v in rng.integers(1, 70, 3)) for _ in range(count)]
+    shapes[3], shapes[4], shapes[5], shapes[6] = (1, 1, 1), (0, 7, 5), (7, 5, 0), (64, 64, 130)
+
+    def rnd(n):
+        return torch.randn(max(1, n), dtype=torch.float64, generator=gen).cuda()
+
+    ms, ns, ks = (list(v) for v in zip(*shapes))
+    A, B, C0 = [rnd(m * k) for m, _, k in shapes], [rnd(n * k) for _, n, k in shapes], [rnd(m * n) for m, n, _ in shapes]
+    lda = [max(1, k if ta == "T" else m) for m, _, k in shapes]
+    ldb = [max(1, n if tb == "T" else k) for _, n, k in shapes]
+    ldc = [max(1, m) for m, _, _ in shapes]
+    many, one = [c.clone() for c in C0], [c.clone() for c in C0]
+    kmx_gpu.gemm_vbatched(ta, tb, ms, ns, ks, 1.5, A, lda, B, ldb, beta, many, ldc)
+    for i in range(count):
+        kmx_gpu.gemm_vbatched(ta, tb, [ms[i]], [ns[i]], [ks[i]], 1.5, [A[i]], [lda[i]], [B[i]], [ldb[i]], beta, [one[i]],
+                              [ldc[i]])
+    for i in range(count):
+        assert torch.equal(many[i], one[i]), (i, shapes[i])
+    wide = rnd(71 * 71)
+    other = [c.clone() for c in C0]
+    lda[0] = 71
+    kmx_gpu.gemm_vbatched(ta, tb, ms, ns, ks, 1.5, [wide] + A[1:], lda, B, ldb, beta, other, ldc)
+    for i in range(1, count):
+        assert torch.equal(other[i], one[i]), (i, shapes[i])
