@@ -161,10 +161,81 @@ hipError_t launch(const AsmArgs& g, int deg, size_t lds, unsigned grid, hipStrea
     }
 }
 
+// The operator's diagonal, a workgroup per element: how often the element's row lists the
+// element itself (once in a connectivity list) times sum_t scale_t prod_k of the diagonal
+// blocks' diagonals.
+struct DiagArgs {
+    KArgs<double> a;
+    double* out;
+    int D, deg, B;
+};
+__global__ void __launch_bounds__(AS_THREADS) k_diagonal(DiagArgs g) {
+    __shared__ int own;
+    const KArgs<double>& a = g.a;
+    const int e = blockIdx.x, tid = threadIdx.x, dd = g.deg * g.deg;
+    if (tid == 0) own = a.row_ptr ? 0 : 1;
+    __syncthreads();
+    if (a.row_ptr) {
+        int n = 0;
+        for (long long q = a.row_ptr[e] + tid; q < a.row_ptr[e + 1]; q += AS_THREADS) n += a.cols[q] == e;
+        if (n) atomicAdd(&own, n);
+        __syncthreads();
+    }
+    for (int r = tid; r < g.B; r += AS_THREADS) {
+        double s = 0.0;
+        for (int t = 0; t < a.nterms; ++t) {
+            double p = a.scale[t];
+            int rr = r;
+            for (int k = g.D - 1; k >= 0; --k) {  // digits of r, dim 1 slowest
+                const int r1 = rr / g.deg, ab = (rr - r1 * g.deg) * (g.deg + 1), I = a.idx1d[(long long)e * g.D + k];
+                p *= a.blk[a.off[t * g.D + k] + ((long long)I * a.nb[k] + I) * dd + ab];
+                rr = r1;
+            }
+            s += p;
+        }
+        g.out[(long long)e * g.B + r] = own ? own * s : 0.0;
+    }
+}
+
+// What the kernels here read of a plan
+void operator_args(const kmx_plan* p, KArgs<double>& a) {
+    a.blk = p->d_blk64;
+    for (int i = 0; i < p->T * p->D; ++i) a.off[i] = p->off[i];
+    for (int k = 0; k < p->D; ++k) a.nb[k] = p->nb[k];
+    for (int t = 0; t < p->T; ++t) a.scale[t] = p->scale[t];
+    a.idx1d = p->d_idx1d;
+    a.row_ptr = p->all_pairs ? nullptr : p->d_row_ptr;
+    a.cols = p->all_pairs ? nullptr : p->d_cols;
+    a.N = p->N;
+    a.nterms = p->T;
+}
+
 }  // namespace
 }  // namespace kmx
 
 using namespace kmx;
+
+extern "C" int kmx_plan_diagonal(kmx_plan* p, double* d, void* stream) {
+    if (!p || (p->N > 0 && !d)) {
+        set_error("kmx_plan_diagonal: null argument");
+        return KMX_E_ARG;
+    }
+    if (p->N == 0) return KMX_OK;
+    DiagArgs g;
+    std::memset(&g, 0, sizeof(g));
+    operator_args(p, g.a);
+    g.out = d;
+    g.D = p->D;
+    g.deg = p->deg;
+    g.B = p->B;
+    hipLaunchKernelGGL(k_diagonal, dim3(unsigned(p->N)), dim3(AS_THREADS), 0, reinterpret_cast<hipStream_t>(stream), g);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+        set_error(std::string("kmx_plan_diagonal: ") + hipGetErrorString(e));
+        return KMX_E_HIP;
+    }
+    return KMX_OK;
+}
 
 extern "C" int kmx_plan_assemble(kmx_plan* p, double* blocks, void* stream) {
     if (!p || (p->P > 0 && !blocks)) {
@@ -174,22 +245,13 @@ extern "C" int kmx_plan_assemble(kmx_plan* p, double* blocks, void* stream) {
     if (p->N == 0 || p->P == 0) return KMX_OK;
     AsmArgs g;
     std::memset(&g, 0, sizeof(g));
-    KArgs<double>& a = g.a;
-    a.blk = p->d_blk64;
-    for (int i = 0; i < p->T * p->D; ++i) a.off[i] = p->off[i];
+    operator_args(p, g.a);
     int st = 0;
     for (int k = 0; k < p->D; ++k) {
-        a.nb[k] = p->nb[k];
         g.strip_off[k] = st;
         st += p->nb[k] * p->deg * p->deg;
     }
     g.strip_term = st;
-    for (int t = 0; t < p->T; ++t) a.scale[t] = p->scale[t];
-    a.idx1d = p->d_idx1d;
-    a.row_ptr = p->all_pairs ? nullptr : p->d_row_ptr;
-    a.cols = p->all_pairs ? nullptr : p->d_cols;
-    a.N = p->N;
-    a.nterms = p->T;
     g.out = blocks;
     g.B = p->B;
     const size_t strips = size_t(st) * p->T * sizeof(double);

@@ -36,6 +36,8 @@ struct ArnoldiArgs {
     double* part1;  // [G][k + 1]
     double* part2;  // [G][k + 2]: the second pass's dots and |w1|^2 last
     double* h;      // [k + 2]
+    const double* scale;  // right scaling S (null: none): w = s0 z + s1 u with z = S v_k,
+    double* z;            // u = A z, and the step leaves z = S v_{k+1}
     long long n, chunk;
     double s0, s1;
     int k, G;
@@ -146,7 +148,7 @@ __device__ __forceinline__ void chunk_update(const ArnoldiArgs& a, long long i0,
 
 __global__ void __launch_bounds__(AR_THREADS) k_arnoldi_first(ArnoldiArgs a) {
     const long long i0 = (long long)blockIdx.x * a.chunk, i1 = chunk_end(a, i0);
-    const double* vk = a.V + (long long)a.k * a.n;
+    const double* vk = a.z ? a.z : a.V + (long long)a.k * a.n;
     for (long long i = i0 + threadIdx.x; i < i1; i += AR_THREADS) a.w[i] = a.s0 * vk[i] + a.s1 * a.u[i];
     __syncthreads();
     chunk_dots(a, i0, i1, a.k + 1, a.part1);
@@ -178,7 +180,10 @@ __global__ void __launch_bounds__(AR_THREADS) k_arnoldi_third(ArnoldiArgs a) {
     }
     __syncthreads();
     const double inv = nrm > 0.0 ? 1.0 / nrm : 0.0;  // breakdown: a zero row, h[k + 1] = 0 tells the caller
-    chunk_update(a, i0, i1, sh, a.V + (long long)(a.k + 1) * a.n, inv);
+    double* v = a.V + (long long)(a.k + 1) * a.n;
+    chunk_update(a, i0, i1, sh, v, inv);  // (ends with a barrier)
+    if (a.z)
+        for (long long i = i0 + threadIdx.x; i < i1; i += AR_THREADS) a.z[i] = a.scale[i] * v[i];
     if (blockIdx.x == 0) {  // h = the two passes' coefficients (h1 from the second launch)
         for (int j = threadIdx.x; j <= a.k; j += AR_THREADS) a.h[j] += sh[j];
         if (threadIdx.x == 0) a.h[a.k + 1] = nrm;
@@ -267,7 +272,8 @@ __global__ void __launch_bounds__(AR_THREADS) k_arnoldi_reg_first(ArnoldiArgs a)
     const bool ok = i < i1;
     RegRows<RB> r;
     reg_load<RB>(a, i, ok, q, r);
-    const double wi = ok ? a.s0 * a.V[(long long)a.k * a.n + i] + a.s1 * a.u[i] : 0.0;
+    const double* vk = a.z ? a.z : a.V + (long long)a.k * a.n;
+    const double wi = ok ? a.s0 * vk[i] + a.s1 * a.u[i] : 0.0;
     if (ok && q == 0) a.w[i] = wi;
     reg_dots<RB>(a, r, wi, q, el, a.k + 1, a.part1);
 }
@@ -311,7 +317,10 @@ __global__ void __launch_bounds__(AR_THREADS) k_arnoldi_reg_third(ArnoldiArgs a)
     }
     const double w2 = reg_combine<RB>(a, r, sh, q, el, w1);  // its barrier also publishes nrm
     const double inv = nrm > 0.0 ? 1.0 / nrm : 0.0;
-    if (ok && q == 0) a.V[(long long)(a.k + 1) * a.n + i] = w2 * inv;
+    if (ok && q == 0) {
+        a.V[(long long)(a.k + 1) * a.n + i] = w2 * inv;
+        if (a.z) a.z[i] = a.scale[i] * (w2 * inv);
+    }
     if (blockIdx.x == 0) {  // h = h1 (from the second launch) + h2
         for (int j = threadIdx.x; j <= a.k; j += AR_THREADS) a.h[j] += sh[j];
         if (threadIdx.x == 0) a.h[a.k + 1] = nrm;
@@ -331,13 +340,15 @@ void launch_reg(const ArnoldiArgs& a, hipStream_t s) {
 
 using namespace kmx;
 
-extern "C" int kmx_arnoldi_step(int64_t n, int k, double* V, const double* u, double s0, double s1, double* h,
-                                double* work, void* stream) {
+static int arnoldi(const char* who, int64_t n, int k, double* V, const double* u, double s0, double s1,
+                   const double* scale, double* z, double* h, double* work, void* stream) {
     if (n <= 0 || k < 0 || k > KMX_ARNOLDI_MAX_K || !V || !u || !h || !work) {
-        set_error("kmx_arnoldi_step: bad arguments (n > 0, 0 <= k <= KMX_ARNOLDI_MAX_K, device pointers)");
+        set_error(std::string(who) + ": bad arguments (n > 0, 0 <= k <= KMX_ARNOLDI_MAX_K, device pointers)");
         return KMX_E_ARG;
     }
     ArnoldiArgs a;
+    a.scale = scale;
+    a.z = z;
     a.n = n;
     a.k = k;
     a.G = int(std::min<long long>(AR_MAX_G, (n + AR_MIN_CHUNK - 1) / AR_MIN_CHUNK));
@@ -366,8 +377,22 @@ extern "C" int kmx_arnoldi_step(int64_t n, int k, double* V, const double* u, do
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
-        set_error(std::string("kmx_arnoldi_step: ") + hipGetErrorString(e));
+        set_error(std::string(who) + ": " + hipGetErrorString(e));
         return KMX_E_HIP;
     }
     return KMX_OK;
+}
+
+extern "C" int kmx_arnoldi_step(int64_t n, int k, double* V, const double* u, double s0, double s1, double* h,
+                                double* work, void* stream) {
+    return arnoldi("kmx_arnoldi_step", n, k, V, u, s0, s1, nullptr, nullptr, h, work, stream);
+}
+
+extern "C" int kmx_arnoldi_step_scaled(int64_t n, int k, double* V, const double* u, double s0, double s1,
+                                       const double* scale, double* z, double* h, double* work, void* stream) {
+    if (!scale || !z) {
+        set_error("kmx_arnoldi_step_scaled: null argument");
+        return KMX_E_ARG;
+    }
+    return arnoldi("kmx_arnoldi_step_scaled", n, k, V, u, s0, s1, scale, z, h, work, stream);
 }

@@ -162,6 +162,15 @@ class Plan:
         check(lib().kmx_plan_assemble(self.handle, _ptr(out) if self.P else None, _stream(stream)))
         return out
 
+    def diagonal(self, out=None, stream=None):
+        """The operator's diagonal (kmx_plan_diagonal): a device vector of dof values."""
+        torch = _torch()
+        if out is None:
+            out = torch.empty(self.dof, dtype=torch.float64, device="cuda")
+        self._check_len(out, out)
+        check(lib().kmx_plan_diagonal(self.handle, _ptr(out) if self.dof else None, _stream(stream)))
+        return out
+
     def apply_host(self, x, prec="fp64"):
         """numpy in, numpy out (copies through the library's staging buffers)."""
         x = np.ascontiguousarray(np.asarray(x, dtype=np.float64))
@@ -328,15 +337,23 @@ class RealSpace:
             pass
 
 
-def arnoldi_step(n, k, V, u, s0, s1, h, work, stream=None):
+def arnoldi_step(n, k, V, u, s0, s1, h, work, stream=None, scale=None, z=None):
     """One Arnoldi step on device tensors (kmx_arnoldi_step): w = s0 V[k] + s1 u
     orthogonalised against V[0..k] (classical Gram-Schmidt twice), h[0..k+1] its
     coefficients and norm, V[k+1] = w / |w|.  V: (>= k+2, n) float64, u: n,
-    h: >= k+2, work: kmx._lib.arnoldi_work(n) float64, all CUDA tensors."""
+    h: >= k+2, work: kmx._lib.arnoldi_work(n) float64, all CUDA tensors.
+    scale, z (n values each): the step of M diag(scale), with z = scale V[k] in place of
+    V[k] on entry and z = scale V[k+1] on return (kmx_arnoldi_step_scaled)."""
     if V.dim() != 2 or V.shape[1] != n or V.shape[0] < k + 2 or not V.is_contiguous():
         raise ValueError("arnoldi_step: V must be a contiguous (>= k+2, n) tensor")
     if u.numel() != n or h.numel() < k + 2 or work.numel() < _lib.arnoldi_work(n):
         raise ValueError("arnoldi_step: u, h or work too small")
+    if scale is not None:
+        if scale.numel() != n or z.numel() != n:
+            raise ValueError("arnoldi_step: scale and z must have n values")
+        check(lib().kmx_arnoldi_step_scaled(int(n), int(k), _ptr(V), _ptr(u), float(s0), float(s1), _ptr(scale),
+                                            _ptr(z), _ptr(h), _ptr(work), _stream(stream)))
+        return
     check(lib().kmx_arnoldi_step(int(n), int(k), _ptr(V), _ptr(u), float(s0), float(s1), _ptr(h), _ptr(work),
                                  _stream(stream)))
 

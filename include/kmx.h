@@ -184,6 +184,11 @@ int kmx_apply_transpose(kmx_plan* plan, const double* x, double* y, int prec, vo
  * Asynchronous on `stream`. */
 int kmx_plan_assemble(kmx_plan* plan, double* blocks, void* stream);
 
+/* The diagonal of that operator: d (DEVICE, N * B doubles) gets sum_t scale_t
+ * A_{t,1}[i_1, i_1] ... A_{t,d}[i_d, i_d] at every row i, zero in the rows of elements
+ * whose pair list leaves the element itself out.  Asynchronous on `stream`. */
+int kmx_plan_diagonal(kmx_plan* plan, double* d, void* stream);
+
 /* Host-pointer convenience for callers without device memory (a MEX gateway):
  * copies x in, applies, copies y out, synchronises. */
 int kmx_apply_host(kmx_plan* plan, const double* x_host, double* y_host, int prec);
@@ -255,6 +260,12 @@ int kmx_batch_rk3(kmx_batch* batch, double* const* fs, const double* dts, int ns
 #define KMX_ARNOLDI_WORK(n) ((n) + 32896)
 int kmx_arnoldi_step(int64_t n, int k, double* V, const double* u, double s0, double s1, double* h, double* work,
                      void* stream);
+
+/* The same step for M S, S = diag(scale) a right preconditioner of M = s0 I + s1 A:
+ * z (DEVICE, n doubles) holds S v_k on entry and u the caller's product A z; w = s0 z +
+ * s1 u, and the step leaves z = S v_{k+1} for the next product. */
+int kmx_arnoldi_step_scaled(int64_t n, int k, double* V, const double* u, double s0, double s1, const double* scale,
+                            double* z, double* h, double* work, void* stream);
 
 /* Y = kron(A1,...,Ak) X for k = 1..KMX_KRON_MAX_FACTORS (kron_multd.m:30-42,
  * Kronmult/kronmult{k}.m; k > 6 as kron_multd.m:43-86's recursion).
