@@ -16,8 +16,10 @@
 // product per level tuple added into the output instead -- 84 tuples x 4 launches
 // on a 3D lev 6 grid, each re-reading and adding all 192^3 points -- took 6.5 ms.)
 // The products run on the FP64 matrix cores (kmx_mma64.h).  3D lev 6 deg 3 (192^3
-// points): 0.106 ms, error against 64 bits 3.5e-16 (4.6e-16 before); the last stage,
-// 2.7 GFLOP of dense products, is 71 us of it.  Same terms, summed in another order.
+// points): 0.106 ms with every child in every tile, the last stage's 2.7 GFLOP 71 us of
+// it; 0.076 (44) since a tile of 64 points leaves out the children whose Meval block is
+// zero on it.  Error against 64 bits 3.5e-16 (4.6e-16 by level tuples).  Same terms,
+// summed in another order.
 #include "kmx_internal.h"
 #include "kmx_mma64.h"
 
@@ -45,7 +47,34 @@ struct StageArgs {
     int items;         // node x beta (node alone in the last dimension)
     int mt, nt;        // tiles per item
     int xcd;           // 1: the row tiles of a column tile run on one XCD
+    // Per node and tile of 64 points the children whose Meval block is not zero there
+    // (null: every child everywhere): lptr[node * ptiles + tile], first columns, and the
+    // child's place in its node's list (last dimension: its element).
+    const int* lptr;
+    const int* lcol;
+    const int* lx;
+    int ptiles;
+    // A zero of Meval times an infinity or a NaN is a NaN everywhere: a stage that stores a
+    // value that is not finite sets *flag to the call's number, and the next ones take
+    // every child.  (A replayed graph finds its own number of a run before: the same
+    // sums, only more of them.)
+    int* flag;
+    int call;
 };
+
+// The children that a tile of a node's points sums over.
+struct Children {
+    const int* col;
+    const int* x;  // (null: 0, 1, ...)
+    int n;
+};
+__device__ __forceinline__ Children children(const StageArgs& a, int q, int tile, bool every, const int* x) {
+    const int c0 = a.cptr[q];
+    if (every) return Children{a.col + c0, x ? x + c0 : nullptr, a.cptr[q + 1] - c0};
+    const int l0 = a.lptr[q * a.ptiles + tile];
+    return Children{a.lcol + l0, a.lx + l0, a.lptr[q * a.ptiles + tile + 1] - l0};
+}
+__device__ __forceinline__ bool finite(double v) { return __builtin_fabs(v) <= 1.7976931348623157e308; }
 
 // k / deg and k % deg of a position in a child list (k < 2^28; magic = 2^32 / deg + 1)
 __device__ __forceinline__ void split_k(int k, const StageArgs& a, int& c, int& b) {
@@ -99,13 +128,14 @@ template <class M>
 struct CoefOperand {
     using Map = M;
     const StageArgs& a;
-    int c0, K, beta0, rows;
+    const int* row;  // the children's elements
+    int K, beta0, rows;
     __device__ __forceinline__ void load(int k0, double (&x)[M::N]) {
 #pragma unroll
         for (int u = 0; u < M::N; ++u) {
             int c, b;
             split_k(min(k0 + M::k(u), K - 1), a, c, b);
-            x[u] = mma64_global(a.in)[(long long)a.row[c0 + c] * a.B + (beta0 + min(M::row(u), rows - 1)) * a.deg + b];
+            x[u] = mma64_global(a.in)[(long long)row[c] * a.B + (beta0 + min(M::row(u), rows - 1)) * a.deg + b];
         }
     }
 };
@@ -119,17 +149,33 @@ __global__ void __launch_bounds__(256, 2) k_rs_last(StageArgs a) {
     const int q = int(blockIdx.x) / tiles, t = int(blockIdx.x) - q * tiles;
     if (q >= a.items) return;
     const int i0 = 16 * (t % a.mt), j0 = 64 * (t / a.mt);
-    const int c0 = a.cptr[q], K = (a.cptr[q + 1] - c0) * a.deg;
+    bool every = !a.lptr;
+    if (!every) {  // (or a coefficient of the node that is not finite)
+        const int c0 = a.cptr[q], n = (a.cptr[q + 1] - c0) * a.B;
+        int bad = 0;
+        for (int i = threadIdx.x; i < n; i += 256) {
+            const int c = i / a.B;
+            bad |= !finite(a.in[(long long)a.row[c0 + c] * a.B + i - c * a.B]);
+        }
+        every = __syncthreads_or(bad);
+    }
+    const Children ch = children(a, q, t / a.mt, every, a.row);
+    const int K = ch.n * a.deg;
     auto column = [&](int k) {
         int c, b;
         split_k(k, a, c, b);
-        return a.col[c0 + c] + b;
+        return ch.col[c] + b;
     };
-    CoefOperand<Mma64Map<16, 32, false>> la{a, c0, K, i0, a.nbeta - i0};
+    CoefOperand<Mma64Map<16, 32, false>> la{a, ch.x, K, i0, a.nbeta - i0};
     LineOperand<Mma64Map<64, 32, false>, decltype(column)> lb(column, a.A + j0, a.M, a.M - j0, K);
     double* out = a.out + (long long)q * a.nbeta * a.M;
-    auto st = [&](int i, int j, double v) { out[(long long)(i0 + i) * a.M + j0 + j] = v; };
+    bool bad = false;
+    auto st = [&](int i, int j, double v) {
+        bad |= !finite(v);
+        out[(long long)(i0 + i) * a.M + j0 + j] = v;
+    };
     mma64_tile<16, 32>(a.nbeta - i0, a.M - j0, K, la, lb, st, lds);
+    if (bad) *a.flag = a.call;
 }
 
 // Dimension k < d: Z_k[node; beta; p, r] = sum_k Meval_k(p, k) Z_{k+1}[child(k); beta, b(k); r].
@@ -152,24 +198,31 @@ __global__ void __launch_bounds__(256, 2) k_rs_mode(StageArgs a) {
     const int q = item / a.nbeta, beta = item - q * a.nbeta;
     const int i0 = 64 * rt;
     const long long j0 = 64LL * ct;
-    const int c0 = a.cptr[q], K = (a.cptr[q + 1] - c0) * a.deg;
+    const int c0 = a.cptr[q];
+    const Children ch = children(a, q, rt, !a.lptr || *a.flag == a.call, nullptr);
+    const int K = ch.n * a.deg;
     const int n = int(min(64LL, a.R - j0));
     auto column = [&](int k) {
         int c, b;
         split_k(k, a, c, b);
-        return a.col[c0 + c] + b;
+        return ch.col[c] + b;
     };
     auto line = [&](int k) {  // of Z_{k+1}: child, beta, b
         int c, b;
         split_k(k, a, c, b);
-        return ((c0 + c) * a.nbeta + beta) * a.deg + b;
+        return ((c0 + (ch.x ? ch.x[c] : c)) * a.nbeta + beta) * a.deg + b;
     };
     using Map = Mma64Map<64, 16, false>;
     LineOperand<Map, decltype(column)> la(column, a.A + i0, a.M, a.M - i0, K);
     LineOperand<Map, decltype(line)> lb(line, a.in + j0, a.R, n, K);
     double* out = a.out + (long long)item * a.M * a.R + j0;
-    auto st = [&](int i, int j, double v) { out[(long long)(i0 + i) * a.R + j] = v; };
+    bool bad = false;
+    auto st = [&](int i, int j, double v) {
+        bad |= !finite(v);
+        out[(long long)(i0 + i) * a.R + j] = v;
+    };
     mma64_tile<64, 16>(a.M - i0, n, K, la, lb, st, lds);
+    if (bad) *a.flag = a.call;
 }
 
 __global__ void __launch_bounds__(256) k_zero(double* y, long long n) {
@@ -200,9 +253,13 @@ struct kmx_realspace {
         int nodes = 0;
         int* d_cptr = nullptr;
         int* d_col = nullptr;
+        int* d_list = nullptr;  // lptr, lcol, lx of StageArgs (null: no lists)
+        size_t o_col = 0, o_x = 0;
     };
     Stage stage[KMX_MAX_DIM];
     int* d_row = nullptr;                   // elements in prefix order
+    int* d_flag = nullptr;
+    unsigned calls = 0;
     double* d_buf[2] = {nullptr, nullptr};  // Z_d, Z_{d-1}, ... in turn
 };
 
@@ -212,10 +269,51 @@ static void free_rs(kmx_realspace* r) {
     for (auto& st : r->stage) {
         if (st.d_cptr) hipFree(st.d_cptr);
         if (st.d_col) hipFree(st.d_col);
+        if (st.d_list) hipFree(st.d_list);
     }
+    if (r->d_flag) hipFree(r->d_flag);
     if (r->d_row) hipFree(r->d_row);
     for (auto& b : r->d_buf)
         if (b) hipFree(b);
+}
+
+// The lists of StageArgs for dimension k, where they leave out a tenth of the products or
+// more: a wavelet of level l is zero on all but 2^(1-l) of its dimension, exactly, so a
+// tile of 64 of 192 points meets 0.42 of 64 cells' blocks, of 3072 points 0.036 of 512's.
+// Leaving a zero block out leaves every sum's bits as they are.
+template <class UP>
+static void build_lists(kmx_realspace* r, int k, const double* meval, const std::vector<int>& cptr,
+                        const std::vector<int>& col, const std::vector<int>& order, const UP& up) {
+    const int M = r->npts[k], deg = r->deg, tiles = (M + 63) / 64, blocks = r->ncols[k] / deg;
+    if (tiles < 2 || col.empty()) return;
+    std::vector<unsigned char> on(size_t(tiles) * blocks, 0);
+    for (int b = 0; b < blocks; ++b)
+        for (int t = 0; t < tiles; ++t) {
+            bool any = false;
+            for (int c = b * deg; c < (b + 1) * deg && !any; ++c)
+                for (int i = 64 * t; i < std::min(M, 64 * t + 64) && !any; ++i) any = !(meval[size_t(c) * M + i] == 0.0);
+            on[size_t(t) * blocks + b] = any;
+        }
+    const int nodes = int(cptr.size()) - 1;
+    if (double(col.size()) * tiles > 1e8) return;
+    std::vector<int> ptr, lcol, lx;
+    for (int q = 0; q < nodes; ++q)
+        for (int t = 0; t < tiles; ++t) {
+            ptr.push_back(int(lcol.size()));
+            for (int c = cptr[size_t(q)]; c < cptr[size_t(q) + 1]; ++c)
+                if (on[size_t(t) * blocks + col[size_t(c)] / deg] ||
+                    (c + 1 == cptr[size_t(q) + 1] && int(lcol.size()) == ptr.back())) {  // (no list is empty)
+                    lcol.push_back(col[size_t(c)]);
+                    lx.push_back(k + 1 == r->D ? order[size_t(c)] : c - cptr[size_t(q)]);
+                }
+        }
+    ptr.push_back(int(lcol.size()));
+    if (double(lcol.size()) > 0.9 * double(col.size()) * tiles) return;
+    r->stage[k].o_col = ptr.size();
+    r->stage[k].o_x = ptr.size() + lcol.size();
+    ptr.insert(ptr.end(), lcol.begin(), lcol.end());
+    ptr.insert(ptr.end(), lx.begin(), lx.end());
+    up(ptr, r->stage[k].d_list);
 }
 
 extern "C" int kmx_realspace_create(int ndim, int deg, int num_elem, const int* elem_idx1d, int index_base,
@@ -311,6 +409,7 @@ extern "C" int kmx_realspace_create(int ndim, int deg, int num_elem, const int* 
             r->stage[k].nodes = int(par.size());
             up(cptr, r->stage[k].d_cptr);
             up(col, r->stage[k].d_col);
+            build_lists(r, k, meval[k], cptr, col, order, up);
             if (k > 0) {  // Z_{k+1} of the comment above (k from 1 there)
                 R *= npts[k];
                 long long nb = 1;
@@ -319,6 +418,7 @@ extern "C" int kmx_realspace_create(int ndim, int deg, int num_elem, const int* 
             }
         }
         up(order, r->d_row);
+        up(std::vector<int>(1, 0), r->d_flag);
         for (int q = 0; q < 2; ++q)
             if (hipMalloc(&r->d_buf[q], size_t(need[q]) * sizeof(double)) != hipSuccess) throw std::bad_alloc();
         *out = r;
@@ -346,6 +446,8 @@ extern "C" int kmx_realspace_apply(kmx_realspace* r, const double* f_w, double* 
     const int D = r->D;
     const double* cur = f_w;
     long long R = 1;
+    if (++r->calls == 0) r->calls = 1;  // never the flag's first value
+    const int call = int(r->calls);
     for (int k = D - 1; k >= 0 && r->N > 0; --k) {
         StageArgs a;
         a.in = cur;
@@ -354,6 +456,13 @@ extern "C" int kmx_realspace_apply(kmx_realspace* r, const double* f_w, double* 
         a.cptr = r->stage[k].d_cptr;
         a.col = r->stage[k].d_col;
         a.row = r->d_row;
+        const kmx_realspace::Stage& st = r->stage[k];
+        a.lptr = st.d_list;
+        a.lcol = st.d_list ? st.d_list + st.o_col : nullptr;
+        a.lx = st.d_list ? st.d_list + st.o_x : nullptr;
+        a.ptiles = (r->npts[k] + 63) / 64;
+        a.flag = r->d_flag;
+        a.call = call;
         a.R = R;
         a.M = r->npts[k];
         a.deg = r->deg;

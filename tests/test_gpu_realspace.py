@@ -126,3 +126,59 @@ def test_realspace_no_elements(kmx_gpu):
     out = torch.full((15,), 7.0, dtype=torch.float64, device="cuda")
     rs.apply(torch.empty(0, dtype=torch.float64, device="cuda"), out)
     assert torch.count_nonzero(out) == 0
+
+
+def _dense(meval, idx, deg, f):
+    """The definition with every zero of Meval multiplied (so 0 x inf is a NaN)."""
+    B = deg ** len(meval)
+    out = np.zeros(int(np.prod([m.shape[0] for m in meval])))
+    with np.errstate(invalid="ignore"):
+        for e, row in enumerate(np.asarray(idx) - 1):
+            M = np.ones((1, 1))
+            for m, J in zip(meval, row):
+                M = np.kron(M, m[:, J * deg:(J + 1) * deg])
+            out += (M * f[e * B:(e + 1) * B]).sum(axis=1)
+    return out
+
+
+@pytest.mark.parametrize("nd,lev,deg,npts", [(1, 6, 3, None), (2, 5, 3, None), (3, 4, 2, (96, 40, 130)),
+                                             (2, 5, 2, (65, 64)), (2, 3, 2, (400, 1))])
+def test_realspace_children_by_tile(kmx_gpu, nd, lev, deg, npts):
+    """Plotting grids of several tiles, where a tile sums over the children that are not zero
+    on it: against the definition, with and without values that are not finite, the finite
+    call after one that was not, and replayed."""
+    import torch
+    from kmx import coeffs as K
+    from kmx import grid as G
+
+    idx = G.hash_table_sparse_nd([lev] * nd, lev, "SG").idx1d
+    meval = [K.matrix_plot_D(deg, lev, -1.0, 1.0)[0] for _ in range(nd)]
+    if npts:  # other numbers of points: rows repeated or left out
+        meval = [m[np.arange(n) * m.shape[0] // n] for m, n in zip(meval, npts)]
+    meval[0] = meval[0].copy()
+    meval[0][:, -deg:] = 0.0  # a block that is zero everywhere
+    rng = np.random.default_rng(nd + lev)
+    f = rng.standard_normal(len(idx) * deg ** nd)
+    rs = kmx_gpu.RealSpace(meval, idx, deg, index_base=1)
+    want = _dense(meval, idx, deg, f)
+    got = rs.apply(torch.from_numpy(f).cuda())
+    assert rel(got.cpu().numpy(), want) <= 1e-13
+    fd, out = torch.from_numpy(f).cuda(), torch.empty_like(got)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        rs.apply(fd, out)
+    last = len(idx) - 1  # (its first index is the finest: perhaps of the zero block)
+    for at, v in ((0, np.inf), (f.size // 2, np.nan), (last * deg ** nd, -np.inf), (f.size - 1, np.inf)):
+        g = f.copy()
+        g[at] = v
+        ref = _dense(meval, idx, deg, g)
+        bad = rs.apply(torch.from_numpy(g).cuda()).cpu().numpy()
+        assert np.array_equal(np.isnan(bad), np.isnan(ref)) and np.array_equal(bad == np.inf, ref == np.inf)
+        assert np.array_equal(bad == -np.inf, ref == -np.inf)
+        assert torch.equal(rs.apply(torch.from_numpy(f).cuda()), got)
+        fd.copy_(torch.from_numpy(g))
+        graph.replay()
+        assert np.array_equal(np.nan_to_num(out.cpu().numpy(), nan=1.5), np.nan_to_num(bad, nan=1.5))
+        fd.copy_(torch.from_numpy(f))
+        graph.replay()
+        assert torch.equal(out, got)
