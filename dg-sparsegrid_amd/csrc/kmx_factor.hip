@@ -920,6 +920,13 @@ int kmx_factor_apply(kmx_plan* p, bool transpose, const KArgs<double>& k, hipStr
     a.splits = f->splits;
     std::lock_guard<std::mutex> lock(f->mu);
     if (f->used && f->last != s) {  // the workspace passes to another stream
+        // a last stream that records a graph now cannot be ordered against: pair by pair
+        const hipError_t q = hipStreamIsCapturing(f->last, &cap);
+        if (cap != hipStreamCaptureStatusNone || q == hipErrorStreamCaptureImplicit) {
+            (void)hipGetLastError();
+            return 0;
+        }
+        (void)hipGetLastError();
         if (hipEventRecord(f->ev, f->last) != hipSuccess || hipStreamWaitEvent(s, f->ev, 0) != hipSuccess) {
             (void)hipGetLastError();  // (a stream that is gone, or captures now)
             if (hipDeviceSynchronize() != hipSuccess) {

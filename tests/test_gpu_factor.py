@@ -147,3 +147,34 @@ def test_streams_threads_and_capture(kmx_gpu):
         g.replay()
         torch.cuda.synchronize()
         assert float((y - ref).norm() / ref.norm()) <= 1e-13
+
+
+def test_apply_while_the_last_stream_records_a_graph(kmx_gpu):
+    """The stream of the last apply records a graph now: an apply on another stream runs at
+    once, outside the graph."""
+    import torch
+
+    mats, idx, rp, cols, _ = case(3, 3, 2, 2, True, seed=5)
+    plan = kmx_gpu.Plan(mats, idx, 2, rp, cols)
+    x = torch.from_numpy(np.random.default_rng(1).standard_normal(plan.dof)).cuda()
+    ref = plan.apply(x).clone()
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    outs = [torch.zeros_like(x) for _ in range(3)]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(a):
+        plan.apply(x, outs[0])
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=a):
+        plan.apply(x, outs[1])
+        with torch.cuda.stream(b):
+            plan.apply(x, outs[2])
+    b.synchronize()
+    assert rel(outs[2].cpu().numpy(), ref.cpu().numpy()) <= 1e-13
+    assert not outs[1].any()
+    for _ in range(3):
+        outs[2].zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert rel(outs[1].cpu().numpy(), ref.cpu().numpy()) <= 1e-13
+        assert not outs[2].any()
