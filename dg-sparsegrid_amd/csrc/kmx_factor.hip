@@ -43,8 +43,10 @@
 #include "kmx_kernels.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cstdlib>
 #include <cstring>
+#include <future>
 #include <map>
 #include <mutex>
 #include <numeric>
@@ -513,6 +515,25 @@ T* fac_upload(const std::vector<T>& h) {
     return d;
 }
 
+// f(begin, end) over [0, n), in up to four parts at a time where `many`
+template <class F>
+void in_parts(int n, bool many, const F& f) {
+    const int parts = many ? std::min(4, n) : 1;
+    std::vector<std::future<void>> others;
+    int done = 0;
+    for (int q = 1; q < parts; ++q) {
+        const int end = int((long long)n * q / parts);
+        try {
+            others.push_back(std::async(std::launch::async, [&f, done, end] { f(done, end); }));
+        } catch (const std::system_error&) {
+            break;  // no thread to be had: the rest here
+        }
+        done = end;
+    }
+    f(done, n);
+    for (auto& o : others) o.get();
+}
+
 // Per dimension the 1D connections of a pair list that is their tensor product over the
 // element set (every pair list row equals the product's row, as sets, without
 // repetitions); false if it is not one.
@@ -521,40 +542,64 @@ bool product_masks(const kmx_plan* p, const std::vector<int>& idx, const std::ve
     const int D = p->D, N = p->N;
     const size_t words = (size_t(N) + 63) / 64;
     double bits = double(N) * double(words) * 8.0;
-    for (int d = 0; d < D; ++d) bits += double(p->nb[d]) * double(words) * 8.0;
+    for (int d = 0; d < D; ++d) bits += double(p->nb[d]) * double(words) * 16.0;
     if (bits > 512e6) return false;
     typedef unsigned long long word;
-    // the rows as bit sets
+    // (3D lev 7, 1,903,000 pairs: the plan took 5.0 ms without this check, 8.7 with it in one
+    // thread and a bit at a time, under 5.5 so)
+    const bool many = rp[size_t(N)] > 100000;
+    std::atomic<bool> product{true};
+    // the rows as bit sets: a word stays in a register while consecutive columns lie in it
     std::vector<word> rows(size_t(N) * words, 0);
-    for (int i = 0; i < N; ++i) {
-        word* row = &rows[size_t(i) * words];
-        for (long long q = rp[size_t(i)]; q < rp[size_t(i) + 1]; ++q) {
-            word& wd = row[size_t(cols[size_t(q)]) / 64];
-            const word bit = word(1) << (cols[size_t(q)] % 64);
-            if (wd & bit) return false;  // a pair listed twice
-            wd |= bit;
+    in_parts(N, many, [&](int i0, int i1) {
+        for (int i = i0; i < i1; ++i) {
+            word* row = &rows[size_t(i) * words];
+            const int* c = cols.data() + rp[size_t(i)];
+            const int* const end = cols.data() + rp[size_t(i) + 1];
+            while (c != end) {
+                const unsigned at = unsigned(*c) / 64;
+                word bits = 0;
+                do bits |= word(1) << (unsigned(*c) % 64);
+                while (++c != end && unsigned(*c) / 64 == at);
+                row[at] |= bits;
+            }
+            long long held = 0;
+            for (size_t k = 0; k < words; ++k) held += __builtin_popcountll(row[k]);
+            if (held != rp[size_t(i) + 1] - rp[size_t(i)]) product = false;  // a pair listed twice
         }
-    }
+    });
+    if (!product) return false;
     // per dimension: (I, J) is connected where a row with index I holds an element with index
     // J; conn: per I the elements j whose J_d is connected to it
     std::vector<std::vector<word>> conn(static_cast<size_t>(D));
     mask.assign(size_t(D), {});
-    for (int d = 0; d < D; ++d) {
-        const int nb = p->nb[d];
-        mask[size_t(d)].assign(size_t(nb) * nb, 0);
-        conn[size_t(d)].assign(size_t(nb) * words, 0);
-        std::vector<word>& c = conn[size_t(d)];
-        for (int i = 0; i < N; ++i)
-            for (size_t k = 0; k < words; ++k) c[size_t(idx[size_t(i) * D + d]) * words + k] |= rows[size_t(i) * words + k];
-        for (int I = 0; I < nb; ++I) {
-            word* set = &c[size_t(I) * words];
-            unsigned char* m = &mask[size_t(d)][size_t(I) * nb];
-            for (int j = 0; j < N; ++j)
-                if (set[size_t(j) / 64] >> (j % 64) & 1) m[idx[size_t(j) * D + d]] = 1;
-            for (int j = 0; j < N; ++j)
-                if (m[idx[size_t(j) * D + d]]) set[size_t(j) / 64] |= word(1) << (j % 64);
+    in_parts(D, many, [&](int d0, int d1) {
+        for (int d = d0; d < d1; ++d) {
+            const int nb = p->nb[d];
+            std::vector<unsigned char>& md = mask[size_t(d)];
+            std::vector<word>& c = conn[size_t(d)];
+            md.assign(size_t(nb) * nb, 0);
+            c.assign(size_t(nb) * words, 0);
+            std::vector<word> with(size_t(nb) * words, 0);  // per J the elements that have it
+            for (int i = 0; i < N; ++i) {
+                const size_t I = size_t(idx[size_t(i) * D + d]);
+                with[I * words + size_t(i) / 64] |= word(1) << (i % 64);
+                for (size_t k = 0; k < words; ++k) c[I * words + k] |= rows[size_t(i) * words + k];
+            }
+            for (int I = 0; I < nb; ++I) {
+                word* set = &c[size_t(I) * words];
+                for (int J = 0; J < nb; ++J) {
+                    const word* w = &with[size_t(J) * words];
+                    word any = 0;
+                    for (size_t k = 0; k < words; ++k) any |= set[k] & w[k];
+                    md[size_t(I) * nb + J] = any != 0;
+                }
+                for (int J = 0; J < nb; ++J)
+                    if (md[size_t(I) * nb + J])
+                        for (size_t k = 0; k < words; ++k) set[k] |= with[size_t(J) * words + k];
+            }
         }
-    }
+    });
     for (int i = 0; i < N; ++i)
         for (size_t k = 0; k < words; ++k) {
             word m = ~word(0);
