@@ -172,8 +172,10 @@ __device__ __forceinline__ int xcd_item(int items) {
 // t[l]: the sums below suffix dimension K + 1 + l; the element's block is contracted
 // along dimension D into t[S - 1], and when the walk leaves a node of depth D - f its
 // sum is contracted along that dimension into the level above.
+// Four waves a SIMD, but three in 3D deg 4, whose 160 registers spilled at four (lev 7, 3
+// terms: 223 us an apply then, 119 at three; lev 6, diffusion: 64, 40).
 template <int D, int DEG>
-__global__ void __launch_bounds__(DOWN_WAVES * 64, 4) k_factor_down(FacArgs a) {
+__global__ void __launch_bounds__(DOWN_WAVES * 64, (D == 3 && DEG == 4 ? 3 : 4)) k_factor_down(FacArgs a) {
     using F = FacShape<D, DEG>;
     constexpr int K = F::K, S = F::S, BS = F::BS;
     static_assert(S >= 1 && S <= 3, "up to three suffix dimensions");
