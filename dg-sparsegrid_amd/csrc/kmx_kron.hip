@@ -565,8 +565,9 @@ bool kron_args_ok(int k, const int* nrow, const int* ncol, const double* const* 
     return true;
 }
 
+// work: 2 chain_workspace() doubles of the caller's for the intermediates, or null
 int kronmult(const char* who, int k, const int* nrow, const int* ncol, const double* const* A,
-             const unsigned char* rowmajor, const double* X, int nvec, double* Y, void* stream) {
+             const unsigned char* rowmajor, const double* X, int nvec, double* Y, double* work, void* stream) {
     if (!kron_args_ok(k, nrow, ncol, A, X, nvec, Y)) {
         set_error(std::string(who) + ": bad arguments");
         return KMX_E_ARG;
@@ -575,7 +576,10 @@ int kronmult(const char* who, int k, const int* nrow, const int* ncol, const dou
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const std::vector<ChainStep> steps = plan_chain(k, nrow, ncol, nvec, X, Y);
     double* buf[2] = {nullptr, nullptr};
-    if (steps.size() > 1) {  // intermediates between the launches
+    if (steps.size() > 1 && work) {
+        buf[0] = work;
+        buf[1] = work + chain_workspace(k, nrow, ncol, nvec);
+    } else if (steps.size() > 1) {  // intermediates between the launches
         const long long maxsz = chain_workspace(k, nrow, ncol, nvec);
         if (hipMalloc(&buf[0], sizeof(double) * maxsz) != hipSuccess ||
             (steps.size() > 2 && hipMalloc(&buf[1], sizeof(double) * maxsz) != hipSuccess)) {
@@ -585,7 +589,7 @@ int kronmult(const char* who, int k, const int* nrow, const int* ncol, const dou
         }
     }
     const hipError_t e = launch_chain(steps, k, nrow, ncol, A, rowmajor, X, nvec, Y, buf, s);
-    if (buf[0]) {
+    if (buf[0] && !work) {
         hipStreamSynchronize(s);
         hipFree(buf[0]);
         if (buf[1]) hipFree(buf[1]);
@@ -601,7 +605,7 @@ int kronmult(const char* who, int k, const int* nrow, const int* ncol, const dou
 
 extern "C" int kmx_kronmult(int k, const int* nrow, const int* ncol, const double* const* A, const double* X,
                             int nvec, double* Y, void* stream) {
-    return kronmult("kmx_kronmult", k, nrow, ncol, A, nullptr, X, nvec, Y, stream);
+    return kronmult("kmx_kronmult", k, nrow, ncol, A, nullptr, X, nvec, Y, nullptr, stream);
 }
 
 // ---- kmx_kronmult without allocation: the chain's two intermediates live in one
@@ -668,9 +672,16 @@ extern "C" int kmx_kronmult_noalloc(int k, const int* nrow, const int* ncol, con
     return kronmult_noalloc("kmx_kronmult_noalloc", k, nrow, ncol, A, nullptr, X, nvec, Y, stream);
 }
 
+extern "C" int64_t kmx_kronmult_work(int k, const int* nrow, const int* ncol, int nvec) {
+    if (k < 1 || k > KMX_KRON_MAX_FACTORS || !nrow || !ncol || nvec < 1) return 0;
+    for (int i = 0; i < k; ++i)
+        if (nrow[i] < 1 || ncol[i] < 1) return 0;
+    return k == 1 ? 0 : 2 * chain_workspace(k, nrow, ncol, nvec);
+}
+
 extern "C" int kmx_kronmult_layout(int k, const int* nrow, const int* ncol, const double* const* A,
                                    const unsigned char* rowmajor, const double* X, int nvec, double* Y, int noalloc,
-                                   void* stream) {
+                                   double* work, void* stream) {
     if (rowmajor && kron_args_ok(k, nrow, ncol, A, X, nvec, Y)) {
         long long values = 0;
         bool any = false;
@@ -684,7 +695,7 @@ extern "C" int kmx_kronmult_layout(int k, const int* nrow, const int* ncol, cons
         }
     }
     return noalloc ? kronmult_noalloc("kmx_kronmult_layout", k, nrow, ncol, A, rowmajor, X, nvec, Y, stream)
-                   : kronmult("kmx_kronmult_layout", k, nrow, ncol, A, rowmajor, X, nvec, Y, stream);
+                   : kronmult("kmx_kronmult_layout", k, nrow, ncol, A, rowmajor, X, nvec, Y, work, stream);
 }
 
 extern "C" int kmx_gemm_vbatched(char transA, char transB, const int* m, const int* n, const int* k, double alpha,

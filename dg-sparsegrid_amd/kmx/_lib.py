@@ -22,6 +22,7 @@ PREC_BF16 = 3
 
 KRON_SCRATCH_ELEMS = 1 << 20
 KRON_ROWMAJOR_VALUES = 1000  # KMX_KRON_ROWMAJOR_VALUES
+KRON_ONE_LAUNCH = 8448  # a chain whose extents never exceed this is one launch (kmx_kron.hip KG_TILE)
 ARNOLDI_MAX_K = 127
 
 
@@ -163,7 +164,9 @@ PROTOTYPES = {
     "kmx_kronmult_noalloc": (C.c_int, [C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_void_p),
                                        C.c_void_p, C.c_int, C.c_void_p, C.c_void_p]),
     "kmx_kronmult_layout": (C.c_int, [C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_void_p),
-                                      C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_void_p]),
+                                      C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_int, C.c_void_p,
+                                      C.c_void_p]),
+    "kmx_kronmult_work": (C.c_int64, [C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int), C.c_int]),
     "kmx_gemm_vbatched": (C.c_int, [C.c_char, C.c_char, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_int),
                                     C.c_double, C.POINTER(C.c_void_p), C.POINTER(C.c_int), C.POINTER(C.c_void_p),
                                     C.POINTER(C.c_int), C.c_double, C.POINTER(C.c_void_p), C.POINTER(C.c_int), C.c_int,

@@ -293,11 +293,14 @@ int kmx_kronmult_noalloc(int k, const int* nrow, const int* ncol, const double* 
 /* kmx_kronmult (noalloc = 0) or kmx_kronmult_noalloc (noalloc != 0) with factors stored
  * by columns or by rows: rowmajor[i] != 0 says that A[i] is row-major (null: none is), so
  * that row-major callers need no transposed copies.  The same results.  With a row-major
- * factor, all factors together may have KMX_KRON_ROWMAJOR_VALUES values (else KMX_E_SHAPE). */
+ * factor, all factors together may have KMX_KRON_ROWMAJOR_VALUES values (else KMX_E_SHAPE).
+ * work (noalloc = 0): null, or kmx_kronmult_work's doubles of DEVICE memory for the chain's
+ * intermediates, clear of X and Y: then nothing is allocated and the call is asynchronous. */
 #define KMX_KRON_ROWMAJOR_VALUES 1000
+int64_t kmx_kronmult_work(int k, const int* nrow, const int* ncol, int nvec);
 int kmx_kronmult_layout(int k, const int* nrow, const int* ncol, const double* const* A,
                         const unsigned char* rowmajor, const double* X, int nvec, double* Y, int noalloc,
-                        void* stream);
+                        double* work, void* stream);
 
 /* Variable-size batched GEMM (Kronmult/gemm_vbatched.m:1-38, magmablas-style):
  * C_i = alpha*op(A_i)*op(B_i) + beta*C_i with op from transA/transB ('N'/'T'),

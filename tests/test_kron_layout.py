@@ -13,16 +13,17 @@ def test_rowmajor_factors_beyond_the_limit_are_refused():
     n = (C.c_int * 2)(25, 25)
     one = (C.c_void_p * 2)(8, 8)  # never read: 1250 values are refused before any launch
     args = (2, n, n, one)
-    assert lib.kmx_kronmult_layout(*args, bytes([0, 1]), 8, 1, 8, 0, None) == L.KMX_E_SHAPE
-    assert lib.kmx_kronmult_layout(*args, bytes([0, 1]), 8, 1, 8, 1, None) == L.KMX_E_SHAPE
-    assert lib.kmx_kronmult_layout(*args, bytes([1, 1]), 8, 0, None, 0, None) == L.KMX_E_ARG
+    assert lib.kmx_kronmult_layout(*args, bytes([0, 1]), 8, 1, 8, 0, None, None) == L.KMX_E_SHAPE
+    assert lib.kmx_kronmult_layout(*args, bytes([0, 1]), 8, 1, 8, 1, None, None) == L.KMX_E_SHAPE
+    assert lib.kmx_kronmult_layout(*args, bytes([1, 1]), 8, 0, None, 0, None, None) == L.KMX_E_ARG
 
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("noalloc", [False, True])
 @pytest.mark.parametrize("shapes,nvec", [([(3, 5)], 1), ([(1, 4), (6, 1), (2, 3)], 7), ([(8, 8)] * 4, 9),
                                          ([(16, 16)] * 3, 5), ([(31, 2), (7, 31), (4, 9)], 33), ([(25, 40)], 3),
-                                         ([(25, 40), (2, 3)], 3), ([(500, 1), (1, 400)], 2), ([(2, 2)] * 12, 1)])
+                                         ([(25, 40), (2, 3)], 3), ([(500, 1), (1, 400)], 2), ([(2, 2)] * 12, 1),
+                                         ([(6, 5)] * 6, 3)])
 def test_factor_layouts_give_the_same_bits(kmx_gpu, shapes, nvec, noalloc):
     """Factors by rows, by columns, as strided views, alone and mixed, up to and beyond the
     values taken by rows: the bits of column-major factors (given Y: copies are made)."""
