@@ -15,9 +15,15 @@
 // each row itself (G <= 128: 16 threads per row each summing at most 8), so no
 // launch waits on a separate reduction.  Every launch has a fixed shape for given
 // (n, k) and allocates nothing, so the step can be captured in a graph.
+// On vectors in the separable sweep's box order the slot sum and the box copy of the
+// product are contiguous, so the first launch forms u itself and the third writes the
+// next box copy: the ops and three launches a step, where the apply's three and three
+// took 13 + 18 us of launches (6D lev 4 deg 2, a whole BE step 2.98 -> 2.70 ms; a step
+// is bound by the latency of its four dependent launches, 4 to 8 us each).
 #include "kmx_internal.h"
 
 #include <algorithm>
+#include <cstring>
 
 namespace kmx {
 namespace {
@@ -38,6 +44,13 @@ struct ArnoldiArgs {
     double* h;      // [k + 2]
     const double* scale;  // right scaling S (null: none): w = s0 z + s1 u with z = S v_k,
     double* z;            // u = A z, and the step leaves z = S v_{k+1}
+    // in box order (box != null): u_i is the sum of the sweep's slots at i (0 where map[i] <
+    // 0), and z's box copy is written beside z
+    void* box;
+    const int* map;
+    long long nb;
+    int nslot;
+    bool f32;
     long long n, chunk;
     double s0, s1;
     int k, G;
@@ -45,6 +58,27 @@ struct ArnoldiArgs {
 
 __device__ __forceinline__ long long chunk_end(const ArnoldiArgs& a, long long i0) {
     return i0 + a.chunk < a.n ? i0 + a.chunk : a.n;
+}
+
+// u at i: the caller's, or the sweep's slots there in op order (as its own slot sum adds them)
+__device__ __forceinline__ double product_at(const ArnoldiArgs& a, long long i) {
+    if (!a.box) return a.u[i];
+    double v = 0.0;
+    if (a.f32) {
+        const float* sl = static_cast<const float*>(a.box) + a.nb + i;
+        for (int q = 0; q < a.nslot; ++q) v += double(sl[(long long)q * a.nb]);
+    } else {
+        const double* sl = static_cast<const double*>(a.box) + a.nb + i;
+        for (int q = 0; q < a.nslot; ++q) v += sl[(long long)q * a.nb];
+    }
+    return a.map[i] >= 0 ? v : 0.0;
+}
+__device__ __forceinline__ void put_z(const ArnoldiArgs& a, long long i, double v) {
+    const double z = a.scale[i] * v;
+    a.z[i] = z;
+    if (!a.box || a.map[i] < 0) return;
+    if (a.f32) static_cast<float*>(a.box)[i] = float(z);
+    else static_cast<double*>(a.box)[i] = z;
 }
 
 __device__ __forceinline__ double wave_sum(double v) {
@@ -149,7 +183,7 @@ __device__ __forceinline__ void chunk_update(const ArnoldiArgs& a, long long i0,
 __global__ void __launch_bounds__(AR_THREADS) k_arnoldi_first(ArnoldiArgs a) {
     const long long i0 = (long long)blockIdx.x * a.chunk, i1 = chunk_end(a, i0);
     const double* vk = a.z ? a.z : a.V + (long long)a.k * a.n;
-    for (long long i = i0 + threadIdx.x; i < i1; i += AR_THREADS) a.w[i] = a.s0 * vk[i] + a.s1 * a.u[i];
+    for (long long i = i0 + threadIdx.x; i < i1; i += AR_THREADS) a.w[i] = a.s0 * vk[i] + a.s1 * product_at(a, i);
     __syncthreads();
     chunk_dots(a, i0, i1, a.k + 1, a.part1);
 }
@@ -183,7 +217,7 @@ __global__ void __launch_bounds__(AR_THREADS) k_arnoldi_third(ArnoldiArgs a) {
     double* v = a.V + (long long)(a.k + 1) * a.n;
     chunk_update(a, i0, i1, sh, v, inv);  // (ends with a barrier)
     if (a.z)
-        for (long long i = i0 + threadIdx.x; i < i1; i += AR_THREADS) a.z[i] = a.scale[i] * v[i];
+        for (long long i = i0 + threadIdx.x; i < i1; i += AR_THREADS) put_z(a, i, v[i]);
     if (blockIdx.x == 0) {  // h = the two passes' coefficients (h1 from the second launch)
         for (int j = threadIdx.x; j <= a.k; j += AR_THREADS) a.h[j] += sh[j];
         if (threadIdx.x == 0) a.h[a.k + 1] = nrm;
@@ -273,7 +307,7 @@ __global__ void __launch_bounds__(AR_THREADS) k_arnoldi_reg_first(ArnoldiArgs a)
     RegRows<RB> r;
     reg_load<RB>(a, i, ok, q, r);
     const double* vk = a.z ? a.z : a.V + (long long)a.k * a.n;
-    const double wi = ok ? a.s0 * vk[i] + a.s1 * a.u[i] : 0.0;
+    const double wi = ok ? a.s0 * vk[i] + a.s1 * product_at(a, i) : 0.0;
     if (ok && q == 0) a.w[i] = wi;
     reg_dots<RB>(a, r, wi, q, el, a.k + 1, a.part1);
 }
@@ -319,12 +353,25 @@ __global__ void __launch_bounds__(AR_THREADS) k_arnoldi_reg_third(ArnoldiArgs a)
     const double inv = nrm > 0.0 ? 1.0 / nrm : 0.0;
     if (ok && q == 0) {
         a.V[(long long)(a.k + 1) * a.n + i] = w2 * inv;
-        if (a.z) a.z[i] = a.scale[i] * (w2 * inv);
+        if (a.z) put_z(a, i, w2 * inv);
     }
     if (blockIdx.x == 0) {  // h = h1 (from the second launch) + h2
         for (int j = threadIdx.x; j <= a.k; j += AR_THREADS) a.h[j] += sh[j];
         if (threadIdx.x == 0) a.h[a.k + 1] = nrm;
     }
+}
+
+__global__ void __launch_bounds__(256) k_box_start(ArnoldiArgs a, const double* v) {
+    const long long i = blockIdx.x * 256ll + threadIdx.x;
+    if (i < a.n) put_z(a, i, v[i]);
+}
+__global__ void __launch_bounds__(256) k_to_box(const double* x, double* xb, const int* map, long long nb) {
+    const long long i = blockIdx.x * 256ll + threadIdx.x;
+    if (i < nb) xb[i] = map[i] >= 0 ? x[map[i]] : 0.0;
+}
+__global__ void __launch_bounds__(256) k_from_box(const double* xb, double* x, const int* map, long long nb) {
+    const long long i = blockIdx.x * 256ll + threadIdx.x;
+    if (i < nb && map[i] >= 0) x[map[i]] = xb[i];
 }
 
 template <int RB>
@@ -340,15 +387,24 @@ void launch_reg(const ArnoldiArgs& a, hipStream_t s) {
 
 using namespace kmx;
 
-static int arnoldi(const char* who, int64_t n, int k, double* V, const double* u, double s0, double s1,
-                   const double* scale, double* z, double* h, double* work, void* stream) {
-    if (n <= 0 || k < 0 || k > KMX_ARNOLDI_MAX_K || !V || !u || !h || !work) {
+static void box_args(ArnoldiArgs& a, const kmx_box_view* b) {
+    a.box = b ? b->arena : nullptr;
+    a.map = b ? b->map : nullptr;
+    a.nb = b ? b->nb : 0;
+    a.nslot = b ? b->nslot : 0;
+    a.f32 = b && b->f32;
+}
+
+static int arnoldi(const char* who, int64_t n, int k, double* V, const double* u, const kmx_box_view* b, double s0,
+                   double s1, const double* scale, double* z, double* h, double* work, void* stream) {
+    if (n <= 0 || k < 0 || k > KMX_ARNOLDI_MAX_K || !V || (!u && !b) || !h || !work) {
         set_error(std::string(who) + ": bad arguments (n > 0, 0 <= k <= KMX_ARNOLDI_MAX_K, device pointers)");
         return KMX_E_ARG;
     }
     ArnoldiArgs a;
     a.scale = scale;
     a.z = z;
+    box_args(a, b);
     a.n = n;
     a.k = k;
     a.G = int(std::min<long long>(AR_MAX_G, (n + AR_MIN_CHUNK - 1) / AR_MIN_CHUNK));
@@ -385,7 +441,7 @@ static int arnoldi(const char* who, int64_t n, int k, double* V, const double* u
 
 extern "C" int kmx_arnoldi_step(int64_t n, int k, double* V, const double* u, double s0, double s1, double* h,
                                 double* work, void* stream) {
-    return arnoldi("kmx_arnoldi_step", n, k, V, u, s0, s1, nullptr, nullptr, h, work, stream);
+    return arnoldi("kmx_arnoldi_step", n, k, V, u, nullptr, s0, s1, nullptr, nullptr, h, work, stream);
 }
 
 extern "C" int kmx_arnoldi_step_scaled(int64_t n, int k, double* V, const double* u, double s0, double s1,
@@ -394,5 +450,84 @@ extern "C" int kmx_arnoldi_step_scaled(int64_t n, int k, double* V, const double
         set_error("kmx_arnoldi_step_scaled: null argument");
         return KMX_E_ARG;
     }
-    return arnoldi("kmx_arnoldi_step_scaled", n, k, V, u, s0, s1, scale, z, h, work, stream);
+    return arnoldi("kmx_arnoldi_step_scaled", n, k, V, u, nullptr, s0, s1, scale, z, h, work, stream);
+}
+
+// ---- the Krylov vectors in box order
+extern "C" int kmx_plan_box_values(kmx_plan* p, int prec, int64_t* nb) {
+    if (!p || !nb) {
+        set_error("kmx_plan_box_values: null argument");
+        return KMX_E_ARG;
+    }
+    kmx_box_view b;
+    *nb = kmx_sweep_box(p, prec, &b) ? b.nb : 0;
+    return KMX_OK;
+}
+
+static int box_of(const char* who, kmx_plan* p, int prec, bool pointers, kmx_box_view* b) {
+    if (!p || !pointers) {
+        set_error(std::string(who) + ": null argument");
+        return KMX_E_ARG;
+    }
+    if (!kmx_sweep_box(p, prec, b)) {
+        set_error(std::string(who) + ": the plan has no lone separable sweep on for this precision");
+        return KMX_E_UNSUPPORTED;
+    }
+    return KMX_OK;
+}
+
+static int box_done(const char* who) {
+    const hipError_t e = hipGetLastError();
+    if (e == hipSuccess) return KMX_OK;
+    set_error(std::string(who) + ": " + hipGetErrorString(e));
+    return KMX_E_HIP;
+}
+
+static dim3 box_grid(long long nb) { return dim3(unsigned((nb + 255) / 256)); }
+
+extern "C" int kmx_plan_to_box(kmx_plan* p, int prec, const double* x, double* xb, void* stream) {
+    kmx_box_view b;
+    const int rc = box_of("kmx_plan_to_box", p, prec, x && xb, &b);
+    if (rc != KMX_OK) return rc;
+    hipLaunchKernelGGL(k_to_box, box_grid(b.nb), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), x, xb, b.map,
+                       b.nb);
+    return box_done("kmx_plan_to_box");
+}
+
+extern "C" int kmx_plan_from_box(kmx_plan* p, int prec, const double* xb, double* x, void* stream) {
+    kmx_box_view b;
+    const int rc = box_of("kmx_plan_from_box", p, prec, x && xb, &b);
+    if (rc != KMX_OK) return rc;
+    hipLaunchKernelGGL(k_from_box, box_grid(b.nb), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), xb, x, b.map,
+                       b.nb);
+    return box_done("kmx_plan_from_box");
+}
+
+extern "C" int kmx_arnoldi_box_start(kmx_plan* p, int prec, const double* v, const double* scale, double* z,
+                                     void* stream) {
+    kmx_box_view b;
+    const int rc = box_of("kmx_arnoldi_box_start", p, prec, v && scale && z, &b);
+    if (rc != KMX_OK) return rc;
+    ArnoldiArgs a;
+    std::memset(&a, 0, sizeof(a));
+    a.n = b.nb;
+    a.scale = scale;
+    a.z = z;
+    box_args(a, &b);
+    hipLaunchKernelGGL(k_box_start, box_grid(b.nb), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), a, v);
+    return box_done("kmx_arnoldi_box_start");
+}
+
+extern "C" int kmx_arnoldi_box_step(kmx_plan* p, int prec, int k, double* V, double s0, double s1,
+                                    const double* scale, double* z, double* h, double* work, void* stream) {
+    kmx_box_view b;
+    int rc = box_of("kmx_arnoldi_box_step", p, prec, V && scale && z && h && work, &b);
+    if (rc != KMX_OK) return rc;
+    if (k < 0 || k > KMX_ARNOLDI_MAX_K) {
+        set_error("kmx_arnoldi_box_step: 0 <= k <= KMX_ARNOLDI_MAX_K");
+        return KMX_E_ARG;
+    }
+    rc = kmx_sweep_box_ops(p, prec, reinterpret_cast<hipStream_t>(stream));
+    if (rc != KMX_OK) return rc;
+    return arnoldi("kmx_arnoldi_box_step", b.nb, k, V, nullptr, &b, s0, s1, scale, z, h, work, stream);
 }

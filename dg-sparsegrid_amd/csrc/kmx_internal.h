@@ -187,5 +187,19 @@ int kmx_sweep_batch_apply(const kmx_sweep_batch* sb, int slot, const kmx::BatchI
 int kmx_sweep_batch_rk3(kmx_sweep_batch* sb, int slot, double* const* fs, const double* dts, int nsteps,
                         hipStream_t s);
 void kmx_sweep_batch_free(kmx_sweep_batch* sb);
+// The boxes of a plan whose forward apply at this precision is a lone separable sweep
+// (false: it is not, or nothing but its sweep may run it): x's box copy at `arena`, op q's
+// sums at arena + (1 + q) nb, FP32 or FP64 values; map[i]: the element-order place of box
+// value i, -1 where the cell is absent (its box copy stays zero, its sums are not used).
+struct kmx_box_view {
+    const int* map;
+    void* arena;
+    long long nb;
+    int nslot;
+    bool f32;
+};
+bool kmx_sweep_box(const kmx_plan* p, int prec, kmx_box_view* out);
+// the ops alone: the slots from the box copy
+int kmx_sweep_box_ops(const kmx_plan* p, int prec, hipStream_t s);
 int kmx_sweep_batch_phases(const kmx_sweep_batch* sb);
 bool kmx_sweep_batch_has16(const kmx_sweep_batch* sb);  // every op separable with BF16 values

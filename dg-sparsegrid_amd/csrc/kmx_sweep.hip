@@ -2476,6 +2476,32 @@ static void launch_sep_phase(const kmx_sweep_batch* sb, const kmx_sweep_batch::P
     else hipLaunchKernelGGL((k_sep_batch<float, bf16_bits>), grid, block, 0, s, sb->d_ops, wgop, rc);
 }
 
+static int box_slot(const kmx_plan* p, int prec) {  // -1: not this path
+    if (!p->sw || !p->sw->separable || !p->sw->self) return -1;
+    const int slot = prec == KMX_PREC_FP64 ? 0 : prec == KMX_PREC_FP32 ? 1 : prec == KMX_PREC_BF16 ? 2 : -1;
+    if (slot < 0 || (slot < 2 && !p->var[slot].sweep) || (slot == 2 && !kmx_sweep_bf16_ok(p))) return -1;
+    if (p->sw->stale || (slot == 0 && !p->sw->fp64) || !p->sw->d_arena[slot ? 1 : 0]) return -1;
+    return slot;
+}
+
+bool kmx_sweep_box(const kmx_plan* p, int prec, kmx_box_view* out) {
+    const int slot = box_slot(p, prec);
+    if (slot < 0) return false;
+    const kmx_sweep_batch* sb = p->sw->self;
+    if (sb->njobs != 1 || (slot == 1 && !sb->has32) || (slot == 2 && !sb->has16)) return false;
+    for (const auto& P : sb->phases)
+        if (P.nwg > 0 && !P.sep_only) return false;
+    *out = kmx_box_view{p->sw->d_ymap, p->sw->d_arena[slot ? 1 : 0], p->sw->nb, int(p->sw->desc.size()), slot > 0};
+    return true;
+}
+
+int kmx_sweep_box_ops(const kmx_plan* p, int prec, hipStream_t s) {
+    const int slot = box_slot(p, prec);
+    for (const auto& P : p->sw->self->phases)
+        if (P.nwg > 0) launch_sep_phase(p->sw->self, P, slot, s);
+    return KMX_OK;
+}
+
 int kmx_sweep_batch_apply(const kmx_sweep_batch* sb, int slot, const BatchIO& io, hipStream_t s) {
     for (const kmx_plan* p : sb->members)
         if (p->sw && p->sw->stale) {

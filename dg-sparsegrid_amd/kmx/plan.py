@@ -171,6 +171,41 @@ class Plan:
         check(lib().kmx_plan_diagonal(self.handle, _ptr(out) if self.dof else None, _stream(stream)))
         return out
 
+    def box_values(self, prec="fp64"):
+        """Values of a vector in the sweep's order (kmx_plan_box_values), 0 without one on."""
+        nb = C.c_int64()
+        check(lib().kmx_plan_box_values(self.handle, _prec(prec), C.byref(nb)))
+        return nb.value
+
+    def to_box(self, x, xb, prec="fp64", stream=None):
+        self._check_len(x, x)
+        if xb.numel() != self.box_values(prec):
+            raise ValueError("to_box: xb must have box_values entries")
+        check(lib().kmx_plan_to_box(self.handle, _prec(prec), _ptr(x), _ptr(xb), _stream(stream)))
+        return xb
+
+    def from_box(self, xb, x, prec="fp64", stream=None):
+        self._check_len(x, x)
+        if xb.numel() != self.box_values(prec):
+            raise ValueError("from_box: xb must have box_values entries")
+        check(lib().kmx_plan_from_box(self.handle, _prec(prec), _ptr(xb), _ptr(x), _stream(stream)))
+        return x
+
+    def arnoldi_box_start(self, v, scale, z, prec="fp64", stream=None):
+        if {v.numel(), scale.numel(), z.numel()} != {self.box_values(prec)}:
+            raise ValueError("arnoldi_box_start: vectors must have box_values entries")
+        check(lib().kmx_arnoldi_box_start(self.handle, _prec(prec), _ptr(v), _ptr(scale), _ptr(z), _stream(stream)))
+
+    def arnoldi_box_step(self, k, V, s0, s1, scale, z, h, work, prec="fp64", stream=None):
+        """One scaled Arnoldi step on box-order vectors (kmx_arnoldi_box_step)."""
+        nb = self.box_values(prec)
+        if V.dim() != 2 or V.shape[1] != nb or V.shape[0] < k + 2 or {scale.numel(), z.numel()} != {nb}:
+            raise ValueError("arnoldi_box_step: V must be a (>= k+2, box_values) tensor, scale and z its rows' size")
+        if h.numel() < k + 2 or work.numel() < _lib.arnoldi_work(nb):
+            raise ValueError("arnoldi_box_step: h or work too small")
+        check(lib().kmx_arnoldi_box_step(self.handle, _prec(prec), int(k), _ptr(V), float(s0), float(s1),
+                                         _ptr(scale), _ptr(z), _ptr(h), _ptr(work), _stream(stream)))
+
     def apply_host(self, x, prec="fp64"):
         """numpy in, numpy out (copies through the library's staging buffers)."""
         x = np.ascontiguousarray(np.asarray(x, dtype=np.float64))

@@ -267,6 +267,21 @@ int kmx_arnoldi_step(int64_t n, int k, double* V, const double* u, double s0, do
 int kmx_arnoldi_step_scaled(int64_t n, int k, double* V, const double* u, double s0, double s1, const double* scale,
                             double* z, double* h, double* work, void* stream);
 
+/* The scaled step of a plan whose applies at `prec` run on its separable dimension sweep, on
+ * vectors in the sweep's own order (boxes of level tuples): kmx_plan_box_values gives their
+ * length nb (0: the plan has no such sweep on for prec; the calls below then return
+ * KMX_E_UNSUPPORTED), kmx_plan_to_box / _from_box reorder (absent cells zero / left out).
+ * V, scale, z: rows of nb values; work: KMX_ARNOLDI_WORK(nb).  kmx_arnoldi_box_start sets z =
+ * S v and the plan's copy of it; the steps that follow on one stream, with no apply of the
+ * plan between them, form A z themselves and leave z and its copy for the next: four launches
+ * a step instead of an apply's three and the step's three. */
+int kmx_plan_box_values(kmx_plan* plan, int prec, int64_t* nb);
+int kmx_plan_to_box(kmx_plan* plan, int prec, const double* x, double* xb, void* stream);
+int kmx_plan_from_box(kmx_plan* plan, int prec, const double* xb, double* x, void* stream);
+int kmx_arnoldi_box_start(kmx_plan* plan, int prec, const double* v, const double* scale, double* z, void* stream);
+int kmx_arnoldi_box_step(kmx_plan* plan, int prec, int k, double* V, double s0, double s1, const double* scale,
+                         double* z, double* h, double* work, void* stream);
+
 /* Y = kron(A1,...,Ak) X for k = 1..KMX_KRON_MAX_FACTORS (kron_multd.m:30-42,
  * Kronmult/kronmult{k}.m; k > 6 as kron_multd.m:43-86's recursion).
  * A[i]: DEVICE pointer, column-major nrow[i] x ncol[i] (rectangular allowed);

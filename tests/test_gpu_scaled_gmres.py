@@ -104,3 +104,89 @@ def test_backward_euler_against_a_dense_solve(kmx_gpu, pde, nd, lev, deg, factor
         bound = 2e-12 * np.linalg.norm(f0) / np.linalg.svd(M, compute_uv=False)[-1]
         assert np.linalg.norm(f1.cpu().numpy() - ref) <= bound
         TS._SOLVERS.pop(plan)  # (a captured product keeps the scales it was captured with)
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32", "bf16"])
+@pytest.mark.parametrize("nd,lev,deg,adapted", [(2, 4, 3, False), (6, 2, 2, False), (3, 3, 3, True), (4, 3, 2, False)])
+def test_box_steps_are_the_steps_in_another_order(kmx_gpu, prec, nd, lev, deg, adapted):
+    """Steps on vectors in the sweep's order against the apply and the scaled step in element
+    order: the same sums in another order.  A chunk run twice gives the same bits."""
+    import torch
+    from kmx import _lib
+    from kmx.plan import arnoldi_step
+
+    pde = K.diffusion_nd(nd, lev + 2 if adapted else lev)
+    tab = G.hash_table_sparse_nd([lev] * nd, lev, "SG")
+    if adapted:
+        tab = G.refine_random(tab, lev + 2, 0.5, np.random.default_rng(1))
+    mats = K.get_coeff_mats(pde, deg)
+    plan = kmx_gpu.Plan(mats, tab.idx1d, deg, None, None, index_base=1, fp32=True, level_blocks=True,
+                        identity=[[d != t for d in range(nd)] for t in range(nd)])
+    assert plan.box_values("fp64") == 0  # not switched on
+    for p in ("fp64", "fp32"):
+        plan.set_sweep(p, True)
+    nb, n, steps = plan.box_values(prec), plan.dof, 5
+    assert nb >= n and (nb > n) == adapted
+    gen = torch.Generator().manual_seed(nd)
+    v = torch.randn(n, dtype=torch.float64, generator=gen).cuda()
+    v /= torch.linalg.vector_norm(v)
+    S = torch.rand(n, dtype=torch.float64, generator=gen).cuda() + 0.5
+    back = torch.empty_like(v)
+    vb = plan.to_box(v, torch.full((nb,), 7.0, dtype=torch.float64, device="cuda"), prec)
+    assert torch.equal(plan.from_box(vb, back, prec), v) and int((vb == 0).sum()) == nb - n
+    dt = 20 * pde.set_dt(pde, 0.01)
+    V = torch.zeros((steps + 1, n), dtype=torch.float64, device="cuda")
+    V[0] = v
+    h, u, z = torch.zeros((steps, steps + 2), dtype=torch.float64, device="cuda"), torch.empty_like(v), S * v
+    work = torch.empty(_lib.arnoldi_work(n), dtype=torch.float64, device="cuda")
+    for k in range(steps):
+        plan.apply(z, u, prec=prec)
+        arnoldi_step(n, k, V, u, 1.0, -dt, h[k], work, scale=S, z=z)
+    Vb = torch.zeros((steps + 1, nb), dtype=torch.float64, device="cuda")
+    Vb[0] = vb
+    Sb, zb, hb = plan.to_box(S, torch.empty_like(vb), prec), torch.empty_like(vb), torch.zeros_like(h)
+    workb = torch.empty(_lib.arnoldi_work(nb), dtype=torch.float64, device="cuda")
+    runs = []
+    for _ in range(2):
+        plan.arnoldi_box_start(Vb[0], Sb, zb, prec)
+        for k in range(steps):
+            plan.arnoldi_box_step(k, Vb, 1.0, -dt, Sb, zb, hb[k], workb, prec)
+        runs.append((Vb.clone(), hb.clone()))
+        plan.apply(v, u, prec=prec)  # the boxes hold another vector now
+    assert torch.equal(runs[0][0], runs[1][0]) and torch.equal(runs[0][1], runs[1][1])
+    # dots in another order, n eps, through 5 steps; a last bit of z may round the other way
+    # in the product's precision, whose unit the later steps carry on
+    tol = {"fp64": 1e-11, "fp32": 1e-5, "bf16": 5e-2}[prec]
+    assert float((hb - h).abs().max()) <= tol * float(h.abs().max())
+    for k in range(steps + 1):
+        d = plan.from_box(Vb[k], back, prec) - V[k]
+        assert float(d.abs().max()) <= tol * max(1.0, float(h.abs().max()))
+        assert int((Vb[k] == 0).sum()) >= nb - n
+    plan.set_sweep("fp32", False)
+    if prec == "fp32":
+        with pytest.raises(ValueError):
+            plan.to_box(v, vb, prec)
+
+
+def test_backward_euler_follows_the_sweep_switch(kmx_gpu):
+    """The solver kept for a plan is one of its present path: switched on, off and on again."""
+    import torch
+    from kmx import timestep as TS
+
+    pde = K.diffusion_nd(3, 4)
+    tab = G.hash_table_sparse_nd([4] * 3, 4, "SG")
+    mats = K.get_coeff_mats(pde, 2)
+    plan = kmx_gpu.Plan(mats, tab.idx1d, 2, None, None, index_base=1, fp32=True, level_blocks=True,
+                        identity=[[d != t for d in range(3)] for t in range(3)])
+    f0 = np.random.default_rng(3).standard_normal(plan.dof)
+    dt = 100 * pde.set_dt(pde, 0.01)
+    M = np.eye(plan.dof) - dt * O.build_A(O.ApplyInputs(mats, tab.idx1d, 2))
+    ref = np.linalg.solve(M, f0)
+    bound = 2e-12 * np.linalg.norm(f0) / np.linalg.svd(M, compute_uv=False)[-1]
+    for on in (True, False, True):
+        for p in ("fp64", "fp32"):
+            plan.set_sweep(p, on)
+        for _ in range(2):
+            f1, hist, _ = TS.backward_euler(plan, torch.from_numpy(f0).cuda(), dt, tol=1e-12)
+            assert hist[-1] <= 1e-12
+            assert np.linalg.norm(f1.cpu().numpy() - ref) <= bound
