@@ -548,7 +548,7 @@ bool product_masks(const kmx_plan* p, const std::vector<int>& idx, const std::ve
     if (bits > 512e6) return false;
     typedef unsigned long long word;
     // (3D lev 7, 1,903,000 pairs: the plan took 5.0 ms without this check, 8.7 with it in one
-    // thread and a bit at a time, under 5.5 so)
+    // thread and a bit at a time, 5.5 to 6.7 so)
     const bool many = rp[size_t(N)] > 100000;
     std::atomic<bool> product{true};
     // the rows as bit sets: a word stays in a register while consecutive columns lie in it

@@ -295,7 +295,7 @@ static void build_lists(kmx_realspace* r, int k, const double* meval, const std:
             on[size_t(t) * blocks + b] = any;
         }
     const int nodes = int(cptr.size()) - 1;
-    if (double(col.size()) * tiles > 1e8) return;
+    if (double(col.size()) * tiles > 2e7) return;  // (160 MB of lists at most)
     std::vector<int> ptr, lcol, lx;
     for (int q = 0; q < nodes; ++q)
         for (int t = 0; t < tiles; ++t) {
