@@ -8,13 +8,7 @@ LaunchFn pick_f64(int D, int deg, int nt, int lds) { return pick_impl<double>(D,
 LaunchFn pick_split_f64(int D, int deg, int nt, bool lds) { return pick_split_impl<double>(D, deg, nt, lds); }
 
 hipError_t launch_generic_f64(const KArgs<double>& a, int D, int deg, int nrows, size_t smem, hipStream_t s) {
-    if (smem > 65536) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_apply_generic<double>),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, int(smem));
-        if (e != hipSuccess) return e;
-    }
-    hipLaunchKernelGGL(k_apply_generic<double>, dim3(nrows), dim3(256), smem, s, a, D, deg);
-    return hipGetLastError();
+    return launch_generic<double>(a, D, deg, nrows, smem, s);
 }
 
 hipError_t launch_batch_f64(const KArgs<double>* args, const int2* items, int nitems, const int* shape,

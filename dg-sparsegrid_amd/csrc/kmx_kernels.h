@@ -580,6 +580,160 @@ __global__ void __launch_bounds__(256) k_apply_generic(KArgs<T> a, int D, int DE
     for (int e = tid; e < B; e += 256) a.y[(long long)row * B + e] = double(acc[e]);
 }
 
+// Blocks of up to 256 values: a wave per pair instead of the workgroup, so that nothing
+// waits at a barrier between the dimensions.  k_apply_generic passes some seven barriers
+// a term and pair, pair after pair (4D lev 3 deg 3, 63 rows, 3,953 pairs, 4 terms: 608 us);
+// here a row's 8 or 16 waves take every 8th or 16th pair, the pair's 1D blocks and two
+// copies of its values in LDS, its sums in registers (at most four values a lane), and
+// add in wave order at the end (35 us; lev 4 1.85 ms -> 91 us, 3D lev 4 deg 5 714 -> 43).
+// Bound by the latency of the chain of contractions; larger blocks keep the whole workgroup busy on one.
+constexpr int AW_VALUES = 4;  // values of a lane
+template <typename T, int D>
+__global__ void __launch_bounds__(1024) k_apply_waves(KArgs<T> a, int DEG) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ long long off[KMX_MAX_TERMS * D];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int waves = int(blockDim.x) >> 6, dd = DEG * DEG, nm = D * dd;
+    int B = 1;
+#pragma unroll
+    for (int k = 0; k < D; ++k) B *= DEG;
+    T* v = reinterpret_cast<T*>(smem) + wave * (2 * B + nm);
+    T* w = v + B;
+    T* m = w + B;
+    for (int i = tid; i < a.nterms * D; i += int(blockDim.x)) off[i] = a.off[i];
+    const int row = a.row_order[blockIdx.x];
+    int I[D];
+#pragma unroll
+    for (int k = 0; k < D; ++k) I[k] = a.idx1d[(long long)row * D + k];
+    // per value: where its fibre along dimension k starts, and its row of the block
+    int from[AW_VALUES][D], mrow[AW_VALUES][D];
+#pragma unroll
+    for (int u = 0; u < AW_VALUES; ++u) {
+        const int e = lane + 64 * u;
+        int stride = 1;
+#pragma unroll
+        for (int k = D - 1; k >= 0; --k) {
+            const int ai = (e / stride) % DEG;
+            from[u][k] = e - ai * stride;
+            mrow[u][k] = k * dd + ai * DEG;
+            stride *= DEG;
+        }
+    }
+    // per block entry this lane fetches (two at most: D deg^2 <= 128 here): dimension and place
+    int mk[2];
+    long long mat[2];
+    bool mok[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int i = lane + 64 * u;
+        mok[u] = i < nm;
+        mk[u] = mok[u] ? i / dd : 0;
+        mat[u] = mok[u] ? i - mk[u] * dd : 0;
+#pragma unroll
+        for (int k = 0; k < D; ++k)
+            if (mk[u] == k) mat[u] += (long long)I[k] * a.nb[k] * dd;
+    }
+    auto settle = [] {  // this wave's LDS writes before its reads (they run in order)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    __syncthreads();
+    T acc[AW_VALUES];
+#pragma unroll
+    for (int u = 0; u < AW_VALUES; ++u) acc[u] = T(0);
+    const long long pb = a.row_ptr ? a.row_ptr[row] : 0;
+    const long long pe = a.row_ptr ? a.row_ptr[row + 1] : a.N;
+    for (long long q = pb + wave; q < pe; q += waves) {
+        const int j = a.row_ptr ? a.cols[q] : int(q);
+        T x[AW_VALUES];
+#pragma unroll
+        for (int u = 0; u < AW_VALUES; ++u) x[u] = lane + 64 * u < B ? T(a.x[(long long)j * B + lane + 64 * u]) : T(0);
+        long long at[2] = {mat[0], mat[1]};
+#pragma unroll
+        for (int k = 0; k < D; ++k) {
+            const int J = a.idx1d[(long long)j * D + k];
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                if (mk[u] == k) at[u] += J * dd;
+        }
+        for (int t = 0; t < a.nterms; ++t) {
+            T b[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) b[u] = mok[u] ? a.blk[off[t * D + mk[u]] + at[u]] : T(0);
+            settle();
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                if (mok[u]) m[lane + 64 * u] = b[u];
+#pragma unroll
+            for (int u = 0; u < AW_VALUES; ++u)
+                if (lane + 64 * u < B) v[lane + 64 * u] = x[u];
+            settle();
+            int stride = 1;
+            T out[AW_VALUES];
+#pragma unroll
+            for (int k = D - 1; k >= 0; --k) {
+                const T* vin = (D - 1 - k) % 2 ? w : v;
+                T* vout = (D - 1 - k) % 2 ? v : w;
+#pragma unroll
+                for (int u = 0; u < AW_VALUES; ++u)
+                    if (lane + 64 * u < B) {
+                        const T* f = vin + from[u][k];
+                        const T* r = m + mrow[u][k];
+                        T s = r[0] * f[0];
+                        for (int c = 1; c < DEG; ++c) s = madd(r[c], f[c * stride], s);
+                        out[u] = s;
+                        if (k > 0) vout[lane + 64 * u] = s;
+                    }
+                settle();
+                stride *= DEG;
+            }
+            const T s = a.scale[t];
+#pragma unroll
+            for (int u = 0; u < AW_VALUES; ++u)
+                if (lane + 64 * u < B) acc[u] = madd(s, out[u], acc[u]);
+        }
+    }
+    __syncthreads();
+    T* sums = reinterpret_cast<T*>(smem);
+#pragma unroll
+    for (int u = 0; u < AW_VALUES; ++u)
+        if (lane + 64 * u < B) sums[wave * B + lane + 64 * u] = acc[u];
+    __syncthreads();
+    for (int e = tid; e < B; e += int(blockDim.x)) {
+        T s = sums[e];
+        for (int q = 1; q < waves; ++q) s += sums[q * B + e];
+        a.y[(long long)row * B + e] = double(s);
+    }
+}
+
+template <typename T, int D>
+hipError_t launch_waves(const KArgs<T>& a, int deg, int B, int nrows, hipStream_t s) {
+    const int waves = B <= 128 ? 16 : 8;  // at most 42 KB of LDS (3D deg 5 in FP64)
+    const size_t smem = size_t(waves) * (2 * B + D * deg * deg) * sizeof(T);
+    hipLaunchKernelGGL((k_apply_waves<T, D>), dim3(nrows), dim3(64 * waves), smem, s, a, deg);
+    return hipGetLastError();
+}
+
+// the generic kernels: a wave per pair where a block's values fit one
+template <typename T>
+hipError_t launch_generic(const KArgs<T>& a, int D, int deg, int nrows, size_t smem, hipStream_t s) {
+    int B = 1;
+    for (int k = 0; k < D; ++k) B *= deg;
+    if (B <= 64 * AW_VALUES && D * deg * deg <= 128) switch (D) {
+            case 2: return launch_waves<T, 2>(a, deg, B, nrows, s);
+            case 3: return launch_waves<T, 3>(a, deg, B, nrows, s);
+            case 4: return launch_waves<T, 4>(a, deg, B, nrows, s);
+            case 5: return launch_waves<T, 5>(a, deg, B, nrows, s);
+        }
+    if (smem > 65536) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_apply_generic<T>),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, int(smem));
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(k_apply_generic<T>, dim3(nrows), dim3(256), smem, s, a, D, deg);
+    return hipGetLastError();
+}
+
 // ---------------------------------------------------------------- launchers
 using LaunchFn = hipError_t (*)(const void* args, int nrows, size_t smem, hipStream_t s);
 
