@@ -60,6 +60,18 @@ static bool strip_fits(const kmx_plan* p, size_t elem, int mode = 1) {
     return strip_bytes(p, elem, mode) <= lds_limit();
 }
 
+// Whether a row's strips go to LDS when nothing was timed.  A lane takes a pair, so rows of
+// up to a workgroup's 256 pairs read most strip entries once or not at all, and staging
+// costs a round of loads, a barrier and occupancy: from L2 they take, FP64, 7.7 against
+// 10.7 us (3D lev 3, 6 terms), 16.0 / 18.7 (lev 5), 4.8 / 8.2 (1D lev 9), 42 / 49 (6D lev 3),
+// and FP32 26.5 / 35.8.  Longer rows are level either way (2D lev 7 adapted 34, 3D lev 6 28).
+// Four lanes a pair of 64 FP64 values read each 16-entry block four times: those stay in LDS
+// (3D lev 4 deg 4, rows of 104: 12.4 / 15.2).
+static int default_strip(const kmx_plan* p, size_t elem) {
+    const bool shortrows = p->P <= 256ll * p->N && !(elem == sizeof(double) && p->D == 3 && p->deg == 4);
+    return !shortrows && strip_fits(p, elem) ? 1 : 0;
+}
+
 // One launch of the pair-by-pair kernel family with an explicit variant.
 static int launch_variant(kmx_plan* p, bool transpose, const double* x, double* y, int prec, kmx_variant v,
                           hipStream_t s) {
@@ -73,7 +85,7 @@ static int launch_variant(kmx_plan* p, bool transpose, const double* x, double* 
             return KMX_E_ARG;
         }
         // LDS mode: 0 none, 1 every strip, 2 every strip but dim 1's (-1: 1 when it fits)
-        int mode = v.lds < 0 ? (strip_fits(p, elem) ? 1 : 0) : v.lds;
+        int mode = v.lds < 0 ? default_strip(p, elem) : v.lds;
         if (mode && !strip_fits(p, elem, mode)) mode = 0;
         if (mode == 2 && (v.kind == 1 || D < 2)) mode = 1;
         if (mode == 1 && !strip_fits(p, elem, 1)) mode = 0;
@@ -350,7 +362,7 @@ extern "C" int kmx_plan_get_variant(const kmx_plan* p, int prec, int* nt, int* l
     }
     const kmx_variant v = p->var[prec_slot(prec)];
     const size_t elem = prec == KMX_PREC_FP64 ? sizeof(double) : sizeof(float);
-    int mode = v.lds < 0 ? (strip_fits(p, elem) ? 1 : 0) : v.lds;
+    int mode = v.lds < 0 ? default_strip(p, elem) : v.lds;
     if (mode && !strip_fits(p, elem, mode)) mode = 0;
     if (mode == 2 && (v.kind == 1 || p->D < 2)) mode = strip_fits(p, elem, 1) ? 1 : 0;
     if (nt) *nt = (v.nt > 0 ? v.nt : 256) * (v.kind == 1 ? -1 : 1);
