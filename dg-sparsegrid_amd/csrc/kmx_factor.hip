@@ -818,7 +818,13 @@ void kmx_factor_build(kmx_plan* p, const std::vector<int>& idx, const std::vecto
     // against 27, lev 7: 66 against 135; 6D lev 4 deg 2: 41 against 77).
     const double lanes = double((G + 63) / 64) * 64.0, rlanes = double((N + 63) / 64) * 64.0;
     const double fac_fma = T * (double(contr) * lanes + double(NV) * rlanes) * unit;
-    if (!env && 18e-6 + fac_fma / (D == 2 ? 6e12 : 7e12) > pair_fma / (D == 2 ? 4.7e12 : 1.1e13)) return;
+    // 3D deg 4, whose 16-entry blocks are cheaper here and whose pairs are split over four
+    // lanes there: 19 us and 1e13 against 11 us and 1.2e13 (lev 5, 6 terms: 28 against 51; lev
+    // 6, 3 terms: 41 / 80; lev 4 adapted, 6 terms: 25 / 35; lev 4, 6 terms: 23 / 20.5).
+    const bool slower = D == 3 && p->deg == 4
+                            ? 19e-6 + fac_fma / 1e13 > 11e-6 + pair_fma / 1.2e13
+                            : 18e-6 + fac_fma / (D == 2 ? 6e12 : 7e12) > pair_fma / (D == 2 ? 4.7e12 : 1.1e13);
+    if (!env && slower) return;
     const double w_elems = double(T) * NV * L.WN * double(G);
     if (w_elems * 8.0 > 1024e6) return;
     auto f = new kmx_factor();
