@@ -55,10 +55,13 @@ struct StageArgs {
     const int* lx;
     int ptiles;
     // A zero of Meval times an infinity or a NaN is a NaN everywhere: a stage that stores a
-    // value that is not finite sets *flag to the call's number, and the next ones take
-    // every child.  (A replayed graph finds its own number of a run before: the same
-    // sums, only more of them.)
+    // value that is not finite sets its own *flag to the call's number, and the next one,
+    // which reads it as *before, takes every child (and stores such a value itself, so it
+    // tells the one after).  No launch reads what it writes: the waves of a workgroup have
+    // to agree on the list, or they pass different numbers of barriers.  (A replayed graph
+    // finds its own number of a run before: the same sums, only more of them.)
     int* flag;
+    const int* before;  // (last dimension: null, it looks at the coefficients themselves)
     int call;
 };
 
@@ -183,6 +186,7 @@ __global__ void __launch_bounds__(256, 2) k_rs_last(StageArgs a) {
 // (its row tiles, which read the same values of Z_{k+1}) share an XCD's L2.
 __global__ void __launch_bounds__(256, 2) k_rs_mode(StageArgs a) {
     __shared__ double lds[mma64_lds<64, 16>()];
+    __shared__ int before;
     const int per = a.xcd ? a.mt * ((a.nt + 7) / 8) * 8 : a.mt * a.nt;
     const int item = int(blockIdx.x) / per, t = int(blockIdx.x) - item * per;
     if (item >= a.items) return;
@@ -199,7 +203,13 @@ __global__ void __launch_bounds__(256, 2) k_rs_mode(StageArgs a) {
     const int i0 = 64 * rt;
     const long long j0 = 64LL * ct;
     const int c0 = a.cptr[q];
-    const Children ch = children(a, q, rt, !a.lptr || *a.flag == a.call, nullptr);
+    bool every = !a.lptr;
+    if (!every) {  // one read for the workgroup, whatever another stream's call writes meanwhile
+        if (threadIdx.x == 0) before = *a.before;
+        __syncthreads();
+        every = before == a.call;
+    }
+    const Children ch = children(a, q, rt, every, nullptr);
     const int K = ch.n * a.deg;
     const int n = int(min(64LL, a.R - j0));
     auto column = [&](int k) {
@@ -258,7 +268,7 @@ struct kmx_realspace {
     };
     Stage stage[KMX_MAX_DIM];
     int* d_row = nullptr;                   // elements in prefix order
-    int* d_flag = nullptr;
+    int* d_flag = nullptr;                  // one per stage
     unsigned calls = 0;
     double* d_buf[2] = {nullptr, nullptr};  // Z_d, Z_{d-1}, ... in turn
 };
@@ -418,7 +428,7 @@ extern "C" int kmx_realspace_create(int ndim, int deg, int num_elem, const int* 
             }
         }
         up(order, r->d_row);
-        up(std::vector<int>(1, 0), r->d_flag);
+        up(std::vector<int>(size_t(ndim), 0), r->d_flag);
         for (int q = 0; q < 2; ++q)
             if (hipMalloc(&r->d_buf[q], size_t(need[q]) * sizeof(double)) != hipSuccess) throw std::bad_alloc();
         *out = r;
@@ -461,7 +471,8 @@ extern "C" int kmx_realspace_apply(kmx_realspace* r, const double* f_w, double* 
         a.lcol = st.d_list ? st.d_list + st.o_col : nullptr;
         a.lx = st.d_list ? st.d_list + st.o_x : nullptr;
         a.ptiles = (r->npts[k] + 63) / 64;
-        a.flag = r->d_flag;
+        a.flag = r->d_flag + k;
+        a.before = k + 1 < D ? r->d_flag + k + 1 : nullptr;
         a.call = call;
         a.R = R;
         a.M = r->npts[k];

@@ -182,3 +182,51 @@ def test_realspace_children_by_tile(kmx_gpu, nd, lev, deg, npts):
         fd.copy_(torch.from_numpy(f))
         graph.replay()
         assert torch.equal(out, got)
+
+
+@pytest.mark.parametrize("nd,lev,deg", [(2, 5, 3), (3, 4, 2)])
+@pytest.mark.parametrize("dim", [0, 1])
+@pytest.mark.parametrize("value", [1e308, np.inf, np.nan])
+def test_realspace_values_lost_in_a_later_stage(kmx_gpu, nd, lev, deg, dim, value):
+    """Finite coefficients and, at a few points of one dimension, evaluation values that
+    overflow the sum (1e308 times sums over 1e3) or are not finite themselves: nothing is
+    finite at those points, and every other point has the bits that it has without them,
+    call after call, eager and replayed."""
+    import torch
+    from kmx import coeffs as K
+    from kmx import grid as G
+
+    idx = G.hash_table_sparse_nd([lev] * nd, lev, "SG").idx1d
+    rng = np.random.default_rng(nd * 10 + dim)
+    # the zeros of real evaluation matrices, 130 points (three tiles), positive values
+    meval = []
+    for _ in range(nd):
+        m = K.matrix_plot_D(deg, lev, -1.0, 1.0)[0]
+        m = m[np.arange(130) * m.shape[0] // 130]
+        meval.append(np.where(m == 0.0, 0.0, rng.uniform(1.0, 2.0, m.shape)))
+    f = torch.from_numpy(rng.uniform(1e3, 2e3, len(idx) * deg ** nd)).cuda()
+    want = kmx_gpu.RealSpace(meval, idx, deg).apply(f)
+    assert bool(torch.isfinite(want).all())
+    points = [70, 129]  # in the second and the third tile
+    hit = [m.copy() for m in meval]
+    hit[dim][points] = np.where(hit[dim][points] == 0.0, 0.0, value)
+    rs = kmx_gpu.RealSpace(hit, idx, deg)
+    shape = [130] * nd
+    keep = [i for i in range(130) if i not in points]
+
+    def check(out):
+        v = out.view(shape).movedim(dim, 0)
+        assert not bool(torch.isfinite(v[points]).any())
+        assert torch.equal(v[keep], want.view(shape).movedim(dim, 0)[keep])
+
+    for _ in range(8):
+        check(rs.apply(f))
+    out = torch.empty_like(want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        rs.apply(f, out)
+    for _ in range(3):
+        graph.replay()
+        check(out)
+        out.zero_()
+        check(rs.apply(f))
