@@ -354,6 +354,28 @@ extern "C" int kmx_plan_get_sweep(const kmx_plan* p, int prec, int* available, i
     return KMX_OK;
 }
 
+extern "C" int kmx_plan_replay_state(const kmx_plan* p, int prec, uint64_t* state) {
+    if (!p || !state || (prec != KMX_PREC_FP64 && prec != KMX_PREC_FP32 && prec != KMX_PREC_BF16)) {
+        set_error("kmx_plan_replay_state: bad arguments");
+        return KMX_E_ARG;
+    }
+    uint64_t h = 14695981039346656037ull;  // FNV-1a over 64-bit words
+    auto mix = [&](uint64_t v) { h = (h ^ v) * 1099511628211ull; };
+    const bool sweep = p->sw && (prec == KMX_PREC_BF16 || p->var[prec_slot(prec)].sweep);
+    mix(sweep ? 2 : 1);
+    if (sweep && kmx_sweep_separable(p)) {
+        mix(kmx_sweep_storage(p));
+    } else {
+        for (int t = 0; t < p->T; ++t) {
+            uint64_t bits;
+            std::memcpy(&bits, &p->scale[t], sizeof bits);
+            mix(bits);
+        }
+    }
+    *state = h;
+    return KMX_OK;
+}
+
 extern "C" int kmx_plan_get_variant(const kmx_plan* p, int prec, int* nt, int* lds) {
     // (the lane-split kind is reported through kmx_plan_get_variant's nt sign: negative = split)
     if (!p || (prec != KMX_PREC_FP64 && prec != KMX_PREC_FP32)) {

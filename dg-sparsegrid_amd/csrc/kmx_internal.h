@@ -155,6 +155,9 @@ int kmx_sweep_apply(kmx_plan* p, int slot, const double* x, double* y, hipStream
 void kmx_sweep_free(kmx_plan* p);
 double kmx_sweep_flops(const kmx_plan* p);
 bool kmx_sweep_separable(const kmx_plan* p);  // has a sweep of the separable form
+// What the launches of the plan's separable sweep read now, by number: storage rebuilt,
+// identity factors replaced
+unsigned long long kmx_sweep_storage(const kmx_plan* p);
 // whether FP64 applies may use the plan's sweep (a separable sweep whose undeclared
 // identity factors are exact to 4 ulps, or a general sweep)
 bool kmx_sweep_fp64_ok(const kmx_plan* p);

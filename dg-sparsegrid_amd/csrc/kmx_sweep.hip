@@ -2238,6 +2238,11 @@ void kmx_sweep_free(kmx_plan* p) {
 
 bool kmx_sweep_separable(const kmx_plan* p) { return p->sw && p->sw->separable; }
 
+unsigned long long kmx_sweep_storage(const kmx_plan* p) {
+    const kmx_sweep* sw = p->sw;  // (every rebuild retires one launch table)
+    return (unsigned long long)sw->retired_batches.size() << 2 | (sw->stale ? 2 : 0) | (sw->fp64 ? 1 : 0);
+}
+
 double kmx_sweep_flops(const kmx_plan* p) { return p->sw ? double(p->sw->flops) : 0.0; }
 
 bool kmx_sweep_fp64_ok(const kmx_plan* p) { return p->sw && (!p->sw->separable || p->sw->fp64); }

@@ -241,6 +241,13 @@ class Plan:
         check(lib().kmx_plan_get_sweep(self.handle, _prec(prec), C.byref(av), C.byref(ac), C.byref(fl)))
         return {"available": bool(av.value), "active": bool(ac.value), "flops": fl.value}
 
+    def replay_state(self, prec="fp64"):
+        """A number that stays the same while a graph that captured an apply at prec replays
+        the operator that apply runs (kmx_plan_replay_state)."""
+        state = C.c_uint64()
+        check(lib().kmx_plan_replay_state(self.handle, _prec(prec), C.byref(state)))
+        return state.value
+
     def sweep_info(self):
         """The dimension sweep's form and storage (kmx_plan_sweep_info)."""
         info = _lib.SweepInfo()

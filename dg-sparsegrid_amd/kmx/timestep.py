@@ -267,6 +267,7 @@ class DeviceGMRES:
         self.hhost = torch.zeros((m, m + 2), dtype=torch.float64).pin_memory()
         self.ystage = torch.zeros(m, dtype=torch.float64).pin_memory()  # least-squares solution, host side
         self.graphs = [None] * (m // self.chunk)
+        self.state = None
         self.scale = torch.ones(nv, dtype=torch.float64, device=device) if scaled else None
         self.z = torch.empty_like(self.scale) if scaled else None
 
@@ -304,6 +305,14 @@ class DeviceGMRES:
             torch.cuda.synchronize()
             self.graphs[ci] = g
         return self.graphs[ci]
+
+    def captured_for(self, state):
+        """The captured steps are of the operator that `state` stands for (any value): with
+        another one than last time they are captured again."""
+        if state != self.state and any(g is not None for g in self.graphs):
+            _torch().cuda.synchronize()  # chunks past the last solve's convergence may still run
+            self.graphs = [None] * len(self.graphs)
+        self.state = state
 
     def _converges_in_flight(self, rs, target):
         """Whether the residual estimates rs (one per step of the cycle so far),
@@ -432,7 +441,8 @@ def backward_euler(plan, f0, dt, rhs=None, tol=1e-10, inner_prec="fp32", inner_t
     apply) drives a correction solved by GMRES with `inner_prec` applies to
     relative accuracy inner_tol, until ||r|| / ||b|| <= tol.  GMRES is scaled by a power of
     the operator's diagonal 1 - dt A_ii where that is over 1 (stiff rows).  The GMRES solver
-    (its captured Arnoldi graphs) is kept per plan and step size for later steps.
+    (its captured Arnoldi graphs) is kept per plan and step size for later steps; what the
+    graphs hold of the operator (Plan.replay_state) is looked at in each step.
     Returns (f1, history of FP64 relative residuals, inner iterations)."""
     torch = _torch()
     b = f0.clone() if rhs is None else f0 + dt * rhs
@@ -453,7 +463,9 @@ def backward_euler(plan, f0, dt, rhs=None, tol=1e-10, inner_prec="fp32", inner_t
                              shift=(1.0, -float(dt)), scaled=True,
                              box=(pref, inner_prec) if boxed else None)
         cache[key] = solver
-    if hasattr(plan, "diagonal"):  # (a stand-in for a plan may have its product alone)
+    if hasattr(plan, "replay_state"):  # (a stand-in for a plan may have its product alone)
+        solver.captured_for(plan.replay_state(inner_prec))
+    if hasattr(plan, "diagonal"):
         d = plan.diagonal().mul_(-float(dt)).add_(1.0).clamp_(min=1.0).pow_(SCALE_POWER)
         solver.scale.copy_(d) if solver.box is None else plan.to_box(d, solver.scale, inner_prec)
     f = f0.clone()  # f0 is a good first guess for small dt

@@ -130,6 +130,13 @@ int kmx_plan_get_variant(const kmx_plan* plan, int prec, int* threads, int* lds_
 int kmx_plan_set_sweep(kmx_plan* plan, int prec, int on);
 int kmx_plan_get_sweep(const kmx_plan* plan, int prec, int* available, int* active, double* flops);
 
+/* What a graph that captures an apply at prec will replay, as one number: while it is the
+ * same, a replay is the operator that kmx_apply runs.  It changes with the path (sweep or
+ * pairs), with the term scales where they are launch arguments (not on a separable sweep,
+ * whose stored operator kmx_plan_set_term_scale refreshes), and with a separable sweep's
+ * storage (kmx_plan_update_term with a matrix of other zero blocks). */
+int kmx_plan_replay_state(const kmx_plan* plan, int prec, uint64_t* state);
+
 /* The separable form of the sweep (every term acts in one dimension; its other
  * factors are the identity).  A factor counts as the identity when declared so
  * (kmx_plan_desc.identity) or within 1e-11 of I entrywise; FP64 applies may use

@@ -190,3 +190,58 @@ def test_backward_euler_follows_the_sweep_switch(kmx_gpu):
             f1, hist, _ = TS.backward_euler(plan, torch.from_numpy(f0).cuda(), dt, tol=1e-12)
             assert hist[-1] <= 1e-12
             assert np.linalg.norm(f1.cpu().numpy() - ref) <= bound
+
+
+@pytest.mark.parametrize("sweep", [False, True])
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_backward_euler_follows_its_operator(kmx_gpu, sweep, prec):
+    """One kept solver through changes of the operator between its steps: term scales (launch
+    arguments of the pair kernels), a matrix of the same zero blocks and one of others (new
+    storage of a separable sweep).  Each step takes the inner steps that a plan made for that
+    operator takes, and solves its system."""
+    import torch
+    from kmx import timestep as TS
+
+    pde = K.diffusion_nd(3, 3)
+    tab = G.hash_table_sparse_nd([3] * 3, 3, "SG")
+    mats = [list(m) for m in K.get_coeff_mats(pde, 2)]
+    scales = [1.0] * 3
+    n = mats[0][0].shape[0]
+
+    def make():
+        p = kmx_gpu.Plan(mats, tab.idx1d, 2, None, None, index_base=1, fp32=True, level_blocks=sweep,
+                         identity=[[d != t for d in range(3)] for t in range(3)] if sweep else None)
+        if sweep:
+            for q in ("fp64", "fp32"):
+                p.set_sweep(q, True)
+        for t, s in enumerate(scales):
+            p.set_term_scale(t, s)
+        return p
+
+    def step(p):
+        f1, hist, inner = TS.backward_euler(p, torch.from_numpy(f0).cuda(), dt, tol=1e-12, inner_prec=prec)
+        assert hist[-1] <= 1e-12
+        A = O.build_A(O.ApplyInputs([[s * m[0]] + m[1:] for s, m in zip(scales, mats)], tab.idx1d, 2))
+        M = np.eye(p.dof) - dt * A
+        bound = 2e-12 * np.linalg.norm(f0) / np.linalg.svd(M, compute_uv=False)[-1]
+        assert np.linalg.norm(f1.cpu().numpy() - np.linalg.solve(M, f0)) <= bound
+        return inner
+
+    plan = make()
+    f0 = np.random.default_rng(5).standard_normal(plan.dof)
+    dt = 100 * pde.set_dt(pde, 0.01)
+    state = plan.replay_state(prec)
+    seen = [step(plan)]
+    assert plan.replay_state(prec) == state
+    for change in ("scales", "values", "blocks", "scales back"):
+        if change == "scales":
+            scales[:] = [0.25, 1.0, 0.5]
+        elif change == "scales back":
+            scales[:] = [1.0] * 3
+        else:
+            mats[1][1] = 0.5 * mats[1][1] if change == "values" else -40.0 * np.eye(n)
+            plan.update_term(1, 1, mats[1][1])
+        for t, s in enumerate(scales):
+            plan.set_term_scale(t, s)
+        assert step(plan) == step(make())
+    assert len(TS._SOLVERS[plan]) == 1
