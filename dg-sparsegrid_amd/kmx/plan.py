@@ -438,7 +438,8 @@ def kronmult(mats, X, stream=None, noalloc=False, Y=None):
 
 
 def gemm_vbatched(transA, transB, ms, ns, ks, alpha, As, ldas, Bs, ldbs, beta, Cs, ldcs, stream=None):
-    """Batched GEMM over device pointers (ints or tensors)."""
+    """Batched GEMM over device pointers (ints or tensors).  On a stream given it is complete
+    when it returns (the operands may belong to another one); under capture it is recorded."""
     cnt = len(ms)
 
     def arr(v):
@@ -466,6 +467,8 @@ def gemm_vbatched(transA, transB, ms, ns, ks, alpha, As, ldas, Bs, ldbs, beta, C
     check(lib().kmx_gemm_vbatched(transA.encode(), transB.encode(), arr(ms), arr(ns), arr(ks), float(alpha),
                                   parr(As), arr(ldas), parr(Bs), arr(ldbs), float(beta), parr(Cs), arr(ldcs), cnt,
                                   _stream(stream)))
+    if stream is not None and cnt and not _torch().cuda.is_current_stream_capturing():
+        check(lib().kmx_sync(_stream(stream)))
 
 
 def kronmult_batch_plan(nrow, ncol, nvec):

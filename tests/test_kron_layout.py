@@ -122,3 +122,33 @@ def test_packed_descriptors_give_the_same_bits(kmx_gpu, ta, tb, beta, count):
     kmx_gpu.gemm_vbatched(ta, tb, ms, ns, ks, 1.5, [wide] + A[1:], lda, B, ldb, beta, other, ldc)
     for i in range(1, count):
         assert torch.equal(other[i], one[i]), (i, shapes[i])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("count", [1, 100, 641])
+def test_gemm_on_a_stream_given_is_complete_on_return(kmx_gpu, count):
+    """Behind work that keeps that stream busy: C may be read, and A and B given back, on the
+    current stream as soon as the call returns.  Recorded into a graph otherwise."""
+    import torch
+
+    n = [6] * count
+    A = torch.randn(count, 36, dtype=torch.float64, device="cuda")
+    Cm = torch.zeros(count, 36, dtype=torch.float64, device="cuda")
+    want = torch.matmul(A.view(-1, 6, 6), A.view(-1, 6, 6)).reshape(count, 36)  # row-major: (B A)^T
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(20_000_000)
+    kmx_gpu.gemm_vbatched("N", "N", n, n, n, 1.0, list(A), n, list(A), n, 0.0, list(Cm), n, stream=side)
+    assert side.query()
+    assert torch.allclose(Cm, want, rtol=0, atol=1e-13)
+    if count <= 640:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            kmx_gpu.gemm_vbatched("N", "N", n, n, n, 1.0, list(A), n, list(A), n, 0.0, list(Cm), n,
+                                  stream=torch.cuda.current_stream())
+        for _ in range(3):
+            Cm.zero_()
+            graph.replay()
+            assert torch.allclose(Cm, want, rtol=0, atol=1e-13)
+            torch.cuda.synchronize()
