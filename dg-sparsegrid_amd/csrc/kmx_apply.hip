@@ -354,6 +354,17 @@ extern "C" int kmx_plan_get_sweep(const kmx_plan* p, int prec, int* available, i
     return KMX_OK;
 }
 
+extern "C" int kmx_plan_get_factored(const kmx_plan* p, int transpose, int* active) {
+    if (!p || !active) {
+        set_error("kmx_plan_get_factored: null argument");
+        return KMX_E_ARG;
+    }
+    const kmx_variant v = p->var[prec_slot(KMX_PREC_FP64)];
+    const bool sweep = p->sw && v.sweep && (!transpose || kmx_sweep_has_transpose(p));
+    *active = !sweep && !v.pairs && kmx_factor_ok(p, transpose != 0) ? 1 : 0;
+    return KMX_OK;
+}
+
 extern "C" int kmx_plan_replay_state(const kmx_plan* p, int prec, uint64_t* state) {
     if (!p || !state || (prec != KMX_PREC_FP64 && prec != KMX_PREC_FP32 && prec != KMX_PREC_BF16)) {
         set_error("kmx_plan_replay_state: bad arguments");

@@ -135,6 +135,7 @@ PROTOTYPES = {
     "kmx_plan_set_sweep": (C.c_int, [C.c_void_p, C.c_int, C.c_int]),
     "kmx_plan_get_sweep": (C.c_int, [C.c_void_p, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int),
                                      C.POINTER(C.c_double)]),
+    "kmx_plan_get_factored": (C.c_int, [C.c_void_p, C.c_int, C.POINTER(C.c_int)]),
     "kmx_plan_replay_state": (C.c_int, [C.c_void_p, C.c_int, C.POINTER(C.c_uint64)]),
     "kmx_plan_sweep_info": (C.c_int, [C.c_void_p, C.POINTER(SweepInfo)]),
     "kmx_realspace_create": (C.c_int, [C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int), C.c_int, C.POINTER(C.c_int),

@@ -241,6 +241,13 @@ class Plan:
         check(lib().kmx_plan_get_sweep(self.handle, _prec(prec), C.byref(av), C.byref(ac), C.byref(fl)))
         return {"available": bool(av.value), "active": bool(ac.value), "flops": fl.value}
 
+    def factored(self, transpose=False):
+        """Whether FP64 applies outside stream capture run with the pair sum factored over the
+        dimensions (kmx_plan_get_factored)."""
+        on = C.c_int()
+        check(lib().kmx_plan_get_factored(self.handle, int(bool(transpose)), C.byref(on)))
+        return bool(on.value)
+
     def replay_state(self, prec="fp64"):
         """A number that stays the same while a graph that captured an apply at prec replays
         the operator that apply runs (kmx_plan_replay_state)."""

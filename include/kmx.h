@@ -130,6 +130,11 @@ int kmx_plan_get_variant(const kmx_plan* plan, int prec, int* threads, int* lds_
 int kmx_plan_set_sweep(kmx_plan* plan, int prec, int on);
 int kmx_plan_get_sweep(const kmx_plan* plan, int prec, int* available, int* active, double* flops);
 
+/* Whether FP64 applies (transpose != 0: adjoint applies) of the plan take their pair sums one
+ * group of dimensions at a time now, where they are not under stream capture (see
+ * KMX_PLAN_LEVEL_BLOCKS): the plan holds that form and runs no sweep. */
+int kmx_plan_get_factored(const kmx_plan* plan, int transpose, int* active);
+
 /* What a graph that captures an apply at prec will replay, as one number: while it is the
  * same, a replay is the operator that kmx_apply runs.  It changes with the path (sweep or
  * pairs), with the term scales where they are launch arguments (not on a separable sweep,

@@ -178,3 +178,46 @@ def test_apply_while_the_last_stream_records_a_graph(kmx_gpu):
         torch.cuda.synchronize()
         assert rel(outs[1].cpu().numpy(), ref.cpu().numpy()) <= 1e-13
         assert not outs[2].any()
+
+
+@pytest.mark.parametrize("nd,lev,deg,T,conn", SHAPES + [(2, 4, 3, 2, True), (3, 3, 3, 2, True), (2, 4, 4, 2, False),
+                                                        (3, 3, 2, 2, True)])
+def test_which_plans_take_the_factored_form(kmx_gpu, monkeypatch, nd, lev, deg, T, conn):
+    """The plans of the tests above run the kernels that they are about: every shape but 2D
+    deg 5 (which no rule picks), with or without an adjoint; not below the size rule, and not
+    while a sweep is on."""
+    mats, idx, rp, cols, _ = case(nd, lev, deg, T, conn, 3)
+    has = (nd, deg) != (2, 5)
+    for adjoint in (False, True):
+        plan = kmx_gpu.Plan(mats, idx, deg, rp, cols, index_base=1, adjoint=adjoint)
+        assert plan.factored() == has and plan.factored(transpose=True) == (has and adjoint)
+        plan.update_term(0, 0, mats[0][0] + 1.0)
+        plan.set_term_scale(0, 0.5)
+        assert plan.factored() == has
+    monkeypatch.setenv("KMX_FACTOR_MIN_FMA", "1e300")
+    assert not kmx_gpu.Plan(mats, idx, deg, rp, cols, index_base=1).factored()
+
+
+def test_which_lists_take_the_factored_form(kmx_gpu):
+    mats, idx, rp, cols, _ = case(2, 4, 2, 2, True, 5)
+    rp, cols = np.asarray(rp), np.asarray(cols)
+    make = lambda i, r, c, **kw: kmx_gpu.Plan(mats, i, 2, r, c, index_base=1, **kw)
+    assert make(idx, rp, cols).factored()
+    assert not make(idx, rp - (rp > 7), np.delete(cols, 7)).factored()
+    assert not make(idx, rp + (rp > 11), np.insert(cols, 11, cols[11])).factored()
+    assert make(idx, None, None).factored()
+    assert not make(np.vstack([idx, idx[:3]]), None, None).factored()
+    general = make(idx, rp, cols, level_blocks=True)  # random factors: a sweep of the general form
+    assert general.factored()
+    general.set_sweep("fp64", True)
+    assert not general.factored()
+    general.set_sweep("fp64", False)
+    assert general.factored()
+
+
+def test_the_size_rule_picks_the_large_plans(kmx_gpu, monkeypatch):
+    """By the rule itself: a 3D level 7 run's plan is factored, a 2D level 3 one is not."""
+    monkeypatch.delenv("KMX_FACTOR_MIN_FMA")
+    for nd, lev, deg, T, want in ((3, 7, 2, 6, True), (2, 3, 2, 2, False)):
+        mats, idx, _, _, _ = case(nd, lev, deg, T, False, 1)
+        assert kmx_gpu.Plan(mats, idx, deg, None, None, index_base=1).factored() == want
