@@ -153,7 +153,7 @@ int kmx_launch_apply(kmx_plan* p, bool transpose, const double* x, double* y, in
         if (kmx_sweep_has_transpose(p)) return kmx_sweep_apply_transpose(p, prec_slot(prec), x, y, s);
     }
     kmx_variant v = p->var[prec_slot(prec)];
-    if (prec == KMX_PREC_FP64 && !v.pairs && kmx_factor_ok(p, transpose)) {
+    if (prec == KMX_PREC_FP64 && kmx_factor_ok(p, transpose)) {
         KArgs<double> k;
         fill_args(k, p, transpose, x, y);
         const int rc = kmx_factor_apply(p, transpose, k, s);
@@ -275,14 +275,14 @@ extern "C" int kmx_plan_autotune(kmx_plan* p, void* stream) {
         }
         if (rc != KMX_OK) break;
         p->var[prec_slot(prec)] = bestv;
-        // 2. the factored sum (FP64) against it
+        // 2. the factored sum (FP64) against it; where it loses, this plan gives it and its
+        // memory back (nothing to keep for others: which form wins goes with the size)
         if (prec == KMX_PREC_FP64 && kmx_factor_ok(p, false)) {
             float ms;
             rc = time_calls([&] { return kmx_launch_apply(p, false, x, y, prec, s); }, s, e0, e1, ms);
             if (rc != KMX_OK) break;
             if (ms < best) best = ms;
-            else bestv.pairs = 1;
-            p->var[prec_slot(prec)] = bestv;
+            else kmx_factor_free(p);
         }
         // 3. the dimension-sweep path against both
         if (p->sw && (prec == KMX_PREC_FP32 || kmx_sweep_fp64_ok(p))) {
@@ -361,7 +361,7 @@ extern "C" int kmx_plan_get_factored(const kmx_plan* p, int transpose, int* acti
     }
     const kmx_variant v = p->var[prec_slot(KMX_PREC_FP64)];
     const bool sweep = p->sw && v.sweep && (!transpose || kmx_sweep_has_transpose(p));
-    *active = !sweep && !v.pairs && kmx_factor_ok(p, transpose != 0) ? 1 : 0;
+    *active = !sweep && kmx_factor_ok(p, transpose != 0) ? 1 : 0;
     return KMX_OK;
 }
 

@@ -56,7 +56,6 @@ struct kmx_variant {
     int lds = -1;
     int kind = 0;          // 0: one lane per pair, 1: pair split over deg lanes
     int sweep = 0;         // 1: the dimension-sweep path (when the plan has one)
-    int pairs = 0;         // 1: pair by pair even where the factored apply serves the plan
 };
 
 // Level-block structure of a plan: elements grouped by their level

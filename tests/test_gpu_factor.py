@@ -221,3 +221,25 @@ def test_the_size_rule_picks_the_large_plans(kmx_gpu, monkeypatch):
     for nd, lev, deg, T, want in ((3, 7, 2, 6, True), (2, 3, 2, 2, False)):
         mats, idx, _, _, _ = case(nd, lev, deg, T, False, 1)
         assert kmx_gpu.Plan(mats, idx, deg, None, None, index_base=1).factored() == want
+
+
+def test_autotune_decides_for_its_own_plan(kmx_gpu):
+    """A plan on which the pair kernels are faster gives the factored form up; what it leaves
+    for later plans of its kind is the pair kernels' variant alone."""
+    import torch
+
+    mats, idx, rp, cols, x = case(2, 3, 2, 2, True, 6)  # far below the size rule
+    plan, other = (kmx_gpu.Plan(mats, idx, 2, rp, cols, index_base=1, adjoint=True) for _ in range(2))
+    xd = torch.from_numpy(x).cuda()
+    want = [plan.apply(xd).cpu().numpy(), plan.apply_transpose(xd).cpu().numpy()]
+    plan.autotune()
+    assert not plan.factored() and not plan.factored(transpose=True)
+    assert rel(plan.apply(xd).cpu().numpy(), want[0]) <= 1e-13
+    assert rel(plan.apply_transpose(xd).cpu().numpy(), want[1]) <= 1e-13
+    plan.update_term(0, 0, mats[0][0])
+    plan.autotune()
+    assert rel(plan.apply(xd).cpu().numpy(), want[0]) <= 1e-13
+    assert other.factored() and other.factored(transpose=True)
+    later = kmx_gpu.Plan(mats, idx, 2, rp, cols, index_base=1, adjoint=True)
+    assert later.factored() and later.factored(transpose=True)
+    assert np.array_equal(later.apply(xd).cpu().numpy(), want[0])
