@@ -625,7 +625,8 @@ struct kmx_factor {
     size_t o_mask[2][KMX_MAX_DIM] = {};  // forward, transposed
     double* d_fac[2] = {nullptr, nullptr};
     double* d_ws = nullptr;  // W, the partial sums, the matrices of d_fac
-    size_t w_elems = 0;
+    size_t w_elems = 0, mat = 0;  // values of W (of `room` classes), of one matrix set
+    int room = 0;
     int ncls = 0, cls_ptr[KMX_MAX_TERMS + 1] = {};
     unsigned char cls_scaled[KMX_MAX_TERMS] = {};
     FacTab tab = {};
@@ -756,6 +757,26 @@ static void factor_layout(const kmx_plan* p, kmx_factor* f, int t, int d, hipStr
             hipLaunchKernelGGL(k_factor_layout, dim3(grid), dim3(256), 0, s, (o ? p->d_blkT64 : p->d_blk64) + off,
                                f->d_fac[o] + f->tab.off[t * p->D + d], p->nb[d], dd,
                                f->masked ? f->d_mask + f->o_mask[o][d] : nullptr);
+}
+
+// The workspace for the classes that there are, with every matrix laid out in it: W of T
+// classes would be three times as much on a 6D diffusion operator (42 -> 17 MB at lev 4).
+static void factor_workspace(const kmx_plan* p, kmx_factor* f, hipStream_t s) {
+    if (f->d_ws) hipFree(f->d_ws);  // (waits for what still runs on it)
+    f->d_ws = f->d_fac[0] = f->d_fac[1] = nullptr;
+    f->room = f->ncls;
+    f->w_elems = size_t(f->ncls) * f->NV * f->launch.WN * size_t(f->G);
+    const size_t ws = (f->w_elems + size_t(f->splits) * p->N * p->B + 31) / 32 * 32;
+    if (hipMalloc(&f->d_ws, (ws + f->mat * (p->d_blkT64 ? 2 : 1)) * sizeof(double)) != hipSuccess) {
+        f->d_ws = nullptr;
+        throw std::bad_alloc();
+    }
+    f->d_fac[0] = f->d_ws + ws;
+    if (p->d_blkT64) f->d_fac[1] = f->d_fac[0] + f->mat;
+    for (int t = 0; t < p->T; ++t)
+        for (int d = 0; d < p->D; ++d) factor_layout(p, f, t, d, s);
+    if (hipStreamSynchronize(s) != hipSuccess || hipGetLastError() != hipSuccess)
+        throw std::runtime_error("factor layout");
 }
 
 void kmx_factor_build(kmx_plan* p, const std::vector<int>& idx, const std::vector<long long>& rp,
@@ -896,29 +917,19 @@ void kmx_factor_build(kmx_plan* p, const std::vector<int>& idx, const std::vecto
         }
         f->vptr = vptr;
         f->list = vcost;
-        size_t mat = 0;
         for (int d = 0; d < D; ++d) f->tab.nb[d] = p->nb[d];
         for (int t = 0; t < T; ++t)
             for (int d = 0; d < D; ++d) {
-                f->tab.off[t * D + d] = (long long)mat;
-                mat += size_t(p->nb[d]) * p->nb[d] * ((p->deg * p->deg + 1) / 2 * 2);
+                f->tab.off[t * D + d] = (long long)f->mat;
+                f->mat += size_t(p->nb[d]) * p->nb[d] * ((p->deg * p->deg + 1) / 2 * 2);
             }
         factor_classes(p, f);
         factor_slots(f);
         // splits of the node list until some 2048 waves run
         const long long wgs = (long long)((N + 63) / 64) * L.NCB;
         f->splits = int(std::max(1LL, std::min<long long>(512 / wgs, NV / (2 * UP_WAVES) + 1)));
-        f->w_elems = size_t(T) * NV * L.WN * size_t(G);  // (a replaced matrix may split a class)
-        const size_t ws = (f->w_elems + size_t(f->splits) * N * p->B + 31) / 32 * 32;
-        if (hipMalloc(&f->d_ws, (ws + mat * (p->d_blkT64 ? 2 : 1)) * sizeof(double)) != hipSuccess ||
-            hipEventCreateWithFlags(&f->ev, hipEventDisableTiming) != hipSuccess)
-            throw std::bad_alloc();
-        f->d_fac[0] = f->d_ws + ws;
-        if (p->d_blkT64) f->d_fac[1] = f->d_fac[0] + mat;
-        for (int t = 0; t < T; ++t)
-            for (int d = 0; d < D; ++d) factor_layout(p, f, t, d, nullptr);
-        if (hipStreamSynchronize(nullptr) != hipSuccess || hipGetLastError() != hipSuccess)
-            throw std::runtime_error("factor layout");
+        if (hipEventCreateWithFlags(&f->ev, hipEventDisableTiming) != hipSuccess) throw std::bad_alloc();
+        factor_workspace(p, f, nullptr);
     } catch (const std::exception&) {  // no room: the plan runs pair by pair
         (void)hipGetLastError();
         kmx_factor_free(p);
@@ -935,6 +946,7 @@ void kmx_factor_term_updated(kmx_plan* p, int term, int dim, hipStream_t s) {
     if (std::memcmp(&tab, &f->tab, sizeof(tab)) == 0) return;
     try {
         factor_slots(f);
+        if (f->ncls > f->room) factor_workspace(p, f, s);  // the matrix split a class
     } catch (const std::exception&) {  // no room: the plan runs pair by pair
         (void)hipGetLastError();
         kmx_factor_free(p);

@@ -243,3 +243,35 @@ def test_autotune_decides_for_its_own_plan(kmx_gpu):
     later = kmx_gpu.Plan(mats, idx, 2, rp, cols, index_base=1, adjoint=True)
     assert later.factored() and later.factored(transpose=True)
     assert np.array_equal(later.apply(xd).cpu().numpy(), want[0])
+
+
+@pytest.mark.parametrize("nd,lev,deg,T,conn", [(3, 3, 3, 3, True), (6, 1, 2, 6, False), (2, 4, 2, 4, True)])
+def test_matrices_that_split_and_join_classes(kmx_gpu, nd, lev, deg, T, conn):
+    """Terms that share matrices share partial sums.  Matrices replaced one by one until no
+    two terms share any, and back: more sums than the plan began with, the same ones again."""
+    import torch
+
+    mats, idx, rp, cols, x = case(nd, lev, deg, T, conn, 8, shared=True)
+    plan = kmx_gpu.Plan(mats, idx, deg, rp, cols, index_base=1, adjoint=True)
+    xd = torch.from_numpy(x).cuda()
+    first = [plan.apply(xd).clone(), plan.apply_transpose(xd).clone()]
+    rng = np.random.default_rng(4)
+    now = [list(tm) for tm in mats]
+
+    def check():
+        assert plan.factored() and plan.factored(transpose=True)
+        for y, ms in ((plan.apply(xd), now), (plan.apply_transpose(xd), [[m.T.copy() for m in tm] for tm in now])):
+            assert rel(y.cpu().numpy(), O.apply_A(O.ApplyInputs(ms, idx, deg, rp, cols), x, nthreads=8)) <= 1e-13
+
+    for t in range(T):
+        for d in range(nd):
+            if d != t % nd:
+                now[t][d] = rng.standard_normal(mats[t][d].shape)
+                plan.update_term(t, d, now[t][d])
+        check()
+    for t in reversed(range(T)):
+        for d in range(nd):
+            now[t][d] = mats[t][d]
+            plan.update_term(t, d, mats[t][d])
+    check()
+    assert torch.equal(plan.apply(xd), first[0]) and torch.equal(plan.apply_transpose(xd), first[1])
