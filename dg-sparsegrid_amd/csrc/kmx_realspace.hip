@@ -154,11 +154,12 @@ __global__ void __launch_bounds__(256, 2) k_rs_last(StageArgs a) {
     const int i0 = 16 * (t % a.mt), j0 = 64 * (t / a.mt);
     bool every = !a.lptr;
     if (!every) {  // (or a coefficient of the node that is not finite)
-        const int c0 = a.cptr[q], n = (a.cptr[q + 1] - c0) * a.B;
+        const int c0 = a.cptr[q];
+        const unsigned B = unsigned(a.B), n = unsigned(a.cptr[q + 1] - c0) * B;
         int bad = 0;
-        for (int i = threadIdx.x; i < n; i += 256) {
-            const int c = i / a.B;
-            bad |= !finite(a.in[(long long)a.row[c0 + c] * a.B + i - c * a.B]);
+        for (unsigned i = threadIdx.x; i < n; i += 256) {
+            const unsigned c = i / B;
+            bad |= !finite(a.in[(long long)a.row[c0 + c] * B + (i - c * B)]);
         }
         every = __syncthreads_or(bad);
     }
@@ -217,14 +218,17 @@ __global__ void __launch_bounds__(256, 2) k_rs_mode(StageArgs a) {
         split_k(k, a, c, b);
         return ch.col[c] + b;
     };
-    auto line = [&](int k) {  // of Z_{k+1}: child, beta, b
+    // line of Z_{k+1}: child, beta, b; from the node's first child on, whose place is in 64
+    // bits (children x deg^k stay below 2^31: a level's cells x deg^d do below 2^30)
+    const double* in = a.in + ((long long)c0 * a.nbeta + beta) * a.deg * a.R + j0;
+    auto line = [&](int k) {
         int c, b;
         split_k(k, a, c, b);
-        return ((c0 + (ch.x ? ch.x[c] : c)) * a.nbeta + beta) * a.deg + b;
+        return (ch.x ? ch.x[c] : c) * a.nbeta * a.deg + b;
     };
     using Map = Mma64Map<64, 16, false>;
     LineOperand<Map, decltype(column)> la(column, a.A + i0, a.M, a.M - i0, K);
-    LineOperand<Map, decltype(line)> lb(line, a.in + j0, a.R, n, K);
+    LineOperand<Map, decltype(line)> lb(line, in, a.R, n, K);
     double* out = a.out + (long long)item * a.M * a.R + j0;
     bool bad = false;
     auto st = [&](int i, int j, double v) {
@@ -354,7 +358,8 @@ extern "C" int kmx_realspace_create(int ndim, int deg, int num_elem, const int* 
             if (hipMemcpy(r->d_meval[k], meval[k], sz * sizeof(double), hipMemcpyHostToDevice) != hipSuccess)
                 throw std::runtime_error("hipMemcpy failed");
         }
-        // element indices, level tuples and cells as the transform takes them
+        // element indices; and the limit on a level tuple's values, which the stages' 32-bit
+        // places inside a node's list rely on
         std::map<std::vector<int>, long long> lev_cells;
         std::vector<int> idx(size_t(num_elem) * ndim);
         for (int e = 0; e < num_elem; ++e) {
@@ -489,7 +494,8 @@ extern "C" int kmx_realspace_apply(kmx_realspace* r, const double* f_w, double* 
             a.xcd = 0;
             grid = (long long)a.items * a.mt * a.nt;
         } else {
-            a.items = r->stage[k].nodes * a.nbeta;
+            const long long items = (long long)r->stage[k].nodes * a.nbeta;
+            a.items = int(std::min<long long>(items, 0x7fffffff));
             a.mt = (a.M + 63) / 64;
             const long long nt = (R + 63) / 64;
             if (nt >= (1LL << 30)) {
@@ -498,7 +504,7 @@ extern "C" int kmx_realspace_apply(kmx_realspace* r, const double* f_w, double* 
             }
             a.nt = int(nt);
             a.xcd = a.mt > 1 && a.nt >= 8 ? 1 : 0;
-            grid = (long long)a.items * a.mt * (a.xcd ? (nt + 7) / 8 * 8 : nt);
+            grid = items * a.mt * (a.xcd ? (nt + 7) / 8 * 8 : nt);
         }
         if (grid >= (1LL << 31)) {
             set_error("kmx_realspace_apply: too many points");
