@@ -43,10 +43,8 @@
 #include "kmx_kernels.h"
 
 #include <algorithm>
-#include <atomic>
 #include <cstdlib>
 #include <cstring>
-#include <future>
 #include <map>
 #include <mutex>
 #include <numeric>
@@ -451,10 +449,24 @@ __global__ void __launch_bounds__(256) k_factor_sum(FacArgs a, KArgs<double> k) 
     }
 }
 
-// [I][J][a][b] blocks of one matrix -> [J][pair][I][2], zero where mask[I * nb + J] is 0
-// and in the half of an odd block's last pair
-__global__ void __launch_bounds__(256) k_factor_layout(const double* __restrict__ blk, double* __restrict__ out, int nb,
-                                                       int dd, const unsigned char* __restrict__ mask) {
+// [I][J][a][b] blocks of the matrices first, first + 1, ... (term by term) -> [J][pair][I][2],
+// zero where the dimension's mask[I * nb + J] is 0 and in the half of an odd block's last pair.
+// blockIdx.y: the matrix, z: forward or transposed.  One launch for all of them: a launch
+// each was 130 us of a 6D plan's set-up.
+struct LayoutArgs {
+    const double* blk[2];
+    double* out[2];
+    long long src[KMX_MAX_TERMS * KMX_MAX_DIM], dst[KMX_MAX_TERMS * KMX_MAX_DIM];
+    const unsigned char* mask;  // null: none
+    long long mask_at[2][KMX_MAX_DIM];
+    int nb[KMX_MAX_DIM];
+    int D, dd, first;
+};
+__global__ void __launch_bounds__(256) k_factor_layout(LayoutArgs g) {
+    const int m = g.first + int(blockIdx.y), d = m % g.D, o = int(blockIdx.z), dd = g.dd, nb = g.nb[d];
+    const double* __restrict__ blk = g.blk[o] + g.src[m];
+    double* __restrict__ out = g.out[o] + g.dst[m];
+    const unsigned char* __restrict__ mask = g.mask ? g.mask + g.mask_at[o][d] : nullptr;
     const int pairs = (dd + 1) / 2;
     const long long n = (long long)nb * nb * pairs * 2;
     for (long long q = blockIdx.x * 256ll + threadIdx.x; q < n; q += (long long)gridDim.x * 256) {
@@ -517,25 +529,6 @@ T* fac_upload(const std::vector<T>& h) {
     return d;
 }
 
-// f(begin, end) over [0, n), in up to four parts at a time where `many`
-template <class F>
-void in_parts(int n, bool many, const F& f) {
-    const int parts = many ? std::min(4, n) : 1;
-    std::vector<std::future<void>> others;
-    int done = 0;
-    for (int q = 1; q < parts; ++q) {
-        const int end = int((long long)n * q / parts);
-        try {
-            others.push_back(std::async(std::launch::async, [&f, done, end] { f(done, end); }));
-        } catch (const std::system_error&) {
-            break;  // no thread to be had: the rest here
-        }
-        done = end;
-    }
-    f(done, n);
-    for (auto& o : others) o.get();
-}
-
 // Per dimension the 1D connections of a pair list that is their tensor product over the
 // element set (every pair list row equals the product's row, as sets, without
 // repetitions); false if it is not one.
@@ -547,61 +540,54 @@ bool product_masks(const kmx_plan* p, const std::vector<int>& idx, const std::ve
     for (int d = 0; d < D; ++d) bits += double(p->nb[d]) * double(words) * 16.0;
     if (bits > 512e6) return false;
     typedef unsigned long long word;
-    // (3D lev 7, 1,903,000 pairs: the plan took 5.0 ms without this check, 8.7 with it in one
-    // thread and a bit at a time, 5.5 to 6.7 so)
-    const bool many = rp[size_t(N)] > 100000;
-    std::atomic<bool> product{true};
     // the rows as bit sets: a word stays in a register while consecutive columns lie in it
+    // (3D lev 7, 1,903,000 pairs: 0.9 of the check's 1.2 ms.  Four threads took 0.4 once warm,
+    // but 3 to 4 ms in each of a process's first plans.)
     std::vector<word> rows(size_t(N) * words, 0);
-    in_parts(N, many, [&](int i0, int i1) {
-        for (int i = i0; i < i1; ++i) {
-            word* row = &rows[size_t(i) * words];
-            const int* c = cols.data() + rp[size_t(i)];
-            const int* const end = cols.data() + rp[size_t(i) + 1];
-            while (c != end) {
-                const unsigned at = unsigned(*c) / 64;
-                word bits = 0;
-                do bits |= word(1) << (unsigned(*c) % 64);
-                while (++c != end && unsigned(*c) / 64 == at);
-                row[at] |= bits;
-            }
-            long long held = 0;
-            for (size_t k = 0; k < words; ++k) held += __builtin_popcountll(row[k]);
-            if (held != rp[size_t(i) + 1] - rp[size_t(i)]) product = false;  // a pair listed twice
+    for (int i = 0; i < N; ++i) {
+        word* row = &rows[size_t(i) * words];
+        const int* c = cols.data() + rp[size_t(i)];
+        const int* const end = cols.data() + rp[size_t(i) + 1];
+        while (c != end) {
+            const unsigned at = unsigned(*c) / 64;
+            word bits = 0;
+            do bits |= word(1) << (unsigned(*c) % 64);
+            while (++c != end && unsigned(*c) / 64 == at);
+            row[at] |= bits;
         }
-    });
-    if (!product) return false;
+        long long held = 0;
+        for (size_t k = 0; k < words; ++k) held += __builtin_popcountll(row[k]);
+        if (held != rp[size_t(i) + 1] - rp[size_t(i)]) return false;  // a pair listed twice
+    }
     // per dimension: (I, J) is connected where a row with index I holds an element with index
     // J; conn: per I the elements j whose J_d is connected to it
     std::vector<std::vector<word>> conn(static_cast<size_t>(D));
     mask.assign(size_t(D), {});
-    in_parts(D, many, [&](int d0, int d1) {
-        for (int d = d0; d < d1; ++d) {
-            const int nb = p->nb[d];
-            std::vector<unsigned char>& md = mask[size_t(d)];
-            std::vector<word>& c = conn[size_t(d)];
-            md.assign(size_t(nb) * nb, 0);
-            c.assign(size_t(nb) * words, 0);
-            std::vector<word> with(size_t(nb) * words, 0);  // per J the elements that have it
-            for (int i = 0; i < N; ++i) {
-                const size_t I = size_t(idx[size_t(i) * D + d]);
-                with[I * words + size_t(i) / 64] |= word(1) << (i % 64);
-                for (size_t k = 0; k < words; ++k) c[I * words + k] |= rows[size_t(i) * words + k];
-            }
-            for (int I = 0; I < nb; ++I) {
-                word* set = &c[size_t(I) * words];
-                for (int J = 0; J < nb; ++J) {
-                    const word* w = &with[size_t(J) * words];
-                    word any = 0;
-                    for (size_t k = 0; k < words; ++k) any |= set[k] & w[k];
-                    md[size_t(I) * nb + J] = any != 0;
-                }
-                for (int J = 0; J < nb; ++J)
-                    if (md[size_t(I) * nb + J])
-                        for (size_t k = 0; k < words; ++k) set[k] |= with[size_t(J) * words + k];
-            }
+    for (int d = 0; d < D; ++d) {
+        const int nb = p->nb[d];
+        std::vector<unsigned char>& md = mask[size_t(d)];
+        std::vector<word>& c = conn[size_t(d)];
+        md.assign(size_t(nb) * nb, 0);
+        c.assign(size_t(nb) * words, 0);
+        std::vector<word> with(size_t(nb) * words, 0);  // per J the elements that have it
+        for (int i = 0; i < N; ++i) {
+            const size_t I = size_t(idx[size_t(i) * D + d]);
+            with[I * words + size_t(i) / 64] |= word(1) << (i % 64);
+            for (size_t k = 0; k < words; ++k) c[I * words + k] |= rows[size_t(i) * words + k];
         }
-    });
+        for (int I = 0; I < nb; ++I) {
+            word* set = &c[size_t(I) * words];
+            for (int J = 0; J < nb; ++J) {
+                const word* w = &with[size_t(J) * words];
+                word any = 0;
+                for (size_t k = 0; k < words; ++k) any |= set[k] & w[k];
+                md[size_t(I) * nb + J] = any != 0;
+            }
+            for (int J = 0; J < nb; ++J)
+                if (md[size_t(I) * nb + J])
+                    for (size_t k = 0; k < words; ++k) set[k] |= with[size_t(J) * words + k];
+        }
+    }
     for (int i = 0; i < N; ++i)
         for (size_t k = 0; k < words; ++k) {
             word m = ~word(0);
@@ -747,16 +733,29 @@ static void factor_slots(kmx_factor* f) {
     f->d_tab = t;
 }
 
-static void factor_layout(const kmx_plan* p, kmx_factor* f, int t, int d, hipStream_t s) {
-    const long long off = p->off[t * p->D + d];
-    const int dd = p->deg * p->deg;
-    const long long n = (long long)p->nb[d] * p->nb[d] * (dd + 1);
-    const unsigned grid = unsigned(std::min<long long>((n + 255) / 256, 8192));
-    for (int o = 0; o < 2; ++o)
-        if (f->d_fac[o])
-            hipLaunchKernelGGL(k_factor_layout, dim3(grid), dim3(256), 0, s, (o ? p->d_blkT64 : p->d_blk64) + off,
-                               f->d_fac[o] + f->tab.off[t * p->D + d], p->nb[d], dd,
-                               f->masked ? f->d_mask + f->o_mask[o][d] : nullptr);
+// Matrices [first, first + count) of the plan into the walks' layout.
+static void factor_layout(const kmx_plan* p, kmx_factor* f, int first, int count, hipStream_t s) {
+    LayoutArgs g;
+    std::memset(&g, 0, sizeof(g));
+    g.blk[0] = p->d_blk64;
+    g.blk[1] = p->d_blkT64;
+    for (int o = 0; o < 2; ++o) {
+        g.out[o] = f->d_fac[o];
+        for (int d = 0; d < p->D; ++d) g.mask_at[o][d] = (long long)f->o_mask[o][d];
+    }
+    g.mask = f->masked ? f->d_mask : nullptr;
+    std::copy(p->off, p->off + p->T * p->D, g.src);
+    std::copy(f->tab.off, f->tab.off + p->T * p->D, g.dst);
+    std::copy(p->nb, p->nb + p->D, g.nb);
+    g.D = p->D;
+    g.dd = p->deg * p->deg;
+    g.first = first;
+    long long n = 0;
+    for (int m = first; m < first + count; ++m)
+        n = std::max(n, (long long)p->nb[m % p->D] * p->nb[m % p->D] * (g.dd + 1));
+    hipLaunchKernelGGL(k_factor_layout, dim3(unsigned(std::min<long long>((n + 255) / 256, 8192)), unsigned(count),
+                                             f->d_fac[1] ? 2u : 1u),
+                       dim3(256), 0, s, g);
 }
 
 // The workspace for the classes that there are, with every matrix laid out in it: W of T
@@ -773,8 +772,7 @@ static void factor_workspace(const kmx_plan* p, kmx_factor* f, hipStream_t s) {
     }
     f->d_fac[0] = f->d_ws + ws;
     if (p->d_blkT64) f->d_fac[1] = f->d_fac[0] + f->mat;
-    for (int t = 0; t < p->T; ++t)
-        for (int d = 0; d < p->D; ++d) factor_layout(p, f, t, d, s);
+    factor_layout(p, f, 0, p->T * p->D, s);
     if (hipStreamSynchronize(s) != hipSuccess || hipGetLastError() != hipSuccess)
         throw std::runtime_error("factor layout");
 }
@@ -939,7 +937,7 @@ void kmx_factor_build(kmx_plan* p, const std::vector<int>& idx, const std::vecto
 void kmx_factor_term_updated(kmx_plan* p, int term, int dim, hipStream_t s) {
     if (!p->fac) return;
     kmx_factor* f = p->fac;
-    factor_layout(p, f, term, dim, s);
+    factor_layout(p, f, term * p->D + dim, 1, s);
     if (hipStreamSynchronize(s) != hipSuccess) throw std::runtime_error("kmx_factor_term_updated: synchronize failed");
     const FacTab tab = f->tab;
     factor_classes(p, f);
