@@ -430,6 +430,21 @@ def gmres(matvec, b, x0=None, tol=1e-6, restart=40, maxiter=400):
 # finer ones share their rows with, the whole inverse takes too much.
 SCALE_POWER = -0.75
 
+# Vectors of up to this many values run the Arnoldi step's register kernels (kmx_gmres.hip:
+# 128 workgroups of 256 values)
+ARNOLDI_SHORT = 32768
+
+
+def box_order(n, nb):
+    """Whether a backward Euler step of n values keeps its Krylov vectors in the order of the
+    plan's sweep, nb values with the absent cells (0: the plan has none): two launches fewer a
+    step, 6D lev 4 deg 2 2.98 -> 2.70 ms.  A step measured in both orders, element over box:
+    1.05 to 1.15 on 2D to 6D grids whose vectors grow by up to 1.9 and stay short, 1.04 to
+    1.08 on long ones that grow by up to 1.43 and 0.97 at 1.69, but 0.77 to 0.84 where short
+    vectors grow long (6D, 32,512 to 33,728 values: 2.04 against 2.45 ms)."""
+    return 0 < nb <= 1.125 * n and not n <= ARNOLDI_SHORT < nb
+
+
 _SOLVERS = weakref.WeakKeyDictionary()  # plan -> {(dt, inner precision, restart, n): DeviceGMRES}
 
 
@@ -450,10 +465,8 @@ def backward_euler(plan, f0, dt, rhs=None, tol=1e-10, inner_prec="fp32", inner_t
     af = torch.empty_like(b)  # A f, FP64
     r = torch.empty_like(b)
 
-    # a plan whose applies are a lone sweep: Krylov vectors in its order, unless absent cells
-    # make them much longer (two launches fewer a step: 6D lev 4 deg 2 2.98 -> 2.70 ms)
     nb = plan.box_values(inner_prec) if hasattr(plan, "box_values") else 0
-    boxed = 0 < nb <= 1.125 * f0.numel()
+    boxed = box_order(f0.numel(), nb)
     key = (float(dt), inner_prec, int(restart), f0.numel(), boxed)
     cache = _SOLVERS.setdefault(plan, {})
     solver = cache.get(key)

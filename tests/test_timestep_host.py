@@ -41,3 +41,22 @@ def test_gmres_holds_back_chunks_only_when_the_queued_steps_converge():
     assert not held(g, [1.0], 1e-3)                      # no step yet
     assert not held(SimpleNamespace(chunk=4, depth=1), rs, 1e-11)  # nothing queued
     assert not held(g, rs, 0.0)  # tol = 0: never converges by estimate
+
+
+def test_krylov_vectors_in_the_sweeps_order():
+    """Not without a sweep, not much longer ones, and not across the end of the register
+    kernels (kmx_gmres.hip: AR_MAX_G workgroups of AR_MIN_CHUNK values)."""
+    import os
+    import re
+
+    from conftest import ROOT
+
+    from kmx import timestep as TS
+
+    src = open(os.path.join(ROOT, "dg-sparsegrid_amd", "csrc", "kmx_gmres.hip")).read()
+    g, c = (int(re.search(rf"constexpr int {n} = (\d+)", src).group(1)) for n in ("AR_MAX_G", "AR_MIN_CHUNK"))
+    assert TS.ARNOLDI_SHORT == g * c
+    assert not TS.box_order(2304, 0) and TS.box_order(2304, 2304) and TS.box_order(32064, 32064)
+    assert TS.box_order(8000, 9000) and not TS.box_order(8000, 9001)
+    assert TS.box_order(32512, 32768) and not TS.box_order(32512, 32769) and not TS.box_order(32768, 33728)
+    assert TS.box_order(32769, 33728)
