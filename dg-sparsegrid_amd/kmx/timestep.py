@@ -398,10 +398,11 @@ class DeviceGMRES:
             if self.scale is None:
                 x.addmv_(self.V[: ls.k].t(), y.to(b.device, non_blocking=True))
             else:
-                d = torch.mv(self.V[: ls.k].t(), y.to(b.device, non_blocking=True)).mul_(self.scale)
-                if self.box is not None:
-                    d = self.box[0]().from_box(d, torch.empty_like(x), self.box[1])
-                x.add_(d)
+                d = torch.mv(self.V[: ls.k].t(), y.to(b.device, non_blocking=True))
+                if self.box is None:
+                    x.addcmul_(self.scale, d)
+                else:
+                    x.add_(self.box[0]().from_box(d.mul_(self.scale), torch.empty_like(x), self.box[1]))
             est = ls.residual() / bnorm
             if est <= tol or it >= maxiter:
                 return x, est, it
@@ -423,12 +424,27 @@ def gmres(matvec, b, x0=None, tol=1e-6, restart=40, maxiter=400):
     return x, float(torch.linalg.vector_norm(b - matvec(x))) / max(float(torch.linalg.vector_norm(b)), 1e-300), it
 
 
-# The scaling's power of the diagonal.  Of 6D, 4D, 3D and 2D diffusion and advection-diffusion
-# steps of 10 to 100 explicit limits, -0.75 needs the fewest steps (6D lev 4 deg 2 at 100
-# limits, three solves: 29, 45, 44 unscaled; 22, 27, 28 at -1; 20, 25, 26 at -0.75; 2D lev 6
-# deg 3 at 30 limits: 38, 55, 54; 36, 66, 65; 32, 58, 55): on the coarse wavelets, which the
-# finer ones share their rows with, the whole inverse takes too much.
-SCALE_POWER = -0.75
+def scale_power(nd, deg):
+    """The power of the operator's diagonal that backward Euler's GMRES is scaled by (0: not).
+    On the coarse wavelets, which the finer ones share their rows with, the whole inverse takes
+    too much, and the more so the higher the degree and the fewer the dimensions.  Inner steps
+    over unscaled ones, three solves each at 3, 30 and 100 explicit limits:
+      diffusion      deg  -1/4              -1/2              -3/4
+      5D, 6D          2   0.83 .. 1.00      0.71 .. 0.91      0.67 .. 0.91
+      1D to 4D        2   0.80 .. 1.00      0.74 .. 1.00      0.79 .. 1.00
+      1D to 4D        3   0.87 .. 0.99      0.80 .. 0.99      0.78 .. 1.10
+      3D            4, 5  0.95 .. 1.00      0.94 .. 1.03      1.00 .. 1.10
+      2D            4, 5  0.96 .. 1.05      1.02 .. 1.17      1.13 .. 1.41
+      1D              4   1.01 .. 1.04      1.07 .. 1.18      1.25 .. 1.41
+    Advection-diffusion gains most from the highest (1D to 3D: 0.58 .. 0.93, 0.43 .. 0.88,
+    0.37 .. 0.89), but the sizes do not tell it from diffusion.  Setting the scale up and
+    applying it is 50 to 70 us a call, the price of a step so mild that it saves nothing."""
+    if nd >= 5:
+        return -0.75
+    if deg <= 3:
+        return -0.5
+    return -0.25 if nd >= 3 else 0.0
+
 
 # Vectors of up to this many values run the Arnoldi step's register kernels (kmx_gmres.hip:
 # 128 workgroups of 256 values)
@@ -455,9 +471,9 @@ def backward_euler(plan, f0, dt, rhs=None, tol=1e-10, inner_prec="fp32", inner_t
     Iterative refinement: the FP64 residual r = b - (I - dt A) f1 (plain FP64
     apply) drives a correction solved by GMRES with `inner_prec` applies to
     relative accuracy inner_tol, until ||r|| / ||b|| <= tol.  GMRES is scaled by a power of
-    the operator's diagonal 1 - dt A_ii where that is over 1 (stiff rows).  The GMRES solver
-    (its captured Arnoldi graphs) is kept per plan and step size for later steps; what the
-    graphs hold of the operator (Plan.replay_state) is looked at in each step.
+    the operator's diagonal 1 - dt A_ii where that is over 1 (stiff rows; scale_power).  The
+    solver (its captured Arnoldi graphs) is kept per plan and step size for later steps; what
+    the graphs hold of the operator (Plan.replay_state) is looked at in each step.
     Returns (f1, history of FP64 relative residuals, inner iterations)."""
     torch = _torch()
     b = f0.clone() if rhs is None else f0 + dt * rhs
@@ -467,20 +483,25 @@ def backward_euler(plan, f0, dt, rhs=None, tol=1e-10, inner_prec="fp32", inner_t
 
     nb = plan.box_values(inner_prec) if hasattr(plan, "box_values") else 0
     boxed = box_order(f0.numel(), nb)
-    key = (float(dt), inner_prec, int(restart), f0.numel(), boxed)
+    power = scale_power(plan.ndim, plan.deg) if hasattr(plan, "diagonal") else 0.0
+    scaled = boxed or power != 0.0
+    key = (float(dt), inner_prec, int(restart), f0.numel(), boxed, scaled)
     cache = _SOLVERS.setdefault(plan, {})
     solver = cache.get(key)
     if solver is None:
         pref = weakref.ref(plan)  # the cache must not keep its own key alive
         solver = DeviceGMRES(lambda x, y: pref().apply(x, y, prec=inner_prec), f0.numel(), restart, f0.device,
-                             shift=(1.0, -float(dt)), scaled=True,
+                             shift=(1.0, -float(dt)), scaled=scaled,
                              box=(pref, inner_prec) if boxed else None)
         cache[key] = solver
     if hasattr(plan, "replay_state"):  # (a stand-in for a plan may have its product alone)
         solver.captured_for(plan.replay_state(inner_prec))
-    if hasattr(plan, "diagonal"):
-        d = plan.diagonal().mul_(-float(dt)).add_(1.0).clamp_(min=1.0).pow_(SCALE_POWER)
-        solver.scale.copy_(d) if solver.box is None else plan.to_box(d, solver.scale, inner_prec)
+    if power:  # (a scale is 1 otherwise)
+        d = torch.rsub(plan.diagonal(), 1.0, alpha=float(dt)).clamp_(min=1.0)
+        if solver.box is None:
+            torch.pow(d, power, out=solver.scale)
+        else:
+            plan.to_box(d.pow_(power), solver.scale, inner_prec)
     f = f0.clone()  # f0 is a good first guess for small dt
     hist, inner = [], 0
     for _ in range(max_refine):

@@ -245,3 +245,30 @@ def test_backward_euler_follows_its_operator(kmx_gpu, sweep, prec):
             plan.set_term_scale(t, s)
         assert step(plan) == step(make())
     assert len(TS._SOLVERS[plan]) == 1
+
+
+@pytest.mark.parametrize("nd,lev,deg", [(1, 9, 2), (1, 9, 3), (1, 7, 4), (2, 7, 3), (2, 6, 4), (3, 6, 2), (3, 5, 3),
+                                        (3, 4, 4), (4, 4, 2), (5, 4, 2), (6, 3, 2)])
+def test_scaling_costs_no_inner_steps(kmx_gpu, monkeypatch, nd, lev, deg):
+    """Diffusion, which the scaling helps least: against the unscaled solver's inner steps over
+    steps of 3, 30 and 100 explicit limits, no more of them (a chance step or two of one solve
+    aside: 3 of a hundred)."""
+    import torch
+    from kmx import timestep as TS
+
+    pde = K.diffusion_nd(nd, lev)
+    tab = G.hash_table_sparse_nd([lev] * nd, lev, "SG")
+    plan = kmx_gpu.Plan(K.get_coeff_mats(pde, deg), tab.idx1d, deg, None, None, index_base=1, fp32=True,
+                        level_blocks=True, identity=[[d != t for d in range(nd)] for t in range(nd)])
+    for p in ("fp64", "fp32"):
+        if plan.sweep(p)["available"]:  # (1D operators have none)
+            plan.set_sweep(p, True)
+    fs = [torch.from_numpy(np.random.default_rng(s).standard_normal(plan.dof)).cuda() for s in range(2)]
+
+    def steps():
+        TS._SOLVERS.pop(plan, None)
+        return sum(TS.backward_euler(plan, f, x * pde.set_dt(pde, 0.01), tol=1e-12)[2] for x in (3, 30, 100) for f in fs)
+
+    scaled = steps()
+    monkeypatch.setattr(TS, "scale_power", lambda nd, deg: 0.0)
+    assert scaled <= 1.03 * steps()
