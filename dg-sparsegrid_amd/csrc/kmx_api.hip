@@ -305,9 +305,10 @@ int kmx_plan_update_term(kmx_plan* p, int term, int dim, const double* mat, void
                           "hipMemcpyAsync");
             }
         }
+        kmx_factor_term_copied(p, term, dim, s);
         // the float staging vectors die here: wait for the copies that read them
         hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
-        kmx_factor_term_updated(p, term, dim, s);
+        kmx_factor_term_updated(p, s);
         kmx_blocks_update_term(p, term, dim, mat, s);
         kmx_sweep_term_updated(p, term, dim);
         ++p->version;

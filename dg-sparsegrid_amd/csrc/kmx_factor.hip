@@ -934,11 +934,13 @@ void kmx_factor_build(kmx_plan* p, const std::vector<int>& idx, const std::vecto
     }
 }
 
-void kmx_factor_term_updated(kmx_plan* p, int term, int dim, hipStream_t s) {
+void kmx_factor_term_copied(kmx_plan* p, int term, int dim, hipStream_t s) {
+    if (p->fac) factor_layout(p, p->fac, term * p->D + dim, 1, s);
+}
+
+void kmx_factor_term_updated(kmx_plan* p, hipStream_t s) {
     if (!p->fac) return;
     kmx_factor* f = p->fac;
-    factor_layout(p, f, term * p->D + dim, 1, s);
-    if (hipStreamSynchronize(s) != hipSuccess) throw std::runtime_error("kmx_factor_term_updated: synchronize failed");
     const FacTab tab = f->tab;
     factor_classes(p, f);
     if (std::memcmp(&tab, &f->tab, sizeof(tab)) == 0) return;

@@ -141,7 +141,9 @@ void kmx_blocks_free(kmx_plan* p);
 // 0 the call has to run pair by pair (stream capture), negative an error.
 void kmx_factor_build(kmx_plan* p, const std::vector<int>& idx, const std::vector<long long>& rp,
                       const std::vector<int>& cols);
-void kmx_factor_term_updated(kmx_plan* p, int term, int dim, hipStream_t s);
+// A replaced matrix: its copy on s, and, once that is done, what follows for the whole plan
+void kmx_factor_term_copied(kmx_plan* p, int term, int dim, hipStream_t s);
+void kmx_factor_term_updated(kmx_plan* p, hipStream_t s);
 bool kmx_factor_ok(const kmx_plan* p, bool transpose);
 int kmx_factor_apply(kmx_plan* p, bool transpose, const kmx::KArgs<double>& k, hipStream_t s);
 void kmx_factor_free(kmx_plan* p);
