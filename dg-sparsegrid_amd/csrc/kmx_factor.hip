@@ -37,9 +37,9 @@
 // block multiplies by zero what the pair list leaves out, which is not the same when x
 // holds an infinity or a NaN.
 //
-// W and the partial sums of y live in a workspace of the plan, one apply at a time: an
-// apply on another stream waits for the last one (event), and an apply under stream
-// capture -- whose replays this cannot order -- runs pair by pair.
+// W and the partial sums of y live in workspaces of the plan, a stream's applies in one of up
+// to four (the fifth stream takes the one longest unused, behind its last apply), and an
+// apply under stream capture -- whose replays this cannot order -- runs pair by pair.
 #include "kmx_kernels.h"
 
 #include <algorithm>
@@ -60,6 +60,8 @@ constexpr int FAC_LIST = 24;   // contractions of a virtual node's list at most
 constexpr int FAC_REC = 8;     // ints per walk record
 constexpr int DOWN_WAVES = 4;  // waves of a workgroup of k_factor_down (each a piece of a list)
 constexpr int FAC_PIECE = 12;  // contractions of a piece aimed at
+constexpr int FAC_SLOTS = 4;   // workspaces of a plan (streams whose applies overlap) at most
+constexpr double FAC_BYTES = 1024e6;  // ... and bytes of them together
 constexpr int UP_WAVES = 4;    // waves of a workgroup of k_factor_up (each a range of nodes)
 
 // Wave-uniform reads (x, the records) through the scalar cache: constant during a launch.
@@ -620,10 +622,15 @@ struct kmx_factor {
     std::vector<int> vptr, list;  // first record and contractions of every virtual node
     int* d_slot = nullptr;
     int nwg = 0;
-    // one apply at a time on the workspace
+    // one apply at a time on a workspace; d_ws holds the first one
+    struct Slot {
+        double* ws = nullptr;
+        hipStream_t last = nullptr;
+        unsigned long long turn = 0;  // of its last apply (0: none yet)
+    };
     std::mutex mu;
-    hipStream_t last = nullptr;
-    bool used = false;
+    Slot slot[FAC_SLOTS];
+    unsigned long long turns = 0;
     hipEvent_t ev = nullptr;
 };
 
@@ -761,7 +768,11 @@ static void factor_layout(const kmx_plan* p, kmx_factor* f, int first, int count
 // The workspace for the classes that there are, with every matrix laid out in it: W of T
 // classes would be three times as much on a 6D diffusion operator (42 -> 17 MB at lev 4).
 static void factor_workspace(const kmx_plan* p, kmx_factor* f, hipStream_t s) {
-    if (f->d_ws) hipFree(f->d_ws);  // (waits for what still runs on it)
+    for (kmx_factor::Slot& t : f->slot) {  // (hipFree waits for what still runs on them)
+        if (t.ws && t.ws != f->d_ws) hipFree(t.ws);
+        t = kmx_factor::Slot();
+    }
+    if (f->d_ws) hipFree(f->d_ws);
     f->d_ws = f->d_fac[0] = f->d_fac[1] = nullptr;
     f->room = f->ncls;
     f->w_elems = size_t(f->ncls) * f->NV * f->launch.WN * size_t(f->G);
@@ -770,6 +781,7 @@ static void factor_workspace(const kmx_plan* p, kmx_factor* f, hipStream_t s) {
         f->d_ws = nullptr;
         throw std::bad_alloc();
     }
+    f->slot[0].ws = f->d_ws;
     f->d_fac[0] = f->d_ws + ws;
     if (p->d_blkT64) f->d_fac[1] = f->d_fac[0] + f->mat;
     factor_layout(p, f, 0, p->T * p->D, s);
@@ -845,7 +857,7 @@ void kmx_factor_build(kmx_plan* p, const std::vector<int>& idx, const std::vecto
                             : 18e-6 + fac_fma / (D == 2 ? 6e12 : 7e12) > pair_fma / (D == 2 ? 4.7e12 : 1.1e13);
     if (!env && slower) return;
     const double w_elems = double(T) * NV * L.WN * double(G);
-    if (w_elems * 8.0 > 1024e6) return;
+    if (w_elems * 8.0 > FAC_BYTES) return;
     auto f = new kmx_factor();
     f->launch = L;
     f->G = G;
@@ -955,6 +967,45 @@ void kmx_factor_term_updated(kmx_plan* p, hipStream_t s) {
 
 bool kmx_factor_ok(const kmx_plan* p, bool transpose) { return p->fac && p->fac->d_fac[transpose ? 1 : 0]; }
 
+// A workspace for an apply on s: the stream's own last one, one that no stream has, or the one
+// whose last apply is longest ago, behind that apply; null if that cannot be waited for.  So
+// that applies on several streams overlap, as the pair kernels' do: 4D lev 5 deg 2, 8 terms,
+// two streams in turn 39 us an apply with one workspace, 16.6 with one each (16.0 pair by
+// pair); 3D lev 5 deg 4, 6 terms 39 and 17.8 (26.9).
+static kmx_factor::Slot* factor_slot(const kmx_plan* p, kmx_factor* f, hipStream_t s) {
+    kmx_factor::Slot* old = f->slot;
+    const size_t bytes = (f->w_elems + size_t(f->splits) * p->N * p->B) * sizeof(double);
+    for (int i = 0; i < FAC_SLOTS && double(bytes) * (i + 1) <= std::max(FAC_BYTES, double(bytes)); ++i) {
+        kmx_factor::Slot& t = f->slot[i];
+        if (t.ws && (!t.turn || t.last == s)) return &t;
+        if (!t.ws) {
+            // (another thread's capture must not see the allocation)
+            hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+            const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+            const hipError_t e = hipMalloc(&t.ws, bytes);
+            if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+            if (e == hipSuccess) return &t;
+            t.ws = nullptr;
+            (void)hipGetLastError();
+            break;
+        }
+        if (t.turn < old->turn) old = &t;
+    }
+    // a last stream that records a graph now cannot be ordered against
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    const hipError_t q = hipStreamIsCapturing(old->last, &cap);
+    (void)hipGetLastError();
+    if (cap != hipStreamCaptureStatusNone || q == hipErrorStreamCaptureImplicit) return nullptr;
+    if (hipEventRecord(f->ev, old->last) != hipSuccess || hipStreamWaitEvent(s, f->ev, 0) != hipSuccess) {
+        (void)hipGetLastError();  // (a stream that is gone, or captures now)
+        if (hipDeviceSynchronize() != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+    }
+    return old;
+}
+
 // 1: launched; 0: this call runs pair by pair; negative: an error
 int kmx_factor_apply(kmx_plan* p, bool transpose, const KArgs<double>& k, hipStream_t s) {
     kmx_factor* f = p->fac;
@@ -966,8 +1017,6 @@ int kmx_factor_apply(kmx_plan* p, bool transpose, const KArgs<double>& k, hipStr
     FacArgs a;
     std::memset(&a, 0, sizeof(a));
     a.x = k.x;
-    a.W = f->d_ws;
-    a.part = f->d_ws + f->w_elems;
     a.fac = f->d_fac[transpose ? 1 : 0];
     std::memcpy(a.scale, p->scale, sizeof(a.scale));
     a.tab = f->d_tab;
@@ -984,25 +1033,13 @@ int kmx_factor_apply(kmx_plan* p, bool transpose, const KArgs<double>& k, hipStr
     a.N = p->N;
     a.splits = f->splits;
     std::lock_guard<std::mutex> lock(f->mu);
-    if (f->used && f->last != s) {  // the workspace passes to another stream
-        // a last stream that records a graph now cannot be ordered against: pair by pair
-        const hipError_t q = hipStreamIsCapturing(f->last, &cap);
-        if (cap != hipStreamCaptureStatusNone || q == hipErrorStreamCaptureImplicit) {
-            (void)hipGetLastError();
-            return 0;
-        }
-        (void)hipGetLastError();
-        if (hipEventRecord(f->ev, f->last) != hipSuccess || hipStreamWaitEvent(s, f->ev, 0) != hipSuccess) {
-            (void)hipGetLastError();  // (a stream that is gone, or captures now)
-            if (hipDeviceSynchronize() != hipSuccess) {
-                (void)hipGetLastError();
-                return 0;
-            }
-        }
-    }
+    kmx_factor::Slot* slot = factor_slot(p, f, s);
+    if (!slot) return 0;
+    a.W = slot->ws;
+    a.part = slot->ws + f->w_elems;
     f->launch.run(a, k, s);
-    f->used = true;
-    f->last = s;
+    slot->last = s;
+    slot->turn = ++f->turns;
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {
         set_error(std::string("factored apply launch: ") + hipGetErrorString(e));
@@ -1018,6 +1055,8 @@ void kmx_factor_free(kmx_plan* p) {
     if (f->d_slot) hipFree(f->d_slot);
     if (f->d_tab) hipFree(f->d_tab);
     if (f->d_mask) hipFree(f->d_mask);
+    for (kmx_factor::Slot& t : f->slot)
+        if (t.ws && t.ws != f->d_ws) hipFree(t.ws);
     if (f->d_ws) hipFree(f->d_ws);
     if (f->ev) hipEventDestroy(f->ev);
     delete f;

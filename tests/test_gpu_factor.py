@@ -275,3 +275,58 @@ def test_matrices_that_split_and_join_classes(kmx_gpu, nd, lev, deg, T, conn):
             plan.update_term(t, d, mats[t][d])
     check()
     assert torch.equal(plan.apply(xd), first[0]) and torch.equal(plan.apply_transpose(xd), first[1])
+
+
+def test_more_streams_than_workspaces(kmx_gpu):
+    """Six streams in turn, in blocks and from threads: the bits of an apply alone; again
+    after a matrix that splits a class (workspaces made anew), and while a graph is recorded."""
+    import threading
+
+    import torch
+
+    mats, idx, rp, cols, _ = case(3, 4, 3, 3, True, 4, shared=True)
+    plan = kmx_gpu.Plan(mats, idx, 3, rp, cols, index_base=1, adjoint=True)
+    streams = [torch.cuda.Stream() for _ in range(6)]
+    xs = [torch.randn(plan.dof, dtype=torch.float64, device="cuda") for _ in streams]
+    for split in (False, True):
+        if split:
+            plan.update_term(2, 0, np.random.default_rng(2).standard_normal(mats[2][0].shape))
+        assert plan.factored()
+        want = [plan.apply(x).clone() for x in xs]
+        wantT = [plan.apply_transpose(x).clone() for x in xs]
+        out = [[torch.zeros_like(x) for _ in range(12)] for x in xs]
+        torch.cuda.synchronize()
+        for q in range(4):  # in turn
+            for k, s in enumerate(streams):
+                plan.apply(xs[k], out[k][q], stream=s)
+        for k, s in enumerate(streams):  # in blocks
+            for q in range(4, 8):
+                plan.apply_transpose(xs[k], out[k][q], stream=s)
+
+        def work(k):
+            for q in range(8, 12):
+                plan.apply(xs[k], out[k][q], stream=streams[k])
+
+        torch.cuda.synchronize()
+        th = [threading.Thread(target=work, args=(k,)) for k in range(6)]
+        for t in th:
+            t.start()
+        for t in th:
+            t.join()
+        torch.cuda.synchronize()
+        for k in range(6):
+            for q in range(12):
+                assert torch.equal(out[k][q], wantT[k] if 4 <= q < 8 else want[k]), (split, k, q)
+    fresh = kmx_gpu.Plan(mats, idx, 3, rp, cols, index_base=1)
+    ref = fresh.apply(xs[0]).clone()
+    graph, a, b = torch.cuda.CUDAGraph(), torch.zeros_like(ref), torch.zeros_like(ref)
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        fresh.apply(xs[0], a)
+        fresh.apply(xs[0], b, stream=streams[1])  # its first apply there: a workspace of its own
+    streams[1].synchronize()
+    assert torch.equal(b, ref) and not a.any()
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float((a - ref).norm() / ref.norm()) <= 1e-13
