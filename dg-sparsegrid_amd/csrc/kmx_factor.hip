@@ -846,15 +846,19 @@ void kmx_factor_build(kmx_plan* p, const std::vector<int>& idx, const std::vecto
     // 6D deg 2, level-limited and adapted sets: the three launches and their walks take 18 us
     // and 6e12 (2D) or 7e12 FMAs / s in whole waves, the pair kernels at best 4.7e12 or 1.1e13
     // (2D lev 7 deg 3 adapted: 26 against 22 us, lev 8: 44 against 139; 3D lev 6 deg 3: 29
-    // against 27, lev 7: 66 against 135; 6D lev 4 deg 2: 41 against 77).
+    // against 27, lev 7: 66 against 135; 6D lev 4 deg 2: 41 against 77).  The pair kernels do
+    // 5.5e12 in 2D deg 2 (lev 8, all pairs, 4 terms: 26.6 against 21.5 us; adapted, 2 terms:
+    // 26.7 against 42.7) and 1.25e13 with 3 terms in 3D (lev 6 deg 3, all pairs: 27.6 against
+    // 25.9; lev 7 deg 2, all pairs: 27.3 against 29.4).
     const double lanes = double((G + 63) / 64) * 64.0, rlanes = double((N + 63) / 64) * 64.0;
     const double fac_fma = T * (double(contr) * lanes + double(NV) * rlanes) * unit;
     // 3D deg 4, whose 16-entry blocks are cheaper here and whose pairs are split over four
     // lanes there: 19 us and 1e13 against 11 us and 1.2e13 (lev 5, 6 terms: 28 against 51; lev
     // 6, 3 terms: 41 / 80; lev 4 adapted, 6 terms: 25 / 35; lev 4, 6 terms: 23 / 20.5).
+    const double pair_rate = D == 2 ? (p->deg == 2 ? 5.5e12 : 4.7e12) : D == 3 && T <= 3 ? 1.25e13 : 1.1e13;
     const bool slower = D == 3 && p->deg == 4
                             ? 19e-6 + fac_fma / 1e13 > 11e-6 + pair_fma / 1.2e13
-                            : 18e-6 + fac_fma / (D == 2 ? 6e12 : 7e12) > pair_fma / (D == 2 ? 4.7e12 : 1.1e13);
+                            : 18e-6 + fac_fma / (D == 2 ? 6e12 : 7e12) > pair_fma / pair_rate;
     if (!env && slower) return;
     const double w_elems = double(T) * NV * L.WN * double(G);
     if (w_elems * 8.0 > FAC_BYTES) return;
