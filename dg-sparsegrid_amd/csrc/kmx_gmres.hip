@@ -374,6 +374,15 @@ __global__ void __launch_bounds__(256) k_from_box(const double* xb, double* x, c
     if (i < nb && map[i] >= 0) x[map[i]] = xb[i];
 }
 
+// max(1, 1 - dt d)^power; in box order with a map
+__global__ void __launch_bounds__(256) k_stiff_scale(const double* d, double* out, const int* map, long long n,
+                                                     double dt, double power) {
+    const long long i = blockIdx.x * 256ll + threadIdx.x;
+    if (i >= n) return;
+    const long long e = map ? map[i] : i;
+    out[i] = e < 0 ? 0.0 : pow(fmax(1.0, 1.0 - dt * d[e]), power);
+}
+
 template <int RB>
 void launch_reg(const ArnoldiArgs& a, hipStream_t s) {
     const dim3 grid(unsigned(a.G)), block(AR_THREADS);
@@ -530,4 +539,29 @@ extern "C" int kmx_arnoldi_box_step(kmx_plan* p, int prec, int k, double* V, dou
     rc = kmx_sweep_box_ops(p, prec, reinterpret_cast<hipStream_t>(stream));
     if (rc != KMX_OK) return rc;
     return arnoldi("kmx_arnoldi_box_step", b.nb, k, V, nullptr, &b, s0, s1, scale, z, h, work, stream);
+}
+
+extern "C" int kmx_plan_stiff_scale(kmx_plan* p, int prec, double dt, double power, double* work, double* out,
+                                    void* stream) {
+    if (!p || (p->N > 0 && (!work || !out))) {
+        set_error("kmx_plan_stiff_scale: null argument");
+        return KMX_E_ARG;
+    }
+    if (p->N == 0) return KMX_OK;
+    kmx_box_view b;
+    std::memset(&b, 0, sizeof(b));
+    b.nb = (long long)p->N * p->B;
+    if (prec >= 0) {
+        if (work == out) {
+            set_error("kmx_plan_stiff_scale: work must not be out in box order");
+            return KMX_E_ARG;
+        }
+        const int rc = box_of("kmx_plan_stiff_scale", p, prec, true, &b);
+        if (rc != KMX_OK) return rc;
+    }
+    const int rc = kmx_plan_diagonal(p, work, stream);
+    if (rc != KMX_OK) return rc;
+    hipLaunchKernelGGL(k_stiff_scale, box_grid(b.nb), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), work, out,
+                       b.map, b.nb, dt, power);
+    return box_done("kmx_plan_stiff_scale");
 }

@@ -147,6 +147,8 @@ PROTOTYPES = {
     "kmx_apply_transpose": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p]),
     "kmx_plan_assemble": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p]),
     "kmx_plan_diagonal": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p]),
+    "kmx_plan_stiff_scale": (C.c_int, [C.c_void_p, C.c_int, C.c_double, C.c_double, C.c_void_p, C.c_void_p,
+                                       C.c_void_p]),
     "kmx_apply_host": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_int]),
     "kmx_batch_create": (C.c_int, [C.POINTER(C.c_void_p), C.c_int, C.POINTER(C.c_void_p)]),
     "kmx_batch_apply": (C.c_int, [C.c_void_p, C.POINTER(C.c_void_p), C.POINTER(C.c_void_p), C.c_int, C.c_void_p]),

@@ -171,6 +171,16 @@ class Plan:
         check(lib().kmx_plan_diagonal(self.handle, _ptr(out) if self.dof else None, _stream(stream)))
         return out
 
+    def stiff_scale(self, dt, power, work, out, prec=None, stream=None):
+        """out = max(1, 1 - dt diagonal)^power (kmx_plan_stiff_scale), with prec in the sweep's
+        order; work: dof values."""
+        if work.numel() != self.dof or out.numel() != (self.dof if prec is None else self.box_values(prec)):
+            raise ValueError("stiff_scale: work must have dof entries, out dof or box_values")
+        check(lib().kmx_plan_stiff_scale(self.handle, -1 if prec is None else _prec(prec), float(dt), float(power),
+                                         _ptr(work) if self.dof else None, _ptr(out) if self.dof else None,
+                                         _stream(stream)))
+        return out
+
     def box_values(self, prec="fp64"):
         """Values of a vector in the sweep's order (kmx_plan_box_values), 0 without one on."""
         nb = C.c_int64()

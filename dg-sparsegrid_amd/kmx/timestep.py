@@ -341,10 +341,10 @@ class DeviceGMRES:
         forming b - M x (callers that need the true residual form it themselves)."""
         torch = _torch()
         m = self.m
-        x = torch.zeros_like(b)
+        x = None  # zero: the first cycle's correction is x itself
         bnorm = float(torch.linalg.vector_norm(b)) if bnorm is None else float(bnorm)
         if bnorm == 0.0:
-            return x, 0.0, 0
+            return torch.zeros_like(b), 0.0, 0
         it, rel, r, beta = 0, 1.0, b, bnorm
         while it < maxiter:
             if r is not b:
@@ -395,19 +395,17 @@ class DeviceGMRES:
                     launch(nxt)
             y = self.ystage[: ls.k]
             y.copy_(torch.from_numpy(ls.solve()))
-            if self.scale is None:
-                x.addmv_(self.V[: ls.k].t(), y.to(b.device, non_blocking=True))
-            else:
-                d = torch.mv(self.V[: ls.k].t(), y.to(b.device, non_blocking=True))
-                if self.box is None:
-                    x.addcmul_(self.scale, d)
-                else:
-                    x.add_(self.box[0]().from_box(d.mul_(self.scale), torch.empty_like(x), self.box[1]))
+            d = torch.mv(self.V[: ls.k].t(), y.to(b.device, non_blocking=True))
+            if self.scale is not None:
+                d.mul_(self.scale)
+            if self.box is not None:
+                d = self.box[0]().from_box(d, torch.empty_like(b), self.box[1])
+            x = d if x is None else x.add_(d)
             est = ls.residual() / bnorm
             if est <= tol or it >= maxiter:
                 return x, est, it
             r = b - self.matvec(x, self.Mx)
-        return x, rel, it
+        return torch.zeros_like(b) if x is None else x, rel, it
 
 
 def gmres(matvec, b, x0=None, tol=1e-6, restart=40, maxiter=400):
@@ -437,8 +435,7 @@ def scale_power(nd, deg):
       2D            4, 5  0.96 .. 1.05      1.02 .. 1.17      1.13 .. 1.41
       1D              4   1.01 .. 1.04      1.07 .. 1.18      1.25 .. 1.41
     Advection-diffusion gains most from the highest (1D to 3D: 0.58 .. 0.93, 0.43 .. 0.88,
-    0.37 .. 0.89), but the sizes do not tell it from diffusion.  Setting the scale up and
-    applying it is 50 to 70 us a call, the price of a step so mild that it saves nothing."""
+    0.37 .. 0.89), but the sizes do not tell it from diffusion."""
     if nd >= 5:
         return -0.75
     if deg <= 3:
@@ -483,7 +480,7 @@ def backward_euler(plan, f0, dt, rhs=None, tol=1e-10, inner_prec="fp32", inner_t
 
     nb = plan.box_values(inner_prec) if hasattr(plan, "box_values") else 0
     boxed = box_order(f0.numel(), nb)
-    power = scale_power(plan.ndim, plan.deg) if hasattr(plan, "diagonal") else 0.0
+    power = scale_power(plan.ndim, plan.deg) if hasattr(plan, "stiff_scale") else 0.0
     scaled = boxed or power != 0.0
     key = (float(dt), inner_prec, int(restart), f0.numel(), boxed, scaled)
     cache = _SOLVERS.setdefault(plan, {})
@@ -497,11 +494,7 @@ def backward_euler(plan, f0, dt, rhs=None, tol=1e-10, inner_prec="fp32", inner_t
     if hasattr(plan, "replay_state"):  # (a stand-in for a plan may have its product alone)
         solver.captured_for(plan.replay_state(inner_prec))
     if power:  # (a scale is 1 otherwise)
-        d = torch.rsub(plan.diagonal(), 1.0, alpha=float(dt)).clamp_(min=1.0)
-        if solver.box is None:
-            torch.pow(d, power, out=solver.scale)
-        else:
-            plan.to_box(d.pow_(power), solver.scale, inner_prec)
+        plan.stiff_scale(dt, power, r, solver.scale, inner_prec if boxed else None)
     f = f0.clone()  # f0 is a good first guess for small dt
     hist, inner = [], 0
     for _ in range(max_refine):

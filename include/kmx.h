@@ -201,6 +201,12 @@ int kmx_plan_assemble(kmx_plan* plan, double* blocks, void* stream);
  * whose pair list leaves the element itself out.  Asynchronous on `stream`. */
 int kmx_plan_diagonal(kmx_plan* plan, double* d, void* stream);
 
+/* The right scaling of M = I - dt A that backward Euler's GMRES takes, kmx_arnoldi_step_scaled's
+ * S: out_i = max(1, 1 - dt A_ii)^power (DEVICE, N * B doubles; prec < 0), or in the order of
+ * kmx_plan_box_values(prec), 0 where a cell is absent.  work: N * B doubles of DEVICE memory
+ * (may be out where prec < 0).  Asynchronous on `stream`. */
+int kmx_plan_stiff_scale(kmx_plan* plan, int prec, double dt, double power, double* work, double* out, void* stream);
+
 /* Host-pointer convenience for callers without device memory (a MEX gateway):
  * copies x in, applies, copies y out, synchronises. */
 int kmx_apply_host(kmx_plan* plan, const double* x_host, double* y_host, int prec);

@@ -272,3 +272,31 @@ def test_scaling_costs_no_inner_steps(kmx_gpu, monkeypatch, nd, lev, deg):
     scaled = steps()
     monkeypatch.setattr(TS, "scale_power", lambda nd, deg: 0.0)
     assert scaled <= 1.03 * steps()
+
+
+@pytest.mark.parametrize("power", [-0.75, -0.5, -0.25, 1.0])
+def test_stiff_scale_is_a_power_of_the_diagonal(kmx_gpu, power):
+    """Against torch, 8 ulps of pow's; in the sweep's order the same values, 0 in absent cells."""
+    import torch
+
+    tab = G.refine_random(G.hash_table_sparse_nd([3] * 3, 3, "SG"), 5, 0.5, np.random.default_rng(1))
+    pde = K.diffusion_nd(3, 5)
+    plan = kmx_gpu.Plan(K.get_coeff_mats(pde, 3), tab.idx1d, 3, None, None, index_base=1, fp32=True, level_blocks=True,
+                        identity=[[d != t for d in range(3)] for t in range(3)])
+    work = torch.empty(plan.dof, dtype=torch.float64, device="cuda")
+    for dt in (-3.0, 0.0, 100 * pde.set_dt(pde, 0.01)):
+        want = (1.0 - dt * plan.diagonal()).clamp(min=1.0).pow(power)
+        got = plan.stiff_scale(dt, power, work, torch.empty_like(work))
+        assert float(((got - want) / want).abs().max()) <= 8 * 2.3e-16
+        assert torch.equal(plan.stiff_scale(dt, power, work, work), got)
+        for p in ("fp64", "fp32"):
+            plan.set_sweep(p, True)
+            nb = plan.box_values(p)
+            assert nb > plan.dof
+            box = plan.stiff_scale(dt, power, work, torch.full((nb,), 7.0, dtype=torch.float64, device="cuda"), p)
+            assert torch.equal(box, plan.to_box(got, torch.empty_like(box), p))
+            plan.set_sweep(p, False)
+    with pytest.raises(ValueError):
+        plan.stiff_scale(1.0, power, work, work[:-1].clone())
+    with pytest.raises(ValueError):
+        plan.stiff_scale(1.0, power, work, torch.empty_like(work), "fp32")  # no sweep on
