@@ -142,22 +142,25 @@ hipError_t launch_as(const AsmArgs& g, int deg, size_t lds, unsigned grid, hipSt
     return hipGetLastError();
 }
 
+// In 1D a pair's block is a block of the strip, read once: the strips stay in global memory
+// (lev 8 deg 4, all pairs, 2 terms: 46.9 us from LDS, 6.5 now; lev 9 deg 4, connected 14.4, 7.7)
 template <int D>
 hipError_t launch(const AsmArgs& g, int deg, size_t lds, unsigned grid, hipStream_t s) {
-    if (lds == 0) return launch_as<D, 1, 1, false>(g, deg, lds, grid, s);
+    constexpr bool LDS = D > 1;
+    if (LDS && lds == 0) return launch_as<D, 1, 1, false>(g, deg, lds, grid, s);
     // both digits while a pair's threads fill a wave: shorter runs store in pieces
     const bool two = D > 1 && (long long)g.B * g.B >= 64ll * deg * deg;
     switch (deg) {
         case 2:
-            return two ? launch_as<D, 2, D == 1 ? 1 : 2, true>(g, deg, lds, grid, s)
-                       : launch_as<D, 2, 1, true>(g, deg, lds, grid, s);
+            return two ? launch_as<D, 2, D == 1 ? 1 : 2, LDS>(g, deg, lds, grid, s)
+                       : launch_as<D, 2, 1, LDS>(g, deg, lds, grid, s);
         case 3:
-            return two ? launch_as<D, 3, D == 1 ? 1 : 3, true>(g, deg, lds, grid, s)
-                       : launch_as<D, 3, 1, true>(g, deg, lds, grid, s);
+            return two ? launch_as<D, 3, D == 1 ? 1 : 3, LDS>(g, deg, lds, grid, s)
+                       : launch_as<D, 3, 1, LDS>(g, deg, lds, grid, s);
         case 4:
-            return two ? launch_as<D, 4, D == 1 ? 1 : 4, true>(g, deg, lds, grid, s)
-                       : launch_as<D, 4, 1, true>(g, deg, lds, grid, s);
-        default: return launch_as<D, 1, 1, true>(g, deg, lds, grid, s);
+            return two ? launch_as<D, 4, D == 1 ? 1 : 4, LDS>(g, deg, lds, grid, s)
+                       : launch_as<D, 4, 1, LDS>(g, deg, lds, grid, s);
+        default: return launch_as<D, 1, 1, LDS>(g, deg, lds, grid, s);
     }
 }
 
@@ -255,7 +258,7 @@ extern "C" int kmx_plan_assemble(kmx_plan* p, double* blocks, void* stream) {
     g.out = blocks;
     g.B = p->B;
     const size_t strips = size_t(st) * p->T * sizeof(double);
-    const size_t lds = strips <= 64 * 1024 ? strips : 0;
+    const size_t lds = p->D > 1 && strips <= 64 * 1024 ? strips : 0;
     // Workgroups: about 2048, each of 16 pairs at least to pay for its strips.  Blocks of 256
     // values and more: two rounds of what the CUs hold (3D lev 5 deg 3, 3.5 thousand: 99 -> 90
     // us; 3D lev 4 deg 4, whose 37 KB of strips leave four a CU: 85 us with 2 thousand, 96 with

@@ -112,3 +112,17 @@ def test_assembled_blocks_by_entries_per_thread(kmx_gpu, nd, lev, deg, T, conn):
     plan = kmx_gpu.Plan(mats, idx, deg, rp, cols)
     A = dense_from_blocks(plan.assemble().cpu().numpy(), plan.N, plan.B, rp, cols)
     assert np.array_equal(A, O.build_A(O.ApplyInputs(mats, idx, deg, rp, cols)))
+
+
+@pytest.mark.parametrize("nd,lev,deg,T,elems", [(1, 6, 2, 3, None), (1, 6, 3, 2, None), (1, 5, 4, 2, None), (1, 5, 5, 2, None),
+                                                (2, 9, 3, 1, 12), (3, 8, 4, 1, 7)])
+def test_assembled_blocks_from_strips_in_global_memory(kmx_gpu, nd, lev, deg, T, elems):
+    """1D, and strips beyond LDS in more dimensions (a few elements of a high level): bit-exact."""
+    rng = np.random.default_rng(nd * 10 + deg)
+    idx = np.asarray(O.hash_table_sparse_nd([lev] * nd, lev, "SG")["idx1d"])
+    if elems:
+        idx = idx[np.sort(rng.permutation(len(idx))[:elems])]
+    mats = [[rng.standard_normal((deg * 2 ** lev,) * 2) for _ in range(nd)] for _ in range(T)]
+    plan = kmx_gpu.Plan(mats, idx, deg)
+    A = dense_from_blocks(plan.assemble().cpu().numpy(), plan.N, plan.B, None, None)
+    assert np.array_equal(A, O.build_A(O.ApplyInputs(mats, idx, deg, None, None)))
