@@ -24,6 +24,7 @@
 #include "kmx_mma64.h"
 
 #include <algorithm>
+#include <cstring>
 #include <map>
 #include <numeric>
 #include <stdexcept>
@@ -265,14 +266,15 @@ struct kmx_realspace {
     // children (nodes of stage k + 1; elements in the last) and the children's columns
     struct Stage {
         int nodes = 0;
-        int* d_cptr = nullptr;
-        int* d_col = nullptr;
-        int* d_list = nullptr;  // lptr, lcol, lx of StageArgs (null: no lists)
-        size_t o_col = 0, o_x = 0;
+        size_t cptr = 0, col = 0;            // (places in d_tab)
+        size_t lptr = 0, lcol = 0, lx = 0;   // of StageArgs
+        bool lists = false;
     };
     Stage stage[KMX_MAX_DIM];
-    int* d_row = nullptr;                   // elements in prefix order
-    int* d_flag = nullptr;                  // one per stage
+    // every index table in one allocation and copy (3D lev 5 deg 2: the plan 1.17 -> 1.01 ms)
+    int* d_tab = nullptr;
+    size_t row = 0;   // elements in prefix order
+    size_t flag = 0;  // one per stage
     unsigned calls = 0;
     double* d_buf[2] = {nullptr, nullptr};  // Z_d, Z_{d-1}, ... in turn
 };
@@ -280,13 +282,7 @@ struct kmx_realspace {
 static void free_rs(kmx_realspace* r) {
     for (auto& m : r->d_meval)
         if (m) hipFree(m);
-    for (auto& st : r->stage) {
-        if (st.d_cptr) hipFree(st.d_cptr);
-        if (st.d_col) hipFree(st.d_col);
-        if (st.d_list) hipFree(st.d_list);
-    }
-    if (r->d_flag) hipFree(r->d_flag);
-    if (r->d_row) hipFree(r->d_row);
+    if (r->d_tab) hipFree(r->d_tab);
     for (auto& b : r->d_buf)
         if (b) hipFree(b);
 }
@@ -295,18 +291,26 @@ static void free_rs(kmx_realspace* r) {
 // more: a wavelet of level l is zero on all but 2^(1-l) of its dimension, exactly, so a
 // tile of 64 of 192 points meets 0.42 of 64 cells' blocks, of 3072 points 0.036 of 512's.
 // Leaving a zero block out leaves every sum's bits as they are.
-template <class UP>
+template <class Put>
 static void build_lists(kmx_realspace* r, int k, const double* meval, const std::vector<int>& cptr,
-                        const std::vector<int>& col, const std::vector<int>& order, const UP& up) {
+                        const std::vector<int>& col, const std::vector<int>& order, const Put& put) {
     const int M = r->npts[k], deg = r->deg, tiles = (M + 63) / 64, blocks = r->ncols[k] / deg;
     if (tiles < 2 || col.empty()) return;
     std::vector<unsigned char> on(size_t(tiles) * blocks, 0);
     for (int b = 0; b < blocks; ++b)
         for (int t = 0; t < tiles; ++t) {
-            bool any = false;
-            for (int c = b * deg; c < (b + 1) * deg && !any; ++c)
-                for (int i = 64 * t; i < std::min(M, 64 * t + 64) && !any; ++i) any = !(meval[size_t(c) * M + i] == 0.0);
-            on[size_t(t) * blocks + b] = any;
+            // (all bits but the sign, a column's run at once: 67 MB of 1D lev 9 deg 4 in 4.7 ms,
+            // 8.7 value by value)
+            unsigned long long any = 0;
+            for (int c = b * deg; c < (b + 1) * deg && !any; ++c) {
+                const double* v = meval + size_t(c) * M;
+                for (int i = 64 * t; i < std::min(M, 64 * t + 64); ++i) {
+                    unsigned long long bits;
+                    std::memcpy(&bits, v + i, sizeof bits);
+                    any |= bits << 1;
+                }
+            }
+            on[size_t(t) * blocks + b] = any != 0;
         }
     const int nodes = int(cptr.size()) - 1;
     if (double(col.size()) * tiles > 2e7) return;  // (160 MB of lists at most)
@@ -323,11 +327,10 @@ static void build_lists(kmx_realspace* r, int k, const double* meval, const std:
         }
     ptr.push_back(int(lcol.size()));
     if (double(lcol.size()) > 0.9 * double(col.size()) * tiles) return;
-    r->stage[k].o_col = ptr.size();
-    r->stage[k].o_x = ptr.size() + lcol.size();
-    ptr.insert(ptr.end(), lcol.begin(), lcol.end());
-    ptr.insert(ptr.end(), lx.begin(), lx.end());
-    up(ptr, r->stage[k].d_list);
+    r->stage[k].lists = true;
+    r->stage[k].lptr = put(ptr);
+    r->stage[k].lcol = put(lcol);
+    r->stage[k].lx = put(lx);
 }
 
 extern "C" int kmx_realspace_create(int ndim, int deg, int num_elem, const int* elem_idx1d, int index_base,
@@ -402,11 +405,12 @@ extern "C" int kmx_realspace_create(int ndim, int deg, int num_elem, const int* 
             for (int k = diff + 1; k <= ndim; ++k) first[size_t(k)].push_back(p);
         }
         if (num_elem > 0) first[0].push_back(0);
-        auto up = [](const std::vector<int>& h, int*& d) {
-            if (h.empty()) return;
-            if (hipMalloc(&d, h.size() * sizeof(int)) != hipSuccess) throw std::bad_alloc();
-            if (hipMemcpy(d, h.data(), h.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess)
-                throw std::runtime_error("hipMemcpy failed");
+        std::vector<int> tab;
+        auto put = [&](const std::vector<int>& h) {
+            const size_t at = tab.size();
+            tab.insert(tab.end(), h.begin(), h.end());
+            tab.resize((tab.size() + 31) / 32 * 32, 0);
+            return at;
         };
         long long need[2] = {1, 1}, R = 1;
         for (int k = ndim - 1; k >= 0; --k) {
@@ -422,9 +426,9 @@ extern "C" int kmx_realspace_create(int ndim, int deg, int num_elem, const int* 
             cptr.push_back(int(c));
             for (size_t q = 0; q < chl.size(); ++q) col[q] = ix(order[size_t(chl[q])], k) * deg;
             r->stage[k].nodes = int(par.size());
-            up(cptr, r->stage[k].d_cptr);
-            up(col, r->stage[k].d_col);
-            build_lists(r, k, meval[k], cptr, col, order, up);
+            r->stage[k].cptr = put(cptr);
+            r->stage[k].col = put(col);
+            build_lists(r, k, meval[k], cptr, col, order, put);
             if (k > 0) {  // Z_{k+1} of the comment above (k from 1 there)
                 R *= npts[k];
                 long long nb = 1;
@@ -432,8 +436,11 @@ extern "C" int kmx_realspace_create(int ndim, int deg, int num_elem, const int* 
                 need[(ndim - 1 - k) & 1] = std::max(need[(ndim - 1 - k) & 1], (long long)par.size() * nb * R);
             }
         }
-        up(order, r->d_row);
-        up(std::vector<int>(size_t(ndim), 0), r->d_flag);
+        r->row = put(order);
+        r->flag = put(std::vector<int>(size_t(ndim), 0));
+        if (hipMalloc(&r->d_tab, tab.size() * sizeof(int)) != hipSuccess) throw std::bad_alloc();
+        if (hipMemcpy(r->d_tab, tab.data(), tab.size() * sizeof(int), hipMemcpyHostToDevice) != hipSuccess)
+            throw std::runtime_error("hipMemcpy failed");
         for (int q = 0; q < 2; ++q)
             if (hipMalloc(&r->d_buf[q], size_t(need[q]) * sizeof(double)) != hipSuccess) throw std::bad_alloc();
         *out = r;
@@ -468,16 +475,16 @@ extern "C" int kmx_realspace_apply(kmx_realspace* r, const double* f_w, double* 
         a.in = cur;
         a.out = k == 0 ? f_r : r->d_buf[(D - 1 - k) & 1];
         a.A = r->d_meval[k];
-        a.cptr = r->stage[k].d_cptr;
-        a.col = r->stage[k].d_col;
-        a.row = r->d_row;
         const kmx_realspace::Stage& st = r->stage[k];
-        a.lptr = st.d_list;
-        a.lcol = st.d_list ? st.d_list + st.o_col : nullptr;
-        a.lx = st.d_list ? st.d_list + st.o_x : nullptr;
+        a.cptr = r->d_tab + st.cptr;
+        a.col = r->d_tab + st.col;
+        a.row = r->d_tab + r->row;
+        a.lptr = st.lists ? r->d_tab + st.lptr : nullptr;
+        a.lcol = st.lists ? r->d_tab + st.lcol : nullptr;
+        a.lx = st.lists ? r->d_tab + st.lx : nullptr;
         a.ptiles = (r->npts[k] + 63) / 64;
-        a.flag = r->d_flag + k;
-        a.before = k + 1 < D ? r->d_flag + k + 1 : nullptr;
+        a.flag = r->d_tab + r->flag + k;
+        a.before = k + 1 < D ? a.flag + 1 : nullptr;
         a.call = call;
         a.R = R;
         a.M = r->npts[k];
