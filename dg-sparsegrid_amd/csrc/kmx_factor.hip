@@ -119,10 +119,6 @@ struct FacShape {
     static constexpr int NC = U / C, NCB = V / CB;
     // W of a node: NCB column groups of BU values (prefix component, column in the group) in pairs
     static constexpr int BUP = (BU + 1) / 2, WN = NCB * BUP * 2;
-    __host__ __device__ static constexpr int w_at(int val, int G) {  // value val of suffix 0
-        const int i = val / V * CB + val % V % CB;
-        return ((val % V / CB * BUP + i / 2) * G) * 2 + i % 2;
-    }
 };
 
 // out[.., a, ..] += sum_b m[a][b] in[.., b, ..] along an index of stride ST of N values

@@ -104,9 +104,10 @@ int kmx_plan_destroy(kmx_plan* plan);
 
 /* Time the kernel variants (workgroup size 128/256/512, LDS staging of the
  * row's coefficient strips on/off; FP64 with factored sums against them) on
- * this plan for FP64 and FP32 and keep the fastest; plans of the same (d, deg, terms, pair density) created later in
- * the process start from that choice.  Synchronous on `stream`; not for use
- * under graph capture.  No counterpart in the reference (MATLAB picks nothing;
+ * this plan for FP64 and FP32 and keep the fastest; plans of the same (d, deg,
+ * terms, pair density) created later in the process start from that variant (a
+ * plan that is faster pair by pair gives the factored form up for itself alone).
+ * Synchronous on `stream`; not for use under graph capture.  No counterpart in the reference (MATLAB picks nothing;
  * its flops_kron{k} method choice is the only cost model it has). */
 int kmx_plan_autotune(kmx_plan* plan, void* stream);
 
