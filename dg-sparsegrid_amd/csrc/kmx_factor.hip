@@ -954,9 +954,9 @@ void kmx_factor_term_updated(kmx_plan* p, hipStream_t s) {
     if (!p->fac) return;
     kmx_factor* f = p->fac;
     const FacTab tab = f->tab;
-    factor_classes(p, f);
-    if (std::memcmp(&tab, &f->tab, sizeof(tab)) == 0) return;
     try {
+        factor_classes(p, f);
+        if (std::memcmp(&tab, &f->tab, sizeof(tab)) == 0) return;
         factor_slots(f);
         if (f->ncls > f->room) factor_workspace(p, f, s);  // the matrix split a class
     } catch (const std::exception&) {  // no room: the plan runs pair by pair
