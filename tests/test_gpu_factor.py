@@ -330,3 +330,30 @@ def test_more_streams_than_workspaces(kmx_gpu):
         graph.replay()
         torch.cuda.synchronize()
         assert float((a - ref).norm() / ref.norm()) <= 1e-13
+
+
+def test_pair_lists_of_long_runs(kmx_gpu):
+    """Rows of whole 64-column runs: a pair listed twice in place of its neighbour, or the next
+    word's, is no product; the same columns in another order are one."""
+    import torch
+
+    mats, idx, rp, cols, x = case(2, 6, 2, 2, True, 12)
+    rp, cols = np.asarray(rp), np.asarray(cols)
+    row = int(np.flatnonzero(np.diff(rp) == len(idx))[0])  # connected to every element
+    at = int(rp[row])
+    assert len(idx) > 192 and np.array_equal(cols[at:at + len(idx)], np.arange(1, len(idx) + 1))
+    xd = torch.from_numpy(x).cuda()
+    for k, c in ((64, 65), (100, 99), (127, 127), (63, 64), (130, 190)):  # cols[k] is k + 1
+        bad = cols.copy()
+        bad[at + k] = c + (c == k + 1)
+        plan = kmx_gpu.Plan(mats, idx, 2, rp, bad, index_base=1)
+        assert not plan.factored()
+        y = plan.apply(xd).cpu().numpy()
+        assert rel(y, O.apply_A(O.ApplyInputs(mats, idx, 2, rp, bad), x)) <= 1e-13
+    want = kmx_gpu.Plan(mats, idx, 2, rp, cols, index_base=1)
+    assert want.factored()
+    for a, b in ((64, 127), (70, 71), (10, 150)):
+        other = cols.copy()
+        other[[at + a, at + b]] = other[[at + b, at + a]]
+        plan = kmx_gpu.Plan(mats, idx, 2, rp, other, index_base=1)
+        assert plan.factored() and torch.equal(plan.apply(xd), want.apply(xd))
